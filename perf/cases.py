@@ -383,13 +383,14 @@ class _Pixels:
                                          "strides": None}
 
 
-def _device_words(frame, words):
-    return torch.as_tensor(_Pixels(int(_abi.lib().tk_frame_image_device(frame._h)), words, frame), device="cuda")
+def _device_words(frame, words, owner):
+    """The frame's pixels in place; the tensor keeps `owner`, which frees them, alive."""
+    return torch.as_tensor(_Pixels(int(_abi.lib().tk_frame_image_device(frame._h)), words, owner), device="cuda")
 
 
 def _frame_state(canvas):
     frame = tk.Frame(_context(), canvas.encode(0))
-    return {"frame": frame, "image": _device_words(frame, frame.width * frame.height).view(frame.height, frame.width)}
+    return {"frame": frame, "image": _device_words(frame, frame.width * frame.height, frame).view(frame.height, frame.width)}
 
 
 def prepare(case, seed):
@@ -420,7 +421,7 @@ def prepare(case, seed):
         scenes = [c.encode(0) for c in canvases]
         batch = tk.Batch(_context(), scenes)
         columns = np.concatenate([[0], np.cumsum([s.tiles_width * s.tiles_height for s in scenes])])
-        words = _device_words(batch.frame, int(columns[-1]) * 256)
+        words = _device_words(batch.frame, int(columns[-1]) * 256, batch)
         st = {"batch": batch, "image": [words[c * 256:c * 256 + s.width * s.height].view(s.height, s.width)
                                         for s, c in zip(scenes, columns)]}
     elif kind == "one_shot":
