@@ -68,11 +68,28 @@ __device__ __forceinline__ uint32_t wave_exclusive_scan(uint32_t v, uint32_t lan
     return x - v;
 }
 
+// Inclusive wrapping-u32 scan across one full 64-lane wave by DPP: row shifts within
+// the rows of 16, then each row's last lane broadcast to the rows after it.  No LDS
+// permutes, whose lane addresses a loop around them would keep in registers.
+__device__ __forceinline__ uint32_t wave_inclusive_scan_dpp(uint32_t v) {
+#define TK_SCAN_STEP(ctrl, rows) v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xf, false);
+    TK_SCAN_STEP(0x111, 0xf)  // row_shr:1
+    TK_SCAN_STEP(0x112, 0xf)  // row_shr:2
+    TK_SCAN_STEP(0x114, 0xf)  // row_shr:4
+    TK_SCAN_STEP(0x118, 0xf)  // row_shr:8
+    TK_SCAN_STEP(0x142, 0xa)  // row_bcast:15 into rows 1 and 3
+    TK_SCAN_STEP(0x143, 0xc)  // row_bcast:31 into rows 2 and 3
+#undef TK_SCAN_STEP
+    return v;
+}
+
 __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) v += (uint32_t)__shfl_xor((int)v, off, 64);
     return v;
 }
+
+__device__ __forceinline__ uint64_t lanes_below(uint32_t lane) { return lane ? (~0ull >> (64u - lane)) : 0ull; }
 
 // Workgroups are dealt to the eight XCDs round-robin in launch order.  This
 // renumbers a launch of `grid` workgroups (a multiple of 8 * chunk) so that each
@@ -257,7 +274,7 @@ __device__ __forceinline__ bool identity_linear(const DrawData &d) {
     return d.la == 1.0f && d.lb == 0.0f && d.lc == 0.0f && d.ld == 1.0f;
 }
 
-__device__ bool sdf_clip_covers(const uint32_t *paint, uint32_t pc, const DrawData &d, uint32_t tx, uint32_t ty) {
+__device__ bool sdf_clip_covers(Const<uint32_t> paint, uint32_t pc, const DrawData &d, uint32_t tx, uint32_t ty) {
     if (d.sdf_offset == kNone || d.shadow_offset != kNone || d.sdf_len < 9u) return false;
     uint32_t base = d.sdf_offset;
     if (paint_word(paint, pc, base) != TK_SDF_KIND_RECT || !identity_linear(d)) return false;
@@ -269,7 +286,7 @@ __device__ bool sdf_clip_covers(const uint32_t *paint, uint32_t pc, const DrawDa
     return rect_covers_tile(rect, radii, d, tx, ty, 0.5f);
 }
 
-__device__ bool sdf_stroke_empty(const uint32_t *paint, uint32_t pc, const DrawData &d, uint32_t tx, uint32_t ty) {
+__device__ bool sdf_stroke_empty(Const<uint32_t> paint, uint32_t pc, const DrawData &d, uint32_t tx, uint32_t ty) {
     if (d.sdf_offset == kNone || d.shadow_offset != kNone || d.sdf_len < 13u || !identity_linear(d)) return false;
     uint32_t base = d.sdf_offset;
     if (paint_word(paint, pc, base) != 3u) return false;  // SDF_KIND_RECT_STROKE
@@ -297,26 +314,26 @@ __device__ bool sdf_stroke_empty(const uint32_t *paint, uint32_t pc, const DrawD
 __device__ __forceinline__ uint32_t brush_base_of(uint32_t paint_brush_base, const DrawData &d) {
     return paint_brush_base + d.brush_offset;
 }
-__device__ __forceinline__ bool nontransparent_solid(const uint32_t *paint, uint32_t pc, uint32_t pbb, const DrawData &d) {
+__device__ __forceinline__ bool nontransparent_solid(Const<uint32_t> paint, uint32_t pc, uint32_t pbb, const DrawData &d) {
     if (d.brush_offset == kNone) return false;
     uint32_t base = brush_base_of(pbb, d);
     return paint_word(paint, pc, base) == TK_BRUSH_SOLID && paint_word(paint, pc, base + 4u) != 0u;
 }
-__device__ __forceinline__ uint32_t solid_color(const uint32_t *paint, uint32_t pc, uint32_t pbb, const DrawData &d) {
+__device__ __forceinline__ uint32_t solid_color(Const<uint32_t> paint, uint32_t pc, uint32_t pbb, const DrawData &d) {
     return paint_word(paint, pc, brush_base_of(pbb, d) + 4u);
 }
-__device__ bool solid_supported_sdf(const uint32_t *paint, uint32_t pc, uint32_t pbb, const DrawData &d) {
+__device__ bool solid_supported_sdf(Const<uint32_t> paint, uint32_t pc, uint32_t pbb, const DrawData &d) {
     if (!nontransparent_solid(paint, pc, pbb, d) || d.sdf_offset == kNone || d.shadow_offset != kNone || d.sdf_len == 0u)
         return false;
     uint32_t kind = paint_word(paint, pc, d.sdf_offset);
     return kind == TK_SDF_KIND_RECT || kind == 5u || kind == 14u;
 }
-__device__ __forceinline__ uint32_t full_tile_solid(const uint32_t *paint, uint32_t pc, uint32_t pbb, const DrawData &d,
+__device__ __forceinline__ uint32_t full_tile_solid(Const<uint32_t> paint, uint32_t pc, uint32_t pbb, const DrawData &d,
                                                     uint32_t tx, uint32_t ty) {
     return nontransparent_solid(paint, pc, pbb, d) && sdf_clip_covers(paint, pc, d, tx, ty) ? solid_color(paint, pc, pbb, d)
                                                                                             : 0u;
 }
-__device__ __forceinline__ bool full_tile_image(const uint32_t *paint, uint32_t pc, uint32_t pbb, const DrawData &d,
+__device__ __forceinline__ bool full_tile_image(Const<uint32_t> paint, uint32_t pc, uint32_t pbb, const DrawData &d,
                                                 uint32_t tx, uint32_t ty) {
     if (d.brush_offset == kNone) return false;
     uint32_t base = brush_base_of(pbb, d);
@@ -388,13 +405,13 @@ __device__ Particle draw_particle(const CoarseCtx &c, uint32_t batch, uint32_t d
     if (draw_index >= cfg.draw_count || in.draw_batch_ids[draw_index] != batch) return p;
     DrawData d = load_draw(in.draws, cfg.draw_count, draw_index);
     if (draw_has_sdf(d)) {
-        if (d.tag == TK_DRAW_BRUSH && !sdf_stroke_empty(in.paint, cfg.paint_words, d, c.tx, c.ty)) {
+        if (d.tag == TK_DRAW_BRUSH && !sdf_stroke_empty(constant(in.paint), cfg.paint_words, d, c.tx, c.ty)) {
             p.valid = true;
-            uint32_t color = full_tile_solid(in.paint, cfg.paint_words, cfg.paint_brush_base, d, c.tx, c.ty);
+            uint32_t color = full_tile_solid(constant(in.paint), cfg.paint_words, cfg.paint_brush_base, d, c.tx, c.ty);
             if (color != 0u) {
                 p.tag = TK_PTCL_COLOR;
                 p.color = color;
-            } else if (full_tile_image(in.paint, cfg.paint_words, cfg.paint_brush_base, d, c.tx, c.ty)) {
+            } else if (full_tile_image(constant(in.paint), cfg.paint_words, cfg.paint_brush_base, d, c.tx, c.ty)) {
                 p.tag = kPtclImage;
                 p.color = draw_index;
             } else {
@@ -418,9 +435,9 @@ __device__ Particle draw_particle(const CoarseCtx &c, uint32_t batch, uint32_t d
     if (d.tag == TK_DRAW_CLIP) p.tag = TK_PTCL_BEGIN_CLIP;
     else if (d.tag == TK_DRAW_PATH_GLYPH) p.tag = kPtclPathGlyph;
     else if (d.solid_rect != 0u && d.lb == 0.0f && d.lc == 0.0f &&
-             nontransparent_solid(in.paint, cfg.paint_words, cfg.paint_brush_base, d) && range.start == range.end)
+             nontransparent_solid(constant(in.paint), cfg.paint_words, cfg.paint_brush_base, d) && range.start == range.end)
         p.tag = TK_PTCL_COLOR;
-    if (p.tag == TK_PTCL_COLOR) p.color = solid_color(in.paint, cfg.paint_words, cfg.paint_brush_base, d);
+    if (p.tag == TK_PTCL_COLOR) p.color = solid_color(constant(in.paint), cfg.paint_words, cfg.paint_brush_base, d);
     else if (d.tag == TK_DRAW_BRUSH || d.tag == TK_DRAW_PATH_GLYPH) p.color = draw_index;
     return p;
 }
@@ -430,7 +447,7 @@ __device__ __forceinline__ uint32_t particle_class_flags(const CoarseCtx &c, uin
     if (tag == kPtclImage) return kClassSdf;
     if (tag == TK_PTCL_SDF) {
         DrawData d = load_draw(c.in->draws, c.cfg->draw_count, draw_index);
-        if (solid_supported_sdf(c.in->paint, c.cfg->paint_words, c.cfg->paint_brush_base, d)) return kClassSdf;
+        if (solid_supported_sdf(constant(c.in->paint), c.cfg->paint_words, c.cfg->paint_brush_base, d)) return kClassSdf;
     }
     return kClassOther;
 }
@@ -438,7 +455,7 @@ __device__ __forceinline__ uint32_t particle_class_flags(const CoarseCtx &c, uin
 // noop_stack_clip (coarse/emit_stack.hlsli:9-17).
 __device__ bool noop_stack_clip(const CoarseCtx &c, const tk_layer_record &layer, const DrawData &d) {
     if (layer.tag != TK_LAYER_CLIP) return false;
-    if (draw_has_sdf(d)) return sdf_clip_covers(c.in->paint, c.cfg->paint_words, d, c.tx, c.ty);
+    if (draw_has_sdf(d)) return sdf_clip_covers(constant(c.in->paint), c.cfg->paint_words, d, c.tx, c.ty);
     uint32_t bd = draw_backdrop(c.in->paths, c.cfg->path_count, d, c.tx, c.ty, c.tw, c.th);
     if (bd == kNone) return false;  // excluded by stack_wrapper_count before any emission
     tk_segment_range range = c.in->segment_ranges[bd];
@@ -457,7 +474,7 @@ __device__ uint32_t layer_class_bits(const CoarseCtx &c, const tk_layer_record &
     const DrawData d = load_draw(in.draws, cfg.draw_count, layer.draw);
     uint32_t bits = 0u;
     if (draw_has_sdf(d)) {
-        const bool covers = sdf_clip_covers(in.paint, cfg.paint_words, d, c.tx, c.ty);
+        const bool covers = sdf_clip_covers(constant(in.paint), cfg.paint_words, d, c.tx, c.ty);
         if (!covers) bits |= draw_hits_tile(d, c.tx, c.ty, c.tw, c.th) ? kLayerCounted : kLayerInvalid;
         if (!(layer.tag == TK_LAYER_CLIP && covers)) bits |= kLayerEmits;
         return bits | kLayerSdf;
@@ -525,10 +542,10 @@ struct FineDraw {
     Affine inv;
 };
 
-__device__ __forceinline__ FineDraw load_fine_draw(const tk_draw_record *draws, uint32_t count, uint32_t index) {
+__device__ __forceinline__ FineDraw load_fine_draw(Const<tk_draw_record> draws, uint32_t count, uint32_t index) {
     FineDraw f{};
     if (index >= count) return f;
-    const tk_draw_record &r = draws[index];
+    const __attribute__((address_space(4))) tk_draw_record &r = draws[index];
     f.brush_offset = r.brush_offset;
     f.sdf_offset = r.sdf_offset;
     f.shadow_offset = r.sdf_shadow_offset;
@@ -541,7 +558,7 @@ __device__ __forceinline__ FineDraw load_fine_draw(const tk_draw_record *draws, 
     return f;
 }
 
-__device__ __forceinline__ uint32_t sample_draw_brush(const tk_fine_config &cfg, const uint32_t *paint,
+__device__ __forceinline__ uint32_t sample_draw_brush(const tk_fine_config &cfg, Const<uint32_t> paint,
                                                       const FineDraw &d, float x, float y, const AtlasView &atlas) {
     if (blob_word(paint, cfg.paint_words, cfg.paint_brush_base, d.brush_offset) == TK_BRUSH_SOLID)
         return blob_word(paint, cfg.paint_words, cfg.paint_brush_base, d.brush_offset + 4u);
@@ -553,7 +570,7 @@ __device__ __forceinline__ AtlasView atlas_of(const tk_fine_inputs &in) {
     return AtlasView{in.atlas, in.atlas_width, in.atlas_height, in.atlas_pages};
 }
 
-__device__ __forceinline__ float sdf_coverage_from_draw(const tk_fine_config &cfg, const uint32_t *paint,
+__device__ __forceinline__ float sdf_coverage_from_draw(const tk_fine_config &cfg, Const<uint32_t> paint,
                                                         const FineDraw &d, float x, float y) {
     float lx, ly;
     affine_point(d.inv, x, y, lx, ly);
@@ -571,72 +588,265 @@ __device__ __attribute__((noinline)) uint32_t glyph_composite(uint32_t destinati
     return src_over_mask_linear_auto_u8(destination, source, coverage);
 }
 
-// Exact coverage sums of one FILL / BEGIN_CLIP record over a 16x16 tile, built
+// The records whose coverage fine builds from segments.
+__device__ __forceinline__ bool is_coverage_tag(uint32_t tag) {
+    return (tag == TK_PTCL_FILL) | (tag == TK_PTCL_BEGIN_CLIP) | (tag == kPtclPathGlyph);
+}
+
+// The value of lane 0, as a scalar: for values every lane holds alike.
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+
+// The value of lane j (below 64), j by lane.
+__device__ __forceinline__ uint32_t lane_value(uint32_t v, uint32_t j) {
+    return (uint32_t)__builtin_amdgcn_ds_bpermute((int)(j << 2), (int)v);
+}
+
+// Exact coverage sums of up to four consecutive records over a 16x16 tile, built
 // segment by segment instead of pixel by pixel, with 64-bit integer atomics in
-// LDS (exact, so the order of arrival does not matter):
-//   base[row]     += the row's edge term,
-//   run[row][fs]  += dy, where fs = full_start (prefix-summed along the row later),
-//   part[row][x]  += area(x) * dy for the straddled pixels x in [partial_start, fs).
-struct CoverageAcc {
-    long long base[16];
-    long long run[256];
-    long long part[256];
+// LDS (exact, so the order of arrival does not matter).  Each record has one
+// difference array per pixel row, whose prefix sum along the row is the pixel's
+// coverage: a row's edge term is added at x = 0, a straddled pixel's
+// area(x) * dy as the step from its left neighbour's, and dy less the last of
+// them at full_start.  So a pixel reads and clears one word (three with the terms
+// kept apart), and four records take one barrier.
+constexpr uint32_t kGroup = 4u;
+struct GroupCoverage {
+    long long d[kGroup][256];
+};
+// The group's segments laid end to end: record 0's are items [0, end0), record 1's
+// [end0, end1) and so on, and item q of record g is segment first<g> + q.  (Named
+// fields: an array indexed in an unrolled loop goes through scratch memory.)
+struct GroupSegments {
+    uint32_t first0, first1, first2, first3, end0, end1, end2, end3;
 };
 
-// All terms of segments [0, n) of one record: lane l takes (segment l / 16,
-// row l % 16), evaluates segment_row_parts for that row once, and adds its terms.
-__device__ __forceinline__ void accumulate_record(const tk_line_segment *segs, uint32_t n, CoverageAcc &acc,
-                                                  uint32_t lane) {
-    const uint32_t row = lane & 15u;
-    // A 32-bit index (n is 32-bit): no 64-bit counter compare and step per pass.
-    for (uint32_t i = lane >> 4; i < n; i += 16u) {
-        const tk_line_segment seg = segs[i];
-        const RowParts p = segment_row_parts(seg.p0x, seg.p0y, seg.p1x, seg.p1y, seg.y_edge, row);
-        if (p.edge != 0.0f) atomicAdd((unsigned long long *)&acc.base[row], (unsigned long long)coverage_fixed(p.edge));
-        if (p.dy != 0.0f) {
-            const int fs = clamp_cell16(ceilf(p.xmax));
-            const int ps = clamp_cell16(floorf(p.xmin));
-            if (fs < 16) atomicAdd((unsigned long long *)&acc.run[row * 16u + fs], (unsigned long long)coverage_fixed(p.dy));
-            float xf = (float)ps;  // exact: 0..16
-            for (int x = ps; x < fs; ++x, xf += 1.0f)
-                atomicAdd((unsigned long long *)&acc.part[row * 16u + x],
-                          (unsigned long long)coverage_fixed(segment_area_at_f(p.xmin, p.xmax, xf) * p.dy));
+__device__ __forceinline__ void add_coverage(long long *word, int32_t term) {
+    atomicAdd((unsigned long long *)word, (unsigned long long)(long long)term);
+}
+
+// One row of a segment into its row of the difference array (dy: the row's terms
+// fit 32 bits, |area * dy| < 2).
+__device__ __forceinline__ void accumulate_row(const tk_line_segment &seg, float slope, uint32_t row, long long *d) {
+    const RowParts p = segment_row_parts(seg.p0x, seg.p0y, seg.p1x, seg.p1y, slope, row);
+    if (p.dy == 0.0f) return;
+    const int fs = clamp_cell16(ceilf(p.xmax));
+    const int ps = clamp_cell16(floorf(p.xmin));
+    const float dy = p.dy * kCoverageOne;  // exact; area * dy then rounds as area * p.dy does
+    int32_t last = 0;
+    if (ps < fs) {
+        float xf = (float)ps;  // exact: 0..16
+        const float xmin = p.xmin - xf, xmax = p.xmax - xf;
+        if (xmin >= 0.0f && xmax <= 1.0f) {  // inside one pixel (a vertical part included): no quotient
+            last = coverage_trunc(fmaf(-0.5f, xmin + xmax, 1.0f) * dy);
+            add_coverage(d + ps, last);
+        } else {
+            const float width = p.xmax - p.xmin;
+            const bool plain = plain_width(width);
+            const float recip = __builtin_amdgcn_rcpf(width);
+            for (int x = ps; x < fs; ++x, xf += 1.0f) {
+                const float area = plain ? segment_area_across(p.xmin, p.xmax, xf, recip)
+                                         : segment_area_at_f(p.xmin, p.xmax, xf);
+                const int32_t t = coverage_trunc(area * dy);
+                add_coverage(d + x, t - last);
+                last = t;
+            }
         }
+    }
+    if (fs < 16) add_coverage(d + fs, coverage_trunc(dy) - last);
+}
+
+// All terms of a group's segments.  Eight lanes take a segment, one per row from
+// the first it crosses: a segment of a flattened curve crosses about three of a
+// tile's 16 rows, and sixteen lanes a segment (one per tile row) ran 2.2 wave
+// passes a record where this runs about 0.9 (sixteen lanes again: 1.79 -> 1.95 ms a
+// frame of 50 000 paths; four: the same there, 2.18 -> 2.34 ms a frame of 200 000
+// polygons, whose segments are longer).  A segment that meets the tile's left edge
+// has its edge term in every row from there down, added apart so that those rows
+// run only that.
+constexpr uint32_t kRowLanes = 8u;
+__device__ __forceinline__ void accumulate_group(const tk_line_segment *segs, const GroupSegments r,
+                                                 GroupCoverage &acc, uint32_t lane) {
+    // A 32-bit index (counts are 32-bit): no 64-bit counter compare and step per pass.
+    for (uint32_t q = lane / kRowLanes; q < r.end3; q += 256u / kRowLanes) {
+        uint32_t at = r.first0, record = 0u;
+        if (q >= r.end0) at = r.first1, record = 1u;
+        if (q >= r.end1) at = r.first2, record = 2u;
+        if (q >= r.end2) at = r.first3, record = 3u;
+        const tk_line_segment seg = segs[at + q];
+        long long *rows = acc.d[record];
+        const float dx = seg.p1x - seg.p0x, dy = seg.p1y - seg.p0y;
+        uint32_t first = (uint32_t)clamp_cell16(floorf(fminf(seg.p0y, seg.p1y)));
+        uint32_t end = (uint32_t)clamp_cell16(ceilf(fmaxf(seg.p0y, seg.p1y)));
+        if (!(dy == dy)) first = 0u, end = 16u;  // an end that is no number: every row
+        const float slope = dx / dy;
+        const uint32_t sub = lane & (kRowLanes - 1u);
+        for (uint32_t row = first + sub; row < end; row += kRowLanes)
+            accumulate_row(seg, slope, row, rows + row * 16u);
+        if (seg.y_edge < 16.0f)
+            for (uint32_t row = (uint32_t)clamp_cell16(floorf(seg.y_edge)) + sub; row < 16u; row += kRowLanes)
+                add_coverage(rows + row * 16u, coverage_trunc(segment_row_edge(dx, seg.y_edge, row) * kCoverageOne));
     }
 }
 
-// Inclusive prefix sum over each 16-lane DPP row (one pixel row of the tile).
+__device__ __forceinline__ void clear_coverage(GroupCoverage &acc, uint32_t lane) {
+#pragma unroll
+    for (uint32_t g = 0; g < kGroup; ++g) acc.d[g][lane] = 0;
+}
+
+// Inclusive prefix sum over each 16-lane DPP row (one pixel row of the tile): four
+// steps of an add with carry whose first operand comes from the lane 1, 2, 4 and 8
+// to the left (0 past the row's end).  Written out because the compiler moves the
+// operands first and makes two 64-bit adds a step (20 instructions for 8); a DPP
+// operand must be two instructions old, hence the s_nop.
 __device__ __forceinline__ long long row16_inclusive_sum(long long v) {
     uint32_t lo = (uint32_t)v, hi = (uint32_t)((unsigned long long)v >> 32);
-#define TK_ROW_SHR_STEP(ctrl)                                                                   \
-    {                                                                                           \
-        uint32_t slo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)lo, ctrl, 0xf, 0xf, true); \
-        uint32_t shi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)hi, ctrl, 0xf, 0xf, true); \
-        uint32_t nlo = lo + slo;                                                                \
-        hi = hi + shi + (nlo < lo ? 1u : 0u);                                                   \
-        lo = nlo;                                                                               \
-    }
-    TK_ROW_SHR_STEP(0x111)  // row_shr:1
-    TK_ROW_SHR_STEP(0x112)  // row_shr:2
-    TK_ROW_SHR_STEP(0x114)  // row_shr:4
-    TK_ROW_SHR_STEP(0x118)  // row_shr:8
-#undef TK_ROW_SHR_STEP
+#define TK_ROW_SHR_ADD(n)                                                                     \
+    "v_add_co_u32_dpp %0, vcc, %0, %0 row_shr:" #n " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+    "v_addc_co_u32_dpp %1, vcc, %1, %1, vcc row_shr:" #n " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+    asm("s_nop 1\n\t" TK_ROW_SHR_ADD(1) "s_nop 0\n\t" TK_ROW_SHR_ADD(2) "s_nop 0\n\t" TK_ROW_SHR_ADD(4)
+        "s_nop 0\n\t" TK_ROW_SHR_ADD(8)
+        : "+v"(lo), "+v"(hi)
+        :
+        : "vcc");
+#undef TK_ROW_SHR_ADD
     return (long long)(((unsigned long long)hi << 32) | lo);
 }
 
-// Reads this lane's pixel (x = lane & 15, y = lane >> 4) out of `acc` and clears
-// the entries it owns.  All 256 lanes call it together, after the barrier that
-// follows accumulate_record; the 16 lanes of a pixel row share one wave, so the
-// row's base word is read by all of them before lane x = 0 clears it.
-__device__ __forceinline__ float take_coverage(CoverageAcc &acc, int32_t backdrop, uint32_t lane) {
-    const uint32_t row = lane >> 4;
-    const long long base = acc.base[row] + backdrop_fixed(backdrop);
-    const long long running = row16_inclusive_sum(acc.run[lane]);
-    const long long partial = acc.part[lane];
-    acc.run[lane] = 0;
-    acc.part[lane] = 0;
-    if ((lane & 15u) == 0u) acc.base[row] = 0;
-    return fixed_to_float(base + running + partial);
+// Reads this lane's pixel (x = lane & 15, y = lane >> 4) of one record out of its
+// difference array and clears the lane's word.  All 256 lanes call it together,
+// after the barrier that follows accumulate_group.
+__device__ __forceinline__ float take_coverage(long long *d, int32_t backdrop, uint32_t lane) {
+    const long long v = row16_inclusive_sum(d[lane]);
+    d[lane] = 0;
+    return fixed_to_float(v + backdrop_fixed(backdrop));
+}
+
+// Segments a record's coverage is summed from (0: its backdrop alone).
+__device__ __forceinline__ uint32_t record_segments(uint32_t start, uint32_t end, uint32_t capacity) {
+    return max(min(end, capacity), start) - start;
+}
+
+// One record of a tile's walk, as scalars.
+struct WalkRecord {
+    uint32_t tag, fill_rule, color, kind;  // kind: the tile kind word's kind of its stream
+    uint32_t mark;                         // what mark(kind, tag, color) gave it (0-15)
+    int32_t backdrop;
+    uint32_t index;                        // its place in the PTCL
+    bool covered;                          // its coverage has segments, summed in `d`
+    bool ends;                             // the last record of its stream
+    long long *d;
+};
+
+// Walks a tile's streams, all batches in order: visit(record) for every record up
+// to each stream's END, with the coverage sums of the records `covers(kind, tag,
+// color)` asks for built four records at a time.  Streams are short (two or three
+// records a batch in a scene of nested layers), so the groups run across them:
+// every wave holds a window of 64 consecutive records, one per lane, and reads
+// what steers the walk with v_readlane.  The workgroup's waves hold the same
+// window, so control flow and barriers are the workgroup's.  mark(kind, tag, color)
+// looks at a record by lane, so that a gather answers for 64 of them.
+template <class Covers, class Mark, class Visit>
+__device__ __forceinline__ void walk_tile(const SceneView &v, const uint32_t *tile_kinds,
+                                          const tk_segment_range *tile_ranges, const tk_ptcl_record *ptcl,
+                                          uint32_t ptcl_capacity, const tk_line_segment *segs,
+                                          uint32_t segment_capacity, GroupCoverage *cov_acc, uint32_t &sel,
+                                          Covers covers, Mark mark, Visit visit) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t q1 = uniform(v.q1);
+    for (uint32_t b0 = uniform(v.q0); b0 < q1; b0 += 64u) {
+        // The streams of 64 batches, one per lane: only where each ends in their
+        // concatenation stays in a register.
+        const auto stream = [&](uint32_t batch, uint32_t &kind, uint32_t &start) {
+            const size_t idx = table_index(v, batch);
+            const uint32_t word = tile_kinds[idx];
+            const tk_segment_range r = tile_ranges[idx];
+            kind = word & TK_TILE_KIND_MASK;
+            start = r.start + (word >> TK_TILE_PREFIX_SHIFT);
+            const uint32_t end = min(r.end, ptcl_capacity);
+            return kind != TK_TILE_KIND_EMPTY && end > start ? end - start : 0u;
+        };
+        uint32_t len = 0u, kind, start;
+        if (b0 + lane < q1) len = stream(b0 + lane, kind, start);
+        const uint32_t upto = wave_inclusive_scan_dpp(len);
+        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)upto, 63);
+        bool stale = false;  // the window starts inside a stream that has ended
+        for (uint32_t w0 = 0u; w0 < total; w0 += 64u) {
+            // Lane r takes record w0 + r: its stream is the first that ends past it.
+            const uint32_t at = w0 + lane;
+            uint32_t j = 0u;
+#pragma unroll
+            for (uint32_t step = 32u; step >= 1u; step >>= 1)
+                if (lane_value(upto, j + step - 1u) <= at) j += step;
+            j = min(j, 63u);
+            const uint32_t end_at = lane_value(upto, j);
+            uint32_t my_kind = TK_TILE_KIND_EMPTY, index = 0u, off = 0u;
+            tk_ptcl_record r{};
+            if (at < total) {
+                off = at - (end_at - stream(b0 + j, my_kind, index));
+                index += off;
+                r = ptcl[index];
+            }
+            const bool last = at + 1u == end_at;
+            // A record after its stream's END does not count.
+            const uint64_t ended = __ballot(at < total && r.tag == TK_PTCL_END), firsts = __ballot(at < total && off == 0u);
+            const uint64_t here = firsts & (lanes_below(lane) | (1ull << lane));
+            const uint32_t from = here ? 63u - (uint32_t)__builtin_clzll(here) : 0u;
+            const bool dead = (ended & lanes_below(lane) & ~lanes_below(from)) != 0u || (here == 0u && stale);
+            const bool live = at < total && !dead;
+            stale = __builtin_amdgcn_readlane((int)(dead || r.tag == TK_PTCL_END), 63) != 0;
+            const uint32_t n =
+                live && covers(my_kind, r.tag, r.color) ? record_segments(r.segment_start, r.segment_end, segment_capacity) : 0u;
+            const uint32_t meta = (r.tag & 0xFFu) | (my_kind << 8) | (r.fill_rule == TK_FILL_EVEN_ODD ? 1u << 16 : 0u) |
+                                  (last || r.tag == TK_PTCL_END ? 1u << 17 : 0u) |
+                                  (live ? mark(my_kind, r.tag, r.color) << 18 : 0u);
+            uint64_t todo = __ballot(live), fills = __ballot(n != 0u);
+            while (todo) {
+                // The next four covered records and every record before the fifth.
+                GroupSegments group;
+                uint32_t sum = 0u;
+                const auto take = [&](uint32_t &first, uint32_t &end) {
+                    const int i = fills ? __builtin_ctzll(fills) : 0;
+                    const uint32_t c = fills ? (uint32_t)__builtin_amdgcn_readlane((int)n, i) : 0u;
+                    first = (uint32_t)__builtin_amdgcn_readlane((int)r.segment_start, i) - sum;
+                    sum += c;
+                    end = sum;
+                    fills &= fills - 1u;
+                };
+                const uint64_t covered = fills;
+                take(group.first0, group.end0);
+                take(group.first1, group.end1);
+                take(group.first2, group.end2);
+                take(group.first3, group.end3);
+                uint64_t range = fills ? todo & ((fills & (0ull - fills)) - 1u) : todo;
+                todo &= ~range;
+                GroupCoverage &acc = cov_acc[sel];
+                if (sum != 0u) {
+                    accumulate_group(segs, group, acc, threadIdx.x);
+                    sel ^= 1u;
+                    __syncthreads();
+                }
+                uint32_t g = 0u;
+                while (range) {
+                    const int i = __builtin_ctzll(range);
+                    range &= range - 1u;
+                    const uint32_t m = (uint32_t)__builtin_amdgcn_readlane((int)meta, i);
+                    WalkRecord rec;
+                    rec.tag = m & 0xFFu;
+                    rec.kind = (m >> 8) & 0xFFu;
+                    rec.fill_rule = (m >> 16) & 1u;
+                    rec.ends = ((m >> 17) & 1u) != 0u;
+                    rec.mark = m >> 18;
+                    rec.backdrop = __builtin_amdgcn_readlane(r.backdrop, i);
+                    rec.color = (uint32_t)__builtin_amdgcn_readlane((int)r.color, i);
+                    rec.index = (uint32_t)__builtin_amdgcn_readlane((int)index, i);
+                    rec.covered = ((covered >> i) & 1ull) != 0u;
+                    rec.d = acc.d[g];
+                    visit(rec);
+                    g += rec.covered ? 1u : 0u;
+                }
+            }
+        }
+    }
 }
 
 }  // namespace
@@ -1028,8 +1238,6 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_cumsum(tk_args_cumsum a) 
 // entries, so per-batch particle counts and emission offsets come from ballots.
 // ---------------------------------------------------------------------------
 
-__device__ __forceinline__ uint64_t lanes_below(uint32_t lane) { return lane ? (~0ull >> (64u - lane)) : 0ull; }
-
 // stack_wrapper_count with the layers of one batch evaluated across the wave:
 // the stack is invalid when any layer rejects the tile, otherwise the count of
 // layers that are not no-ops.
@@ -1046,7 +1254,7 @@ __device__ uint32_t stack_wrapper_count_wave(const CoarseCtx &c, uint32_t batch,
             const tk_layer_record layer = in.layers[i];
             const DrawData d = load_draw(in.draws, cfg.draw_count, layer.draw);
             if (draw_has_sdf(d)) {
-                if (!sdf_clip_covers(in.paint, cfg.paint_words, d, c.tx, c.ty)) {
+                if (!sdf_clip_covers(constant(in.paint), cfg.paint_words, d, c.tx, c.ty)) {
                     if (!draw_hits_tile(d, c.tx, c.ty, c.tw, c.th)) invalid = true;
                     else counted = true;
                 }
@@ -1657,221 +1865,234 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_coarse_emit_scenes_persis
 
 // The colour sample_draw_brush returns for a draw whose brush does not depend on
 // the pixel (solid, and the kinds sample_brush maps to the header colour or to
-// 0), so that a fill reads one word pair instead of the draw record and then
-// its brush header (shared/brush/sample.hlsli:15-42).
+// 0), so that a fill reads one table entry instead of the draw record and then
+// its brush header (shared/brush/sample.hlsli:15-42); the entry holds the colour's
+// bytes as floats too, which the blend takes from scalar registers.
 extern "C" __global__ __launch_bounds__(256) void tk_k_draw_brush(tk_args_draw_brush a) {
     const uint32_t d = blockIdx.x * 256u + threadIdx.x;
     if (d >= a.draw_count) return;
     const uint32_t offset = a.draws[d].brush_offset;
-    const uint32_t kind = blob_word(a.paint, a.paint_words, a.paint_brush_base, offset);
-    const uint32_t color = blob_word(a.paint, a.paint_words, a.paint_brush_base, offset + 4u);
+    const uint32_t kind = blob_word(constant(a.paint), a.paint_words, a.paint_brush_base, offset);
+    const uint32_t color = blob_word(constant(a.paint), a.paint_words, a.paint_brush_base, offset + 4u);
     uint32_t flag = 1u, value = color;
     if (kind == TK_BRUSH_LINEAR || kind == TK_BRUSH_RADIAL || kind == TK_BRUSH_SWEEP || kind == TK_BRUSH_FOUR_CORNER ||
         kind == TK_BRUSH_IMAGE)
         flag = 0u, value = 0u;
     else if (kind == 6u)  // BRUSH_PATTERN
         value = 0u;
-    a.table[2u * d] = flag;
-    a.table[2u * d + 1u] = value;
+    uint4 *entry = reinterpret_cast<uint4 *>(a.table + (size_t)d * TK_DRAW_BRUSH_WORDS);
+    entry[0] = make_uint4(flag, value, 0u, 0u);
+    entry[1] = make_uint4(__float_as_uint((float)(value & 255u)), __float_as_uint((float)((value >> 8) & 255u)),
+                          __float_as_uint((float)((value >> 16) & 255u)), __float_as_uint((float)(value >> 24)));
 }
+
+// Marks of fine's walk.
+constexpr uint32_t kFlatTranslucent = 1u, kFlatOpaque = 2u;
 
 // fine_tile_main for every batch: one 256-lane workgroup per tile, one lane per
 // pixel.  Between batches the pixel goes through the RGBA8 store/load round trip
 // the reference performs on its target.  kScenes: a batch of scenes.
+//
+// Bound by VALU issue on large frames and by a tile's chain of records on small
+// ones.  So everything that steers the walk is scalar (walk_tile; draws, paint and
+// brush entries come by scalar loads), coverage is built for four records at a time
+// (their segments fill the four waves' lanes together, their loads are in flight
+// together, one barrier), and a record reads one LDS word per pixel.  Before, one
+// record at a time through vector loads and exec masks: 65 536 tiles of 2.4 M fills
+// with 1.8 segments each 3.12 -> 1.28 ms, 16 384 tiles of 0.61 M fills with 11
+// under 32 clips 1.34 -> 0.77 ms, 256 tiles of 17 600 fills 386 -> 208 us.
 template <bool kScenes, bool kPersistent>
 __device__ __forceinline__ void fine_tile(const tk_args_fine &a) {
     // Clip levels beyond the four register slots: clip_spill_depth * 256 bytes of
     // dynamic LDS, sized by the launch.
     extern __shared__ uint8_t clip_spill[];
-    __shared__ CoverageAcc cov_acc[2];  // double-buffered: one barrier per fill
-    __shared__ uint32_t batch_kind[256];
-    __shared__ tk_segment_range batch_range[256];
+    __shared__ GroupCoverage cov_acc[2];  // double-buffered: one barrier per group
     __shared__ uint32_t s_item;
     const tk_fine_config &cfg = a.cfg;
     const uint32_t columns = a.list.columns;  // table columns: listed tiles, or every tile
     const uint32_t lane = threadIdx.x;
+    const Const<uint32_t> paint = constant(a.in.paint);
+    const Const<uint32_t> brushes = constant(a.draw_brush);
 
-    // Cleared once per workgroup: each take_coverage clears the entries it read.
-    cov_acc[0].run[lane] = 0;
-    cov_acc[0].part[lane] = 0;
-    cov_acc[1].run[lane] = 0;
-    cov_acc[1].part[lane] = 0;
-    if (lane < 16u) {
-        cov_acc[0].base[lane] = 0;
-        cov_acc[1].base[lane] = 0;
-    }
+    // Cleared once per workgroup: each take_coverage clears the words it read.
+    clear_coverage(cov_acc[0], lane);
+    clear_coverage(cov_acc[1], lane);
+    __syncthreads();
     uint32_t acc_sel = 0u;
 
     auto tile = [&](uint32_t column) {
         const SceneView v = scene_view<kScenes>(a.scenes, column, columns, cfg.batch_count, cfg.tiles_width,
                                                 cfg.tiles_height, cfg.width, cfg.height, cfg.clear_color);
-        const uint32_t tile_ix = a.list.tiles ? a.list.tiles[column] : v.local;  // the tile of its canvas
+        const uint32_t tile_ix = uniform(a.list.tiles ? a.list.tiles[column] : v.local);  // the tile of its canvas
         if (tile_ix >= cfg.tile_count) return;
         const uint32_t lx = lane & 15u, ly = lane >> 4;
         const uint32_t gx = (tile_ix % v.tw) * 16u + lx;
         const uint32_t gy = (tile_ix / v.tw) * 16u + ly;
         const float sx = (float)gx + 0.5f, sy = (float)gy + 0.5f;
-        const uint32_t *paint = a.in.paint;
-        const tk_ptcl_record *ptcl = a.in.ptcl;
-        const tk_line_segment *segs = a.in.segments;
-
         Px pixel = rgba8_to_unorm(v.clear);
-        for (uint32_t b0 = v.q0; b0 < v.q1; b0 += 256u) {
-          // This tile's (kind, range) word pairs of up to 256 batches, one load per lane.
-          __syncthreads();
-          if (b0 + lane < v.q1) {
-              const size_t idx = table_index(v, b0 + lane);
-              batch_kind[lane] = a.in.tile_kinds[idx];
-              batch_range[lane] = a.in.tile_ptcl_ranges[idx];
-          }
-          __syncthreads();
-          const uint32_t chunk = min(256u, v.q1 - b0);
-          for (uint32_t bj = 0; bj < chunk; ++bj) {
-            const uint32_t kind_word = batch_kind[bj];
-            const uint32_t kind = kind_word & TK_TILE_KIND_MASK;
-            if (kind == TK_TILE_KIND_EMPTY) continue;
-            const tk_segment_range r = batch_range[bj];
-            const uint32_t pstart = r.start + (kind_word >> TK_TILE_PREFIX_SHIFT);
-            const uint32_t pend = min(r.end, cfg.ptcl_capacity);
-            if (kind == TK_TILE_KIND_INTERPRETER) {
-                uint32_t clip_mask = 255u, clip_depth = 0u;
-                uint32_t cs0 = 255u, cs1 = 255u, cs2 = 255u, cs3 = 255u;
-                auto push_clip = [&](uint32_t mask) {
-                    uint32_t dd = clip_depth;
-                    if (dd == 0u) { cs0 = mask; clip_depth = 1u; }
-                    else if (dd == 1u) { cs1 = mask; clip_depth = 2u; }
-                    else if (dd == 2u) { cs2 = mask; clip_depth = 3u; }
-                    else if (dd == 3u) { cs3 = mask; clip_depth = 4u; }
-                    else {
-                        uint32_t spill = dd - 4u;
-                        if (spill < cfg.clip_spill_depth) {
-                            clip_spill[spill * 256u + lane] = (uint8_t)mask;
-                            clip_depth = dd + 1u;
-                        } else if (a.in.status) {
-                            atomicOr(a.in.status, 2u);  // deeper than the scene's declared clip depth
-                        }
-                    }
-                };
-                for (uint32_t pi = pstart; pi < pend; ++pi) {
-                    const tk_ptcl_record rec = ptcl[pi];
-                    const uint32_t tag = rec.tag;
-                    if (tag == TK_PTCL_END) break;
-                    if (tag == TK_PTCL_COLOR) {
-                        if (clip_mask != 0u) {
-                            if (clip_mask == 255u && premul_opaque(rec.color)) pixel = rgba8_to_unorm(rec.color);
-                            else pixel = src_over_premul_unorm(pixel, scale_premul_u8_to_unorm(rec.color, clip_mask));
-                        }
-                    } else if (tag == kPtclImage) {
-                        // interpreter.hlsli:65-74: an image covering the whole tile
-                        if (clip_mask != 0u) {
-                            const uint32_t color = sample_draw_brush(
-                                cfg, paint, load_fine_draw(a.in.draws, cfg.draw_count, rec.color), sx, sy, atlas_of(a.in));
-                            if (clip_mask == 255u && premul_opaque(color)) pixel = rgba8_to_unorm(color);
-                            else pixel = src_over_premul_unorm(pixel, scale_premul_u8_to_unorm(color, clip_mask));
-                        }
-                    } else if (tag == TK_PTCL_SDF) {
-                        if (clip_mask != 0u) {
-                            FineDraw d = load_fine_draw(a.in.draws, cfg.draw_count, rec.color);
-                            float coverage = sdf_coverage_from_draw(cfg, paint, d, sx, sy);
-                            uint32_t alpha = combine_alpha(coverage_to_u8(coverage), clip_mask);
-                            if (alpha != 0u) {
-                                uint32_t color = sample_draw_brush(cfg, paint, d, sx, sy, atlas_of(a.in));
-                                if (alpha == 255u && premul_opaque(color)) pixel = rgba8_to_unorm(color);
-                                else pixel = src_over_premul_unorm(pixel, scale_premul_u8_to_unorm(color, alpha));
-                            }
-                        }
-                    } else if (tag == TK_PTCL_END_CLIP) {
-                        if (clip_depth > 0u) {
-                            clip_depth -= 1u;
-                            if (clip_depth == 0u) clip_mask = cs0;
-                            else if (clip_depth == 1u) clip_mask = cs1;
-                            else if (clip_depth == 2u) clip_mask = cs2;
-                            else if (clip_depth == 3u) clip_mask = cs3;
-                            else {
-                                uint32_t spill = clip_depth - 4u;
-                                if (spill < cfg.clip_spill_depth) clip_mask = clip_spill[spill * 256u + lane];
-                            }
-                        } else {
-                            clip_mask = 255u;
-                        }
-                    } else if (tag == TK_PTCL_BEGIN_SDF_CLIP) {
-                        uint32_t parent = clip_mask, alpha = 0u;
-                        if (parent != 0u) {
-                            FineDraw d = load_fine_draw(a.in.draws, cfg.draw_count, rec.color);
-                            alpha = coverage_to_u8(sdf_coverage_from_draw(cfg, paint, d, sx, sy));
-                        }
-                        push_clip(parent);
-                        clip_mask = combine_alpha(parent, alpha);
-                    } else if (tag == TK_PTCL_FILL || tag == TK_PTCL_BEGIN_CLIP || tag == kPtclPathGlyph) {
-                        const uint32_t s0 = rec.segment_start, s1 = min(rec.segment_end, cfg.segment_capacity);
-                        const uint32_t n = s1 > s0 ? s1 - s0 : 0u;
-                        // Issued before the coverage work so that its latency overlaps it.
-                        uint32_t brush_flag = 0u, brush_color = 0u;
-                        if (tag != TK_PTCL_BEGIN_CLIP && rec.color < cfg.draw_count) {
-                            brush_flag = a.draw_brush[2u * rec.color];
-                            brush_color = a.draw_brush[2u * rec.color + 1u];
-                        }
-                        CoverageAcc &acc = cov_acc[acc_sel];
-                        acc_sel ^= 1u;
-                        accumulate_record(segs + s0, n, acc, lane);
-                        __syncthreads();
-                        const float v = take_coverage(acc, rec.backdrop, lane);
-                        uint32_t alpha = coverage_to_alpha(v, rec.fill_rule);
-                        if (tag == TK_PTCL_BEGIN_CLIP) {
-                            push_clip(clip_mask);
-                            clip_mask = combine_alpha(clip_mask, alpha);
-                        } else {
-                            uint32_t masked = combine_alpha(alpha, clip_mask);
-                            if (masked != 0u) {
-                                uint32_t color = brush_color;
-                                if (brush_flag == 0u)
-                                    color = sample_draw_brush(cfg, paint, load_fine_draw(a.in.draws, cfg.draw_count, rec.color),
-                                                              sx, sy, atlas_of(a.in));
-                                if (tag == kPtclPathGlyph)  // text compositing (interpreter.hlsli:205-206)
-                                    pixel = rgba8_to_unorm(glyph_composite(unorm_to_rgba8(pixel), color, masked));
-                                else if (masked == 255u && premul_opaque(color)) pixel = rgba8_to_unorm(color);
-                                else pixel = src_over_premul_unorm(pixel, scale_premul_u8_to_unorm(color, masked));
-                            }
-                        }
-                    }
-                    // Glyph-image, opacity and blend records are not produced on this path.
-                }
-            } else if (kind == TK_TILE_KIND_COLOR) {
-                for (uint32_t pi = pstart; pi < pend; ++pi) {
-                    const tk_ptcl_record rec = ptcl[pi];
-                    if (rec.tag == TK_PTCL_END) break;
-                    if (premul_opaque(rec.color)) pixel = rgba8_to_unorm(rec.color);
-                    else pixel = src_over_premul_unorm(pixel, rgba8_to_unorm(rec.color));
-                }
-            } else {  // TILE_KIND_SDF / TILE_KIND_MIXED
-                for (uint32_t pi = pstart; pi < pend; ++pi) {
-                    const tk_ptcl_record rec = ptcl[pi];
-                    if (rec.tag == TK_PTCL_END) break;
-                    if (rec.tag == TK_PTCL_COLOR) {
-                        if (premul_opaque(rec.color)) pixel = rgba8_to_unorm(rec.color);
-                        else pixel = src_over_premul_unorm(pixel, rgba8_to_unorm(rec.color));
-                    } else if (rec.tag == kPtclImage) {
-                        const uint32_t color = sample_draw_brush(
-                            cfg, paint, load_fine_draw(a.in.draws, cfg.draw_count, rec.color), sx, sy, atlas_of(a.in));
-                        if (premul_opaque(color)) pixel = rgba8_to_unorm(color);
-                        else pixel = src_over_premul_unorm(pixel, rgba8_to_unorm(color));
-                    } else {
-                        FineDraw d = load_fine_draw(a.in.draws, cfg.draw_count, rec.color);
-                        float coverage = 0.0f;
-                        if ((int32_t)gx >= d.pb[0] && (int32_t)gy >= d.pb[1] && (int32_t)gx < d.pb[2] && (int32_t)gy < d.pb[3])
-                            coverage = sdf_coverage_from_draw(cfg, paint, d, sx, sy);
-                        uint32_t alpha = coverage_to_u8(coverage);
-                        if (alpha != 0u) {
-                            uint32_t color = blob_word(paint, cfg.paint_words, cfg.paint_brush_base, d.brush_offset + 4u);
-                            if (alpha == 255u && premul_opaque(color)) pixel = rgba8_to_unorm(color);
-                            else pixel = src_over_premul_unorm(pixel, scale_premul_u8_to_unorm(color, alpha));
-                        }
-                    }
+        uint32_t clip_mask = 255u, clip_depth = 0u;
+        uint32_t cs0 = 255u, cs1 = 255u, cs2 = 255u, cs3 = 255u;
+        auto push_clip = [&](uint32_t mask) {
+            uint32_t dd = clip_depth;
+            if (dd == 0u) { cs0 = mask; clip_depth = 1u; }
+            else if (dd == 1u) { cs1 = mask; clip_depth = 2u; }
+            else if (dd == 2u) { cs2 = mask; clip_depth = 3u; }
+            else if (dd == 3u) { cs3 = mask; clip_depth = 4u; }
+            else {
+                uint32_t spill = dd - 4u;
+                if (spill < cfg.clip_spill_depth) {
+                    clip_spill[spill * 256u + lane] = (uint8_t)mask;
+                    clip_depth = dd + 1u;
+                } else if (a.in.status) {
+                    atomicOr(a.in.status, 2u);  // deeper than the scene's declared clip depth
                 }
             }
-            pixel = rgba8_to_unorm(unorm_to_rgba8(pixel));
-          }
-        }
+        };
+        // A fill of a flat colour that is not transparent, in a stream with coverage:
+        // most records.  paint_record below would do the same, through the branches
+        // and copies that its other kinds need (2.2 times the instructions).
+        const auto paint_flat_fill = [&](const WalkRecord &rec) {
+            const Const<uint32_t> entry = brushes + (size_t)rec.color * TK_DRAW_BRUSH_WORDS;
+            const float r = asfloat(entry[4]), g = asfloat(entry[5]), b = asfloat(entry[6]), a8 = asfloat(entry[7]);
+            float v = (float)rec.backdrop;
+            if (rec.covered) v = take_coverage(rec.d, rec.backdrop, lane);
+            float masked = fill_u8_uniform(v, rec.fill_rule);
+            if (clip_depth != 0u) masked = (float)combine_alpha_u8((uint32_t)masked, clip_mask);  // depth 0: a full mask
+            // src_over_premul_unorm of the scaled colour, whose alpha is below 1 here; where
+            // `masked` is 0 it leaves the pixel as it is.
+            const float scale = masked * (1.0f / 65025.0f);
+            const float src_a = a8 * scale, inv = 1.0f - src_a;
+            const Px over{r * scale + pixel.r * inv, g * scale + pixel.g * inv, b * scale + pixel.b * inv,
+                          src_a + pixel.a * inv};
+            if (rec.mark == kFlatOpaque) {  // a full mask replaces the pixel
+                const bool full = masked == 255.0f;
+                pixel = Px{full ? r * kChannelScale : over.r, full ? g * kChannelScale : over.g,
+                           full ? b * kChannelScale : over.b, full ? a8 * kChannelScale : over.a};
+            } else {
+                pixel = over;
+            }
+        };
+        const auto paint_record = [&](const WalkRecord &rec) {
+            // COLOR tiles hold colour records only; SDF and MIXED tiles colours, images
+            // and solid SDF rectangles (fine/specialized.hlsli:19-111): no clips, no coverage.
+            const bool special = rec.kind != TK_TILE_KIND_INTERPRETER;
+            uint32_t tag = rec.tag;
+            if (special) {
+                if (rec.kind == TK_TILE_KIND_COLOR) tag = TK_PTCL_COLOR;
+                else if (tag != TK_PTCL_COLOR && tag != kPtclImage) tag = TK_PTCL_SDF;
+            }
+            // What the record draws: a colour every pixel shares (flat, its bytes as
+            // floats in flat_*) or its draw's brush, under `masked` (0-255).
+            uint32_t masked = clip_mask, color = rec.color;
+            bool flat = true;
+            float flat_r = 0.0f, flat_g = 0.0f, flat_b = 0.0f, flat_a = 0.0f;
+            if (__builtin_expect(!special & is_coverage_tag(tag), 1)) {
+                float v = (float)rec.backdrop;  // no boundary in the tile
+                if (rec.covered) v = take_coverage(rec.d, rec.backdrop, lane);
+                masked = combine_alpha_u8((uint32_t)fill_u8_uniform(v, rec.fill_rule), clip_mask);
+                if (tag == TK_PTCL_BEGIN_CLIP) {
+                    push_clip(clip_mask);
+                    clip_mask = masked;
+                    return;
+                }
+                flat = false;
+            } else if (tag == TK_PTCL_END_CLIP) {
+                if (clip_depth > 0u) {
+                    clip_depth -= 1u;
+                    if (clip_depth == 0u) clip_mask = cs0;
+                    else if (clip_depth == 1u) clip_mask = cs1;
+                    else if (clip_depth == 2u) clip_mask = cs2;
+                    else if (clip_depth == 3u) clip_mask = cs3;
+                    else {
+                        uint32_t spill = clip_depth - 4u;
+                        if (spill < cfg.clip_spill_depth) clip_mask = clip_spill[spill * 256u + lane];
+                    }
+                } else {
+                    clip_mask = 255u;
+                }
+                return;
+            } else if (tag == TK_PTCL_SDF || tag == TK_PTCL_BEGIN_SDF_CLIP) {
+                const FineDraw d = load_fine_draw(constant(a.in.draws), cfg.draw_count, rec.color);
+                uint32_t alpha = 0u;
+                const bool reached = !special || ((int32_t)gx >= d.pb[0] && (int32_t)gy >= d.pb[1] &&
+                                                  (int32_t)gx < d.pb[2] && (int32_t)gy < d.pb[3]);
+                if (reached && clip_mask != 0u) alpha = coverage_to_u8(sdf_coverage_from_draw(cfg, paint, d, sx, sy));
+                masked = combine_alpha_u8(alpha, clip_mask);
+                if (tag == TK_PTCL_BEGIN_SDF_CLIP) {
+                    push_clip(clip_mask);
+                    clip_mask = masked;
+                    return;
+                }
+                if (special) color = blob_word(paint, cfg.paint_words, cfg.paint_brush_base, d.brush_offset + 4u);
+                else flat = false;
+            } else if (tag == kPtclImage) {
+                flat = false;
+            } else if (tag != TK_PTCL_COLOR) {
+                return;  // glyph-image, opacity and blend records are not produced on this path
+            }
+            // The floats of a flat colour come with its table entry, or from its bytes.
+            if (flat) {
+                flat_r = (float)(color & 255u);
+                flat_g = (float)((color >> 8) & 255u);
+                flat_b = (float)((color >> 16) & 255u);
+                flat_a = (float)(color >> 24);
+            } else if (rec.color < cfg.draw_count) {
+                const Const<uint32_t> entry = brushes + (size_t)rec.color * TK_DRAW_BRUSH_WORDS;
+                flat = entry[0] != 0u;
+                color = entry[1];
+                flat_r = asfloat(entry[4]);
+                flat_g = asfloat(entry[5]);
+                flat_b = asfloat(entry[6]);
+                flat_a = asfloat(entry[7]);
+            }
+            // In a special tile a colour or image is not scaled by a coverage.
+            const bool whole = special && tag != TK_PTCL_SDF;
+            if (flat && tag != kPtclPathGlyph) {
+                if ((color >> 24) != 0u && masked != 0u) {
+                    // src_over_premul_unorm of the scaled colour: its alpha is in (0, 1) unless the
+                    // colour is opaque under a full mask, which replaces the pixel
+                    const float scale = whole ? kChannelScale : (float)masked * (1.0f / 65025.0f);
+                    const Px src{flat_r * scale, flat_g * scale, flat_b * scale, flat_a * scale};
+                    const float inv = 1.0f - src.a;
+                    pixel = Px{src.r + pixel.r * inv, src.g + pixel.g * inv, src.b + pixel.b * inv, src.a + pixel.a * inv};
+                    if (premul_opaque(color) && masked == 255u)
+                        pixel = Px{flat_r * kChannelScale, flat_g * kChannelScale, flat_b * kChannelScale,
+                                   flat_a * kChannelScale};
+                }
+            } else if (masked != 0u) {
+                if (!flat)
+                    color = sample_draw_brush(cfg, paint, load_fine_draw(constant(a.in.draws), cfg.draw_count, rec.color),
+                                              sx, sy, atlas_of(a.in));
+                if (tag == kPtclPathGlyph)  // text compositing (interpreter.hlsli:205-206)
+                    pixel = rgba8_to_unorm(glyph_composite(unorm_to_rgba8(pixel), color, masked));
+                else if (masked == 255u && premul_opaque(color)) pixel = rgba8_to_unorm(color);
+                else
+                    pixel = src_over_premul_unorm(pixel, whole ? rgba8_to_unorm(color)
+                                                               : scale_premul_u8_to_unorm(color, masked));
+            }
+        };
+        walk_tile(v, a.in.tile_kinds, a.in.tile_ptcl_ranges, a.in.ptcl, cfg.ptcl_capacity, a.in.segments,
+                  cfg.segment_capacity, cov_acc, acc_sel,
+                  [](uint32_t kind, uint32_t tag, uint32_t) {
+                      return kind == TK_TILE_KIND_INTERPRETER && is_coverage_tag(tag);
+                  },
+                  [&](uint32_t kind, uint32_t tag, uint32_t color) -> uint32_t {
+                      if (kind != TK_TILE_KIND_INTERPRETER || tag != TK_PTCL_FILL || color >= cfg.draw_count) return 0u;
+                      const uint2 entry = *reinterpret_cast<const uint2 *>(a.draw_brush + (size_t)color * TK_DRAW_BRUSH_WORDS);
+                      if (entry.x == 0u || (entry.y >> 24) == 0u) return 0u;
+                      return premul_opaque(entry.y) ? kFlatOpaque : kFlatTranslucent;
+                  },
+                  [&](const WalkRecord &rec) {
+                      if (__builtin_expect(rec.mark != 0u, 1)) paint_flat_fill(rec);
+                      else if (rec.tag != TK_PTCL_END) paint_record(rec);
+                      if (rec.ends) {
+                          pixel = Px{quantized_channel(pixel.r), quantized_channel(pixel.g), quantized_channel(pixel.b),
+                                     quantized_channel(pixel.a)};
+                          clip_mask = 255u;
+                          clip_depth = 0u;
+                          cs0 = cs1 = cs2 = cs3 = 255u;
+                      }
+                  });
         if (gx < v.width && gy < v.height) a.rgba[v.image + (size_t)gy * v.width + gx] = unorm_to_rgba8(pixel);
     };
 
@@ -1887,7 +2108,7 @@ __device__ __forceinline__ void fine_tile(const tk_args_fine &a) {
     for (;;) {
         if (lane == 0u) s_item = queue_next(a.queue, blockIdx.x & 7u, qi, a.xcd_run, columns);
         __syncthreads();
-        const uint32_t column = s_item;
+        const uint32_t column = uniform(s_item);
         __syncthreads();
         if (column == ~0u) return;
         tile(column);
@@ -1954,7 +2175,7 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_brush_words(tk_args_brush
     const uint32_t id = blockIdx.x * 256u + threadIdx.x;
     if (id >= a.count) return;
     const uint32_t *q = a.requests + (size_t)id * 4u;
-    a.out[id] = sample_brush(a.paint, a.paint_words, a.paint_brush_base, q[0], asfloat(q[1]), asfloat(q[2]));
+    a.out[id] = sample_brush(constant(a.paint), a.paint_words, a.paint_brush_base, q[0], asfloat(q[1]), asfloat(q[2]));
 }
 
 // ===========================================================================
@@ -2059,11 +2280,12 @@ struct DiffPaint {
     float w0, w1, w2, w3;
 };
 __device__ __forceinline__ DiffPaint diff_paint(const float *paint, uint32_t draw, float x, float y) {
-    const float4 *r = reinterpret_cast<const float4 *>(paint + (size_t)draw * kDiffPaintFloats);
-    const float4 h0 = r[0];
-    DiffPaint p{r[4], 1.0f, 0.0f, 0.0f, 0.0f};
+    const Const<float> words = constant(paint) + (size_t)draw * kDiffPaintFloats;
+    const auto r = [&](uint32_t i) { return make_float4(words[4u * i], words[4u * i + 1u], words[4u * i + 2u], words[4u * i + 3u]); };
+    const float4 h0 = r(0);
+    DiffPaint p{r(4), 1.0f, 0.0f, 0.0f, 0.0f};
     if (h0.x == 0.0f) return p;
-    const float4 h1 = r[1], h2 = r[2];
+    const float4 h1 = r(1), h2 = r(2);
     const float dx = h0.w - h0.y, dy = h1.x - h0.z, den = dx * dx + dy * dy;
     const float px = x - h0.y, py = y - h0.z;
     float w0 = 0.0f, w1 = 0.0f, w2 = 0.0f, w3 = 0.0f;
@@ -2108,7 +2330,7 @@ __device__ __forceinline__ DiffPaint diff_paint(const float *paint, uint32_t dra
             w3 = 1.0f;
         }
     }
-    const float4 s0 = r[4], s1 = r[5], s2 = r[6], s3 = r[7];
+    const float4 s0 = r(4), s1 = r(5), s2 = r(6), s3 = r(7);
     p.c = make_float4(w0 * s0.x + w1 * s1.x + w2 * s2.x + w3 * s3.x, w0 * s0.y + w1 * s1.y + w2 * s2.y + w3 * s3.y,
                       w0 * s0.z + w1 * s1.z + w2 * s2.z + w3 * s3.z, w0 * s0.w + w1 * s1.w + w2 * s2.w + w3 * s3.w);
     p.w0 = w0;
@@ -2177,73 +2399,68 @@ struct ClipMask {
 // which needs the tile's coverage accumulator, in for_each_fill) and keeps it in
 // the record's slot of `adj`; the backward reads it from there.
 template <bool kKept>
-__device__ __forceinline__ bool clip_record(const tk_args_fine_diff &a, const DiffTile &t, uint32_t pi,
-                                            const tk_ptcl_record &rec, ClipMask &clip) {
-    if (rec.tag == TK_PTCL_END_CLIP) {
+__device__ __forceinline__ bool clip_record(const tk_args_fine_diff &a, const DiffTile &t, uint32_t pi, uint32_t tag,
+                                            uint32_t draw, ClipMask &clip) {
+    if (tag == TK_PTCL_END_CLIP) {
         clip.pop();
         return true;
     }
-    if (rec.tag != TK_PTCL_BEGIN_SDF_CLIP && !(kKept && rec.tag == TK_PTCL_BEGIN_CLIP)) return false;
+    if (tag != TK_PTCL_BEGIN_SDF_CLIP && !(kKept && tag == TK_PTCL_BEGIN_CLIP)) return false;
     const size_t slot = (size_t)pi * 256u + t.lane;
     float coverage = 0.0f;
     if constexpr (kKept) {
         if (pi < a.adj_records) coverage = a.adj[slot];
     } else {
-        const FineDraw d = load_fine_draw(a.in.draws, a.cfg.draw_count, rec.color);
-        coverage = sdf_coverage_from_draw(a.cfg, a.in.paint, d, (float)t.gx + 0.5f, (float)t.gy + 0.5f);
+        const FineDraw d = load_fine_draw(constant(a.in.draws), a.cfg.draw_count, draw);
+        coverage = sdf_coverage_from_draw(a.cfg, constant(a.in.paint), d, (float)t.gx + 0.5f, (float)t.gy + 0.5f);
         if (pi < a.adj_records) a.adj[slot] = coverage;
     }
     return clip.push(coverage);
 }
 
-// Calls body(pi, rec, mask) for every FILL record of the tile's streams, bottom
-// to top, with the pixel's clip mask; flags any record kind it does not take.
-// kClips: the scene has clip layers (their records are taken into the mask; a
-// path clip's coverage, its alpha under its fill rule, comes from
-// path_clip(pi, rec), called by the whole workgroup).
+// Calls body(rec, coverage, mask) for every FILL record of the tile's streams,
+// bottom to top, with the pixel's coverage by it and its clip mask; flags any
+// record kind it does not take.  kClips: the scene has clip layers (their records
+// are taken into the mask; a path clip's, from its coverage, comes from
+// path_clip(rec, coverage)).  The walk is fine's.
 template <bool kClips, class Body, class PathClip>
-__device__ __forceinline__ void for_each_fill(const tk_args_fine_diff &a, const DiffTile &t, Body body,
-                                              PathClip path_clip) {
+__device__ __forceinline__ void for_each_fill(const tk_args_fine_diff &a, const DiffTile &t, GroupCoverage *cov_acc,
+                                              Body body, PathClip path_clip) {
     const tk_fine_config &cfg = a.cfg;
-    for (uint32_t b = t.v.q0; b < t.v.q1; ++b) {
-        const size_t idx = table_index(t.v, b);
-        const uint32_t kind_word = a.in.tile_kinds[idx];
-        if ((kind_word & TK_TILE_KIND_MASK) == TK_TILE_KIND_EMPTY) continue;
-        const tk_segment_range r = a.in.tile_ptcl_ranges[idx];
-        const uint32_t pend = min(r.end, cfg.ptcl_capacity);
-        ClipMask clip{1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 0u};
-        for (uint32_t pi = r.start + (kind_word >> TK_TILE_PREFIX_SHIFT); pi < pend; ++pi) {
-            const tk_ptcl_record rec = a.in.ptcl[pi];
-            if (rec.tag == TK_PTCL_END) break;
-            if (rec.tag == TK_PTCL_FILL && rec.color < cfg.draw_count) {
-                body(pi, rec, clip.m);
-            } else if (kClips && rec.tag == TK_PTCL_BEGIN_CLIP) {
-                if (!clip.push(path_clip(pi, rec)) && t.lane == 0u && a.status) atomicOr(a.status, 1u);
-            } else if (!kClips || !clip_record<false>(a, t, pi, rec, clip)) {
-                if (t.lane == 0u && a.status) atomicOr(a.status, 1u);
-            }
-        }
-    }
+    uint32_t sel = 0u;
+    clear_coverage(cov_acc[0], t.lane);
+    clear_coverage(cov_acc[1], t.lane);
+    __syncthreads();
+    const auto covers = [&](uint32_t, uint32_t tag, uint32_t color) {
+        return ((tag == TK_PTCL_FILL) & (color < cfg.draw_count)) | (kClips & (tag == TK_PTCL_BEGIN_CLIP));
+    };
+    ClipMask clip{1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 0u};
+    walk_tile(t.v, a.in.tile_kinds, a.in.tile_ptcl_ranges, a.in.ptcl, cfg.ptcl_capacity, a.in.segments,
+              cfg.segment_capacity, cov_acc, sel, covers, [](uint32_t, uint32_t, uint32_t) { return 0u; },
+              [&](const WalkRecord &rec) {
+                  if (rec.tag != TK_PTCL_END) {
+                      float cov = (float)rec.backdrop;
+                      if (rec.covered) cov = take_coverage(rec.d, rec.backdrop, t.lane);
+                      if (rec.tag == TK_PTCL_FILL && rec.color < cfg.draw_count) {
+                          body(rec, cov, clip.m);
+                      } else if (kClips && rec.tag == TK_PTCL_BEGIN_CLIP) {
+                          if (!clip.push(path_clip(rec, cov)) && t.lane == 0u && a.status) atomicOr(a.status, 1u);
+                      } else if (!kClips || !clip_record<false>(a, t, rec.index, rec.tag, rec.color, clip)) {
+                          if (t.lane == 0u && a.status) atomicOr(a.status, 1u);
+                      }
+                  }
+                  if (rec.ends) clip = ClipMask{1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 0u};
+              });
 }
 
 // kKeep: keep each record's coverage (a path clip's mask) in its slot of `adj`
 // for the backward; otherwise the backward recomputes it from the segments.
 template <bool kScenes, bool kClips, bool kKeep>
 __device__ __forceinline__ void fine_diff_forward_tile(const tk_args_fine_diff &a) {
-    __shared__ CoverageAcc cov_acc[2];
+    __shared__ GroupCoverage cov_acc[2];
     DiffTile t;
     if (!diff_tile<kScenes>(a, t)) return;
     const uint32_t lane = t.lane;
-    cov_acc[0].run[lane] = 0;
-    cov_acc[0].part[lane] = 0;
-    cov_acc[1].run[lane] = 0;
-    cov_acc[1].part[lane] = 0;
-    if (lane < 16u) {
-        cov_acc[0].base[lane] = 0;
-        cov_acc[1].base[lane] = 0;
-    }
-    uint32_t sel = 0u;
-    __syncthreads();
     const float sx = (float)t.gx + 0.5f, sy = (float)t.gy + 0.5f;
     Px px = rgba8_to_unorm(t.v.clear);
     bool overflow = false;
@@ -2251,30 +2468,19 @@ __device__ __forceinline__ void fine_diff_forward_tile(const tk_args_fine_diff &
     const uint32_t tx = t.tile % t.v.tw, ty = t.tile / t.v.tw;
     // A path clip's mask: its coverage turned into alpha by its fill rule, kept
     // in the record's slot of `adj` for the backward.
-    auto path_clip = [&](uint32_t pi, const tk_ptcl_record &rec) {
-        const uint32_t s0 = rec.segment_start, s1 = min(rec.segment_end, a.cfg.segment_capacity);
-        CoverageAcc &acc = cov_acc[sel];
-        sel ^= 1u;
-        accumulate_record(a.in.segments + s0, s1 > s0 ? s1 - s0 : 0u, acc, lane);
-        __syncthreads();
+    auto path_clip = [&](const WalkRecord &rec, float cov) {
         float slope;
-        const float m = diff_alpha(take_coverage(acc, rec.backdrop, lane), rec.fill_rule, slope);
+        const float m = diff_alpha(cov, rec.fill_rule, slope);
         if (kKeep) {
-            if (pi < a.adj_records) a.adj[(size_t)pi * 256u + lane] = m;
+            if (rec.index < a.adj_records) a.adj[(size_t)rec.index * 256u + lane] = m;
             else overflow = true;
         }
         return m;
     };
-    for_each_fill<kClips>(a, t, [&](uint32_t pi, const tk_ptcl_record &rec, float mask) {
-        const uint32_t s0 = rec.segment_start, s1 = min(rec.segment_end, a.cfg.segment_capacity);
+    for_each_fill<kClips>(a, t, cov_acc, [&](const WalkRecord &rec, float cov, float mask) {
+        const uint32_t pi = rec.index;
         const float4 c = diff_paint(a.colors, rec.color, sx, sy).c;
-        // Issued before the coverage work so that its latency overlaps it.
-        const uint4 box = reinterpret_cast<const uint4 *>(a.draw_tiles)[rec.color];
-        CoverageAcc &acc = cov_acc[sel];
-        sel ^= 1u;
-        accumulate_record(a.in.segments + s0, s1 > s0 ? s1 - s0 : 0u, acc, lane);
-        __syncthreads();
-        const float cov = take_coverage(acc, rec.backdrop, lane);
+        const Const<uint32_t> box = constant(a.draw_tiles) + 4u * (size_t)rec.color;
         float slope;
         const float alpha = diff_alpha(cov, rec.fill_rule, slope) * mask;
         const float f = 1.0f - alpha * c.w;
@@ -2287,10 +2493,10 @@ __device__ __forceinline__ void fine_diff_forward_tile(const tk_args_fine_diff &
             if (pi < a.adj_records) a.adj[(size_t)pi * 256u + lane] = cov;
             else overflow = true;
         }
-        if (lane == 0u && box.w != 0u) {  // where the line pass finds this path's record in this tile
-            const uint32_t x0 = box.y & 0xFFFFu, y0 = box.y >> 16, x1 = box.z & 0xFFFFu, y1 = box.z >> 16;
+        if (lane == 0u && box[3] != 0u) {  // where the line pass finds this path's record in this tile
+            const uint32_t x0 = box[1] & 0xFFFFu, y0 = box[1] >> 16, x1 = box[2] & 0xFFFFu, y1 = box[2] >> 16;
             if (tx >= x0 && ty >= y0 && tx < x1 && ty < y1) {
-                const uint32_t bd = box.x + (ty - y0) * (x1 - x0) + tx - x0;
+                const uint32_t bd = box[0] + (ty - y0) * (x1 - x0) + tx - x0;
                 if (bd < a.rec_of_count) a.rec_of[bd] = pi;
             }
         }
@@ -2308,7 +2514,7 @@ __device__ __forceinline__ void fine_diff_forward_tile(const tk_args_fine_diff &
 // them (the exact sums do not depend on the segment order).
 template <bool kScenes, bool kClips, bool kKeep>
 __device__ __forceinline__ void fine_diff_backward_tile(const tk_args_fine_diff &a) {
-    __shared__ CoverageAcc cov_acc[kKeep ? 1 : 2];
+    __shared__ GroupCoverage cov_acc[2];  // (unused, and not allocated, where the coverages were kept)
     DiffTile t;
     if (!diff_tile<kScenes>(a, t)) return;
     const uint32_t lane = t.lane;
@@ -2320,11 +2526,11 @@ __device__ __forceinline__ void fine_diff_backward_tile(const tk_args_fine_diff 
     const Transmit total{__uint_as_float(tw.x), (int)tw.y, (int)tw.z};
     Transmit below{1.0f, 0, 0};
     Px res = rgba8_to_unorm(t.v.clear);
-    auto record = [&](uint32_t pi, const tk_ptcl_record &rec, float cov, float mask) {
-        const DiffPaint paint = diff_paint(a.colors, rec.color, sx, sy);
+    auto record = [&](uint32_t pi, uint32_t draw, uint32_t fill_rule, float cov, float mask) {
+        const DiffPaint paint = diff_paint(a.colors, draw, sx, sy);
         const float4 c = paint.c;
         float slope;
-        const float alpha = diff_alpha(cov, rec.fill_rule, slope) * mask;
+        const float alpha = diff_alpha(cov, fill_rule, slope) * mask;
         slope *= mask;
         const float f = 1.0f - alpha * c.w;
         below.mul(f);
@@ -2337,10 +2543,9 @@ __device__ __forceinline__ void fine_diff_backward_tile(const tk_args_fine_diff 
         // four-channel wave sum per stop the paint has (the stop count is uniform).
         const float w = T * alpha;
         const float gr = w * g.x, gg = w * g.y, gb = w * g.z, ga = w * (g.w - g_res);
-        float *out = a.color_grad + (size_t)rec.color * kDiffPaintFloats + 16u + sum4_channel(lane);
-        const float stops = a.colors[(size_t)rec.color * kDiffPaintFloats] == 0.0f
-                                ? 1.0f
-                                : a.colors[(size_t)rec.color * kDiffPaintFloats + 5u];
+        float *out = a.color_grad + (size_t)draw * kDiffPaintFloats + 16u + sum4_channel(lane);
+        const Const<float> head = constant(a.colors) + (size_t)draw * kDiffPaintFloats;
+        const float stops = head[0] == 0.0f ? 1.0f : head[5];
         const float sum0 = wave_sum4(paint.w0 * gr, paint.w0 * gg, paint.w0 * gb, paint.w0 * ga, lane);
         if ((lane & 63u) >= 60u) atomicAdd(out, sum0);
         if (stops > 1.0f) {
@@ -2361,31 +2566,14 @@ __device__ __forceinline__ void fine_diff_backward_tile(const tk_args_fine_diff 
         res.a = res.a * f + alpha * c.w;
     };
     if constexpr (!kKeep) {
-        cov_acc[0].run[lane] = 0;
-        cov_acc[0].part[lane] = 0;
-        cov_acc[1].run[lane] = 0;
-        cov_acc[1].part[lane] = 0;
-        if (lane < 16u) {
-            cov_acc[0].base[lane] = 0;
-            cov_acc[1].base[lane] = 0;
-        }
-        uint32_t sel = 0u;
-        __syncthreads();
-        auto cover = [&](const tk_ptcl_record &rec) {
-            const uint32_t s0 = rec.segment_start, s1 = min(rec.segment_end, a.cfg.segment_capacity);
-            CoverageAcc &acc = cov_acc[sel];
-            sel ^= 1u;
-            accumulate_record(a.in.segments + s0, s1 > s0 ? s1 - s0 : 0u, acc, lane);
-            __syncthreads();
-            return take_coverage(acc, rec.backdrop, lane);
-        };
-        auto path_clip = [&](uint32_t, const tk_ptcl_record &rec) {
+        auto path_clip = [&](const WalkRecord &rec, float cov) {
             float slope;
-            return diff_alpha(cover(rec), rec.fill_rule, slope);
+            return diff_alpha(cov, rec.fill_rule, slope);
         };
-        for_each_fill<kClips>(a, t, [&](uint32_t pi, const tk_ptcl_record &rec, float mask) {
-            record(pi, rec, cover(rec), mask);
-        }, path_clip);
+        for_each_fill<kClips>(
+            a, t, cov_acc,
+            [&](const WalkRecord &rec, float cov, float mask) { record(rec.index, rec.color, rec.fill_rule, cov, mask); },
+            path_clip);
         return;
     }
     // The walk of for_each_fill, software-pipelined: the next record and its
@@ -2408,8 +2596,8 @@ __device__ __forceinline__ void fine_diff_backward_tile(const tk_args_fine_diff 
             tk_ptcl_record nrec{};
             if (more) nrec = a.in.ptcl[next];
             const float ncov = more ? coverage(next) : 0.0f;
-            if (rec.tag == TK_PTCL_FILL && rec.color < draws) record(pi, rec, cov, clip.m);
-            else if ((!kClips || !clip_record<true>(a, t, pi, rec, clip)) && lane == 0u && a.status)
+            if (rec.tag == TK_PTCL_FILL && rec.color < draws) record(pi, rec.color, rec.fill_rule, cov, clip.m);
+            else if ((!kClips || !clip_record<true>(a, t, pi, rec.tag, rec.color, clip)) && lane == 0u && a.status)
                 atomicOr(a.status, 1u);
             if (!more) break;
             pi = next;

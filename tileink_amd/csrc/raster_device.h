@@ -289,10 +289,27 @@ TKD uint32_t coverage_to_alpha(float v, uint32_t rule) {
     if (rule == 1u) alpha = fabsf(v - 2.0f * rintf(0.5f * v));
     return coverage_to_u8(alpha);
 }
+// coverage_to_alpha's u8 as a float, for a coverage that is a number, where every
+// lane has the same rule: a branch on it, so each rule runs its own instructions
+// (the empty asm keeps the branch from becoming a select).  Both rules give at most
+// 1, so coverage_to_u8's clamp is left out; 2 * rint(v / 2) is exact, so the fused
+// form rounds as the separate one.
+TKD float fill_u8_uniform(float v, uint32_t rule) {
+    float alpha;
+    if (rule == 1u) {
+        alpha = fabsf(fmaf(-2.0f, rintf(0.5f * v), v));
+        asm volatile("");
+    } else {
+        alpha = __builtin_amdgcn_fmed3f(fabsf(v), 0.0f, 1.0f);
+    }
+    return truncf(alpha * 255.0f + 0.5f);
+}
 TKD float signum_f32(float v) { return v < 0.0f ? -1.0f : 1.0f; }
 TKD uint32_t rgba8_pack(uint32_t r, uint32_t g, uint32_t b, uint32_t a) { return r | (g << 8) | (b << 16) | (a << 24); }
 TKD uint32_t chan_u8(float v) { return (uint32_t)clampf(v * 255.0f + 0.5f, 0.0f, 255.0f); }  // in [0, 255], as above
 TKD uint32_t unorm_to_rgba8(Px p) { return rgba8_pack(chan_u8(p.r), chan_u8(p.g), chan_u8(p.b), chan_u8(p.a)); }
+// A channel through unorm_to_rgba8 and back through rgba8_to_unorm.
+TKD float quantized_channel(float v) { return truncf(clampf(v * 255.0f + 0.5f, 0.0f, 255.0f)) * kChannelScale; }
 TKD Px rgba8_to_unorm(uint32_t p) {
     return Px{(float)(p & 255u) * kChannelScale, (float)((p >> 8) & 255u) * kChannelScale,
               (float)((p >> 16) & 255u) * kChannelScale, (float)(p >> 24) * kChannelScale};
@@ -302,6 +319,12 @@ TKD uint32_t mul_div255(uint32_t a, uint32_t b) {
     return (product + (product >> 8)) >> 8;
 }
 TKD uint32_t combine_alpha(uint32_t a, uint32_t b) { return mul_div255(a, b); }
+// combine_alpha of two values in [0, 255]: a 24-bit product (full rate, where a
+// 32-bit one takes four issue slots).
+TKD uint32_t combine_alpha_u8(uint32_t a, uint32_t b) {
+    const uint32_t product = __umul24(a, b) + 128u;
+    return (product + (product >> 8)) >> 8;
+}
 TKD float straight_channel(uint32_t premul, uint32_t alpha) { return alpha == 0u ? 0.0f : (float)premul / (float)alpha; }
 TKD uint32_t scale_premul_u8(uint32_t source, uint32_t factor) {
     if (factor == 0u) return 0u;
@@ -349,24 +372,26 @@ TKD float rem_euclid_f32(float value, float modulus) { return fmaf(-floorf(value
 // Row-sweep area coverage (shared/coverage.hlsli:7-51)
 // ---------------------------------------------------------------------------
 
+// The row's edge term of a segment (y_edge: where it meets the tile's left edge).
+TKD float segment_row_edge(float delta_x, float y_edge, uint32_t y) {
+    return signum_f32(delta_x) * clampf((float)y - y_edge + 1.0f, 0.0f, 1.0f);
+}
+// The row's other terms, for a slope delta x / delta y (unused where the segment
+// does not cross the row).
 struct RowParts {
-    float edge, dy, xmin, xmax;
+    float dy, xmin, xmax;
 };
-
-TKD RowParts segment_row_parts(float p0x, float p0y, float p1x, float p1y, float y_edge, uint32_t y) {
-    float delta_x = p1x - p0x, delta_y = p1y - p0y;
+TKD RowParts segment_row_parts(float p0x, float p0y, float p1x, float p1y, float slope, uint32_t y) {
     float row_y = (float)y, local_y = p0y - row_y;
     float y0 = clampf(local_y, 0.0f, 1.0f), y1 = clampf(p1y - row_y, 0.0f, 1.0f);
     float dy = y0 - y1;
-    float row_edge = signum_f32(delta_x) * clampf(row_y - y_edge + 1.0f, 0.0f, 1.0f);
-    if (dy == 0.0f) return RowParts{row_edge, dy, 0.0f, 0.0f};
-    float slope = delta_x / delta_y;
+    if (dy == 0.0f) return RowParts{dy, 0.0f, 0.0f};
     bool nearer_p0 = fabsf(local_y - 0.5f) <= fabsf(p1y - row_y - 0.5f);
     float anchor_x = nearer_p0 ? p0x : p1x;
     float anchor_y = nearer_p0 ? local_y : p1y - row_y;
     float sx0 = fmaf(y0 - anchor_y, slope, anchor_x);
     float sx1 = fmaf(y1 - anchor_y, slope, anchor_x);
-    return RowParts{row_edge, dy, fminf(sx0, sx1), fmaxf(sx0, sx1)};
+    return RowParts{dy, fminf(sx0, sx1), fmaxf(sx0, sx1)};
 }
 
 // segment_area_at with the pixel's x already in FP32 (an integer 0..15, exact).
@@ -378,6 +403,31 @@ TKD float segment_area_at_f(float xmin_abs, float xmax_abs, float xf) {
     float left = clampf(xmin, 0.0f, 1.0f), right = clampf(xmax, 0.0f, 1.0f);
     float full = clampf(-xmin, 0.0f, width);
     return fmaf(right - left, fmaf(-0.5f, left + right, 1.0f), full) / width;
+}
+// The share of pixel x that lies right of the line part [xmin_abs, xmax_abs] where
+// that part leaves the pixel on some side: segment_area_at_f's last case, its
+// quotient from `recip`, a reciprocal of about the part's width.  xmax - xmin and
+// the width before the shift by xf differ by rounding only (under 2^-22 of it), so
+// one Newton step gives this pixel's own reciprocal, and two residual corrections
+// round the quotient as a division does (Markstein 1990: a faithful quotient, its
+// exact residual by a fused multiply-add, one more step).  plain_width says which
+// widths this holds for: those in [2^-60, 2^60], where no residual that reaches a
+// 2^-30 term underflows, whose significand is not within 8 units of a power of two
+// (one of all ones is the theorem's exception; the pixel's width is within 2 units).
+// 8 full-rate instructions for a division's 11, one of them quarter rate.
+TKD bool plain_width(float width) {
+    const uint32_t bits = __float_as_uint(width);
+    return bits - 0x21800000u <= 0x5d800000u - 0x21800000u && ((bits + 8u) & 0x7FFFFFu) >= 16u;
+}
+TKD float segment_area_across(float xmin_abs, float xmax_abs, float xf, float recip) {
+    const float xmin = xmin_abs - xf, xmax = xmax_abs - xf, width = xmax - xmin;
+    const float left = clampf(xmin, 0.0f, 1.0f), right = clampf(xmax, 0.0f, 1.0f);
+    const float full = clampf(-xmin, 0.0f, width);
+    const float a = fmaf(right - left, fmaf(-0.5f, left + right, 1.0f), full);
+    const float y = fmaf(fmaf(-width, recip, 1.0f), recip, recip);
+    float q = a * y;
+    q = fmaf(fmaf(-width, q, a), y, q);
+    return fmaf(fmaf(-width, q, a), y, q);
 }
 TKD float segment_area_at(float xmin_abs, float xmax_abs, uint32_t x) {
     return segment_area_at_f(xmin_abs, xmax_abs, (float)x);
@@ -392,19 +442,23 @@ TKD float segment_area_at(float xmin_abs, float xmax_abs, uint32_t x) {
 // Every term lies in (-2, 2): the edge term is signum * a clamp to [0, 1], dy is
 // the difference of two values clamped to [0, 1], and the area factor is at most
 // 1 up to rounding.  So t * 2^30 (exact, a power-of-two scaling) fits an int32
-// and one truncating v_cvt_i32_f32 gives trunc(t * 2^30); a NaN term counts as 0.
-TKD long long coverage_fixed(float t) {
-    const int32_t q = (int32_t)(t * 1073741824.0f);
-    return t == t ? (long long)q : 0ll;
+// and one truncating v_cvt_i32_f32 gives trunc(t * 2^30); the instruction takes a
+// NaN to 0 (a C++ conversion of one is undefined, so it is named here).
+constexpr float kCoverageOne = 1073741824.0f;  // 2^30
+TKD int32_t coverage_trunc(float scaled) {  // scaled: the term times kCoverageOne
+    int32_t q;
+    asm("v_cvt_i32_f32_e32 %0, %1" : "=v"(q) : "v"(scaled));
+    return q;
 }
+TKD long long coverage_fixed(float t) { return coverage_trunc(t * kCoverageOne); }
 // Back to FP32: the sum floored to a multiple of 2^-24 (at most 6e-8 below it),
 // then one rounding.  hi = floor(v / 2^30) and the top 24 of the 30 fraction bits
 // convert exactly (|hi| < 2^24 for any coverage sum), the scaling by 2^-24 is
-// exact, and only the add rounds.
+// exact (so the fused add rounds as a plain one), and only the add rounds.
 TKD float fixed_to_float(long long v) {
     const float hi = (float)(int32_t)(v >> 30);
-    const float lo = (float)(((uint32_t)v & 0x3FFFFFFFu) >> 6) * 5.9604644775390625e-8f;
-    return hi + lo;
+    const float lo = (float)(((uint32_t)v & 0x3FFFFFFFu) >> 6);
+    return fmaf(lo, 5.9604644775390625e-8f, hi);
 }
 TKD long long backdrop_fixed(int32_t backdrop) { return (long long)backdrop * 1073741824LL; }
 
@@ -414,8 +468,9 @@ TKD float exact_fill_value(const tk_line_segment *segs, int32_t backdrop, uint32
     long long base = backdrop_fixed(backdrop), running = 0, partial = 0;
     for (uint32_t i = start; i < end; ++i) {
         const tk_line_segment seg = segs[i];
-        RowParts parts = segment_row_parts(seg.p0x, seg.p0y, seg.p1x, seg.p1y, seg.y_edge, y);
-        base += coverage_fixed(parts.edge);
+        const float dx = seg.p1x - seg.p0x;
+        const RowParts parts = segment_row_parts(seg.p0x, seg.p0y, seg.p1x, seg.p1y, dx / (seg.p1y - seg.p0y), y);
+        base += coverage_fixed(segment_row_edge(dx, seg.y_edge, y));
         if (parts.dy != 0.0f) {
             int full_start = clamp_cell16(ceilf(parts.xmax));
             if (full_start < 16 && (int)x >= full_start) running += coverage_fixed(parts.dy);
@@ -432,18 +487,26 @@ TKD float exact_fill_value(const tk_line_segment *segs, int32_t backdrop, uint32
 // (shared/sdf/{base,basic,coverage,data}.hlsli, shared/brush/*.hlsli, shared/affine.hlsli)
 // ---------------------------------------------------------------------------
 
+// Buffers that no kernel reading them writes, addressed as constant memory: a read
+// at an index the compiler knows to be the same in every lane becomes a scalar load.
+// (From an ordinary pointer it does not, once the kernel has stored or synchronised.)
+template <class T>
+using Const = const __attribute__((address_space(4))) T *;
+template <class T>
+TKD Const<T> constant(const T *p) { return (Const<T>)(uintptr_t)p; }
+
 // Bounds-checked word read with robust-buffer semantics: out of range reads 0.
-TKD uint32_t paint_word(const uint32_t *paint, uint32_t count, uint32_t index) {
+TKD uint32_t paint_word(Const<uint32_t> paint, uint32_t count, uint32_t index) {
     return index < count ? paint[index] : 0u;
 }
 // sdf_word / brush_word (shared/sdf/data.hlsli:3-8, shared/brush/data.hlsli:3-14).
-TKD uint32_t blob_word(const uint32_t *paint, uint32_t count, uint32_t base, uint32_t index) {
+TKD uint32_t blob_word(Const<uint32_t> paint, uint32_t count, uint32_t base, uint32_t index) {
     if (base < count) {
         if (index < count - base) return paint[base + index];
     }
     return 0u;
 }
-TKD float blob_float(const uint32_t *paint, uint32_t count, uint32_t base, uint32_t index) {
+TKD float blob_float(Const<uint32_t> paint, uint32_t count, uint32_t base, uint32_t index) {
     return asfloat(blob_word(paint, count, base, index));
 }
 
@@ -509,7 +572,7 @@ TKD float sdf_coverage_from_sample(const SdfSample &s, const Affine &inv) {
 
 // sdf_coverage_from_blob (shared/sdf/coverage.hlsli:13-74) for the rectangle kinds
 // on this path; other SDF kinds contribute no coverage here.
-TKD float sdf_coverage_from_blob(const uint32_t *paint, uint32_t count, uint32_t base, float x, float y,
+TKD float sdf_coverage_from_blob(Const<uint32_t> paint, uint32_t count, uint32_t base, float x, float y,
                                  const Affine &inv) {
     uint32_t kind = blob_word(paint, count, base, 0u);
     float x0 = blob_float(paint, count, base, 1u), y0 = blob_float(paint, count, base, 2u);
@@ -548,7 +611,7 @@ TKD float apply_extend(float t, uint32_t extend) {
     }
     return clampf(t, 0.0f, 1.0f);
 }
-TKD uint32_t sample_ramp(const uint32_t *paint, uint32_t count, uint32_t brush_base, uint32_t payload_offset,
+TKD uint32_t sample_ramp(Const<uint32_t> paint, uint32_t count, uint32_t brush_base, uint32_t payload_offset,
                          uint32_t payload_len, float t, uint32_t extend) {
     if (payload_len == 0u) return 0u;
     uint32_t last = payload_len - 1u;
@@ -565,7 +628,7 @@ TKD uint32_t sample_ramp(const uint32_t *paint, uint32_t count, uint32_t brush_b
 // (sample_brush below), so fine carries one inlined copy of it.
 //
 // linear_t: sample_linear (shared/brush/linear.hlsli:5-14).
-TKD float linear_t(const uint32_t *paint, uint32_t count, uint32_t brush_base, float x, float y, uint32_t base) {
+TKD float linear_t(Const<uint32_t> paint, uint32_t count, uint32_t brush_base, float x, float y, uint32_t base) {
     float p[10];
     for (int i = 0; i < 10; ++i) p[i] = blob_float(paint, count, brush_base, base + (uint32_t)i);
     float tx = fmaf(p[4], x, fmaf(p[6], y, p[8]));
@@ -580,7 +643,7 @@ TKD float linear_t(const uint32_t *paint, uint32_t count, uint32_t brush_base, f
 // gradient: t from the quadratic |q - t dc| = r0 + t dr with r0 + t dr >= 0;
 // has_t is false where no such t exists (the sample is transparent).
 constexpr float kRadialQuadraticEpsilon = 0.000001f;  // shared/brush/radial.hlsli:4
-TKD float radial_t(const uint32_t *paint, uint32_t count, uint32_t brush_base, float x, float y, uint32_t base,
+TKD float radial_t(Const<uint32_t> paint, uint32_t count, uint32_t brush_base, float x, float y, uint32_t base,
                    bool &has_t) {
     float p[12];
     for (int i = 0; i < 12; ++i) p[i] = blob_float(paint, count, brush_base, base + (uint32_t)i);
@@ -645,7 +708,7 @@ TKD float sweep_atan2(float y, float x) {
 // sweep_t: sample_sweep (shared/brush/sweep.hlsli:5-20), the angle from the
 // centre measured from the start orientation in the direction of the signed span.
 constexpr float kGradientTau = 6.2831855f;  // shared/brush/sweep.hlsli:4
-TKD float sweep_t(const uint32_t *paint, uint32_t count, uint32_t brush_base, float x, float y, uint32_t base) {
+TKD float sweep_t(Const<uint32_t> paint, uint32_t count, uint32_t brush_base, float x, float y, uint32_t base) {
     const float cx = blob_float(paint, count, brush_base, base), cy = blob_float(paint, count, brush_base, base + 1u);
     const float start_angle = blob_float(paint, count, brush_base, base + 2u);
     const float span = blob_float(paint, count, brush_base, base + 3u);
@@ -666,7 +729,7 @@ TKD float sweep_t(const uint32_t *paint, uint32_t count, uint32_t brush_base, fl
 
 // sample_four_corner (shared/brush/four_corner.hlsli:5-15): bilinear blend of the
 // corner colours tl, tr, br, bl over the bounds.
-TKD uint32_t sample_four_corner(const uint32_t *paint, uint32_t count, uint32_t brush_base, float x, float y,
+TKD uint32_t sample_four_corner(Const<uint32_t> paint, uint32_t count, uint32_t brush_base, float x, float y,
                                 uint32_t base, uint32_t payload) {
     const float x0 = blob_float(paint, count, brush_base, base), y0 = blob_float(paint, count, brush_base, base + 1u);
     const float x1 = blob_float(paint, count, brush_base, base + 2u), y1 = blob_float(paint, count, brush_base, base + 3u);
@@ -845,7 +908,7 @@ TKD uint32_t sample_pattern_atlas(const AtlasView &a, float px, float py, uint32
 }
 // sample_atlas_brush (pattern.hlsli:44-54), for a header whose placement the
 // encoding patched: words 2-6 = x, y, page, width, height.
-TKD uint32_t sample_image_brush(const uint32_t *paint, uint32_t count, uint32_t brush_base, uint32_t data_base,
+TKD uint32_t sample_image_brush(Const<uint32_t> paint, uint32_t count, uint32_t brush_base, uint32_t data_base,
                                 const AtlasView &atlas, float x, float y) {
     const uint32_t base = data_base + TK_BRUSH_HEADER_WORDS;
     const uint32_t sx = blob_word(paint, count, brush_base, data_base + 5u);
@@ -866,7 +929,7 @@ TKD uint32_t sample_image_brush(const uint32_t *paint, uint32_t count, uint32_t 
 
 // sample_brush (shared/brush/sample.hlsli:15-42) for the solid, linear, radial,
 // sweep, four-corner and image brushes.
-TKD uint32_t sample_brush(const uint32_t *paint, uint32_t count, uint32_t brush_base, uint32_t data_base, float x,
+TKD uint32_t sample_brush(Const<uint32_t> paint, uint32_t count, uint32_t brush_base, uint32_t data_base, float x,
                           float y, const AtlasView &atlas = AtlasView{nullptr, 0u, 0u, 0u}) {
     uint32_t kind = blob_word(paint, count, brush_base, data_base);
     uint32_t extend = blob_word(paint, count, brush_base, data_base + 1u);

@@ -328,7 +328,7 @@ tk_status run_coarse(tk_context *ctx, const tk_coarse_config &cfg, const tk_coar
     return TK_OK;
 }
 
-// `draw_brush` holds 2 * cfg.draw_count words; it is rebuilt here from the draws
+// `draw_brush` holds TK_DRAW_BRUSH_WORDS * cfg.draw_count words; it is rebuilt here from the draws
 // and paint before fine reads it.
 tk_status run_fine(tk_context *ctx, const tk_fine_config &cfg, const tk_fine_inputs &in, uint32_t *rgba,
                    uint32_t *draw_brush, tk_tile_list list = tk_tile_list{nullptr, 0u},
@@ -990,7 +990,7 @@ tk_status frame_create(tk_context *ctx, const tk_scene *s, const BatchLayout *ba
     ALLOC(status, 4);
     ALLOC(diff_status, 1);
     ALLOC(ptcl, f->ptcl_capacity);
-    ALLOC(draw_brush, 2 * std::max<uint64_t>(s->draw_count, 1));
+    ALLOC(draw_brush, TK_DRAW_BRUSH_WORDS * std::max<uint64_t>(s->draw_count, 1));
     ALLOC(active_tiles, T);
     ALLOC(damage_sat, uint64_t(s->tiles_width + 1) * (s->tiles_height + 1));
     ALLOC(path_active, std::max<uint64_t>(s->path_count, 1));
@@ -2390,7 +2390,7 @@ tk_status tk_fine(tk_context *ctx, const tk_fine_config *cfg, const tk_fine_inpu
     if (!ctx || !cfg || !in || !rgba) return fail(TK_ERR_INVALID, "null argument");
     if (uint64_t(cfg->tiles_width) * cfg->tiles_height != cfg->tile_count)
         return fail(TK_ERR_INVALID, "tile_count must equal tiles_width * tiles_height");
-    TK_TRY(ensure_draw_brush(ctx, 2 * size_t(cfg->draw_count)));
+    TK_TRY(ensure_draw_brush(ctx, TK_DRAW_BRUSH_WORDS * size_t(cfg->draw_count)));
     return run_fine(ctx, *cfg, *in, rgba, ctx->draw_brush);
 }
 

@@ -153,8 +153,10 @@ struct tk_args_layer_classes {
     tk_tile_list list;
 };
 
-// Per-draw brush words for fine: two words per draw, {1, colour} when the draw's
-// brush colour does not depend on the pixel, {0, 0} when it must be sampled.
+// Per-draw brush words for fine, eight per draw: {1, colour, 0, 0, the colour's
+// four bytes as floats} when the draw's brush colour does not depend on the pixel,
+// zeros when it must be sampled.
+#define TK_DRAW_BRUSH_WORDS 8u
 struct tk_args_draw_brush {
     const tk_draw_record *draws;
     uint32_t draw_count;
