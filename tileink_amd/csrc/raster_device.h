@@ -25,21 +25,24 @@ constexpr float kChannelScale = 1.0f / 255.0f;       // shared/pixel.hlsli:5
 constexpr float kGradientEpsilon = 0.00000011920929f; // shared/brush/ramp.hlsli:6
 constexpr uint32_t kNone = TK_INVALID_INDEX;
 
+// Float to integer as the hardware converts: truncated, saturated, NaN to 0 (what
+// the shaders' casts lower to).  The instructions by name: the C++ conversion is
+// undefined outside the range, and range checks around it cost five instructions
+// and two branches.
 TKD uint32_t f2u(float v) {
-    if (!(v > 0.0f)) return 0u;
-    if (v >= 4294967296.0f) return 0xFFFFFFFFu;
-    return (uint32_t)v;
+    uint32_t r;
+    asm("v_cvt_u32_f32_e32 %0, %1" : "=v"(r) : "v"(v));
+    return r;
 }
 TKD int32_t f2i(float v) {
-    if (!(v == v)) return 0;
-    if (v <= -2147483648.0f) return (int32_t)0x80000000u;
-    if (v >= 2147483648.0f) return 0x7FFFFFFF;
-    return (int32_t)v;
+    int32_t r;
+    asm("v_cvt_i32_f32_e32 %0, %1" : "=v"(r) : "v"(v));
+    return r;
 }
 TKD float clampf(float x, float lo, float hi) { return fminf(fmaxf(x, lo), hi); }
 TKD int clampi(int x, int lo, int hi) { return min(max(x, lo), hi); }
 // clampi(f2i(v), 0, 16) for every v (NaN included, as fmaxf(NaN, 0) = 0) without
-// f2i's range branches: v is clamped in FP32 first, so the conversion is exact.
+// an out-of-range conversion: v is clamped in FP32 first, so the conversion is exact.
 TKD int clamp_cell16(float v) { return (int)fminf(fmaxf(v, 0.0f), 16.0f); }
 TKD float asfloat(uint32_t u) { return __uint_as_float(u); }
 TKD uint32_t asuint(float f) { return __float_as_uint(f); }
@@ -442,13 +445,10 @@ TKD float segment_area_at(float xmin_abs, float xmax_abs, uint32_t x) {
 // Every term lies in (-2, 2): the edge term is signum * a clamp to [0, 1], dy is
 // the difference of two values clamped to [0, 1], and the area factor is at most
 // 1 up to rounding.  So t * 2^30 (exact, a power-of-two scaling) fits an int32
-// and one truncating v_cvt_i32_f32 gives trunc(t * 2^30); the instruction takes a
-// NaN to 0 (a C++ conversion of one is undefined, so it is named here).
+// and one truncating conversion gives trunc(t * 2^30); a NaN term counts as 0.
 constexpr float kCoverageOne = 1073741824.0f;  // 2^30
 TKD int32_t coverage_trunc(float scaled) {  // scaled: the term times kCoverageOne
-    int32_t q;
-    asm("v_cvt_i32_f32_e32 %0, %1" : "=v"(q) : "v"(scaled));
-    return q;
+    return f2i(scaled);
 }
 TKD long long coverage_fixed(float t) { return coverage_trunc(t * kCoverageOne); }
 // Back to FP32: the sum floored to a multiple of 2^-24 (at most 6e-8 below it),
