@@ -1,0 +1,129 @@
+"""The one-kernel scan of scenes laid out path by path (tk_k_path_scan): runs of
+small paths, paths at the edges of a run's tables, large paths shared out by tile
+rows, and the scenes it leaves to the separate stages, all against the oracle."""
+import numpy as np
+import pytest
+
+import tileink_amd as tk
+
+import oracle
+
+from helpers import channel_diff, compare_frame, read_frame, tile_sorted_segments
+
+pytestmark = pytest.mark.gpu
+
+RUN = 1024    # lines and tiles per run (TK_PATH_SCAN_RUN)
+LINES = 4096  # lines of the longest path it takes (TK_PATH_SCAN_LINES)
+
+
+def _box(canvas, x0, y0, tiles_x, tiles_y, rng):
+    """A concave polygon whose tile box is tiles_x by tiles_y tiles from (x0, y0)."""
+    w, h = 16 * tiles_x - 2, 16 * tiles_y - 2
+    mid = rng.uniform(0.2, 0.8, 2)
+    path = tk.BezPath().move_to(16 * x0 + 1, 16 * y0 + 1)
+    for u, v in ((1, 0), (mid[0], mid[1]), (1, 1), (0, 1)):
+        path.line_to(16 * x0 + 1 + u * w, 16 * y0 + 1 + v * h)
+    canvas.push_path(path.close_path(), tk.Color(*rng.uniform(0, 1, 3), 0.5), rule=tk.FillRule(int(rng.integers(2))))
+
+
+def _zigzag(canvas, lines, width, height, rng):
+    """One path of exactly `lines` lines."""
+    pts = rng.uniform((0.0, 0.0), (width, height), (lines, 2))
+    path = tk.BezPath().move_to(*pts[0])
+    for p in pts[1:]:
+        path.line_to(*p)
+    canvas.push_path(path.close_path(), tk.Color(0.2, 0.6, 0.9, 0.5), rule=tk.FillRule.EvenOdd)
+
+
+def _matches(ctx, canvas):
+    gpu, ref, bad = compare_frame(ctx, canvas)
+    assert not bad, (bad, channel_diff(gpu["image"], ref["image"]))
+
+
+# tile boxes: single tiles, a table's last row, one tile past 2 RUN (the first shared
+# size, one band), past 3 RUN, and many bands of uneven rows
+@pytest.mark.parametrize("tiles", [(1, 1), (64, 32), (683, 3), (64, 48), (96, 33), (131, 67), (1024, 5)])
+def test_path_sizes_match_oracle(ctx, tiles):
+    rng = np.random.default_rng(tiles[0])
+    tw, th = max(tiles[0] + 2, 20), max(tiles[1] + 2, 12)
+    canvas = tk.Canvas(16 * min(tw, 1024), 16 * th)
+    for k in range(5):
+        for _ in range(40):
+            _box(canvas, int(rng.integers(0, 15)), int(rng.integers(0, 8)), *rng.integers(1, 5, 2), rng)
+        _box(canvas, 0, k % 2, *tiles, rng)
+        canvas.push_path(tk.BezPath().move_to(-90, 5).line_to(-20, 9).line_to(-30, 40).close_path(), tk.Color(1, 0, 0, 1))
+    _matches(ctx, canvas)
+
+
+def test_shared_rows_meet_lines_that_leave_the_canvas(ctx):
+    rng = np.random.default_rng(5)
+    canvas = tk.Canvas(1500, 1100)
+    for k in range(6):
+        path = tk.BezPath().move_to(*rng.uniform(-900, 2400, 2))
+        for _ in range(12):
+            path.line_to(*rng.uniform(-900, 2400, 2))
+        canvas.push_path(path.close_path(), tk.Color(*rng.uniform(0, 1, 3), 0.4), rule=tk.FillRule(k % 2))
+        canvas.push_stroke(path, 7.0, tk.Color(0, 0.3 * (k % 3), 1, 0.6))
+    _matches(ctx, canvas)
+
+
+@pytest.mark.parametrize("lines,width,height", [(LINES, 200, 200), (LINES + 1, 200, 200), (300, 16 * (RUN + 1), 64)])
+def test_long_and_wide_paths_match_oracle(ctx, lines, width, height):
+    rng = np.random.default_rng(lines)
+    canvas = tk.Canvas(width, height)
+    _zigzag(canvas, 50, width, height, rng)
+    _zigzag(canvas, lines, width, height, rng)
+    _zigzag(canvas, 30, width, height, rng)
+    _matches(ctx, canvas)
+
+
+def _mixed_canvas():
+    rng = np.random.default_rng(11)
+    canvas = tk.Canvas(1300, 900)
+    for k in range(60):
+        if k % 20 == 7:
+            _zigzag(canvas, 40, 1300, 900, rng)
+        _box(canvas, int(rng.integers(0, 70)), int(rng.integers(0, 45)), *rng.integers(1, 12, 2), rng)
+    return canvas
+
+
+def test_lines_in_another_order_give_the_same_frame(ctx):
+    """Lines that do not lie path by path go through the separate stages, to the same
+    tables, segments and image; an update changes the route of a frame."""
+    arrays = _mixed_canvas().arrays(0)
+    shuffled = tk.SceneArrays.__new__(tk.SceneArrays)
+    shuffled.__dict__.update(arrays.__dict__)
+    shuffled.lines = arrays.lines[np.random.default_rng(1).permutation(len(arrays.lines))].copy()
+    scenes = [arrays.to_scene(), shuffled.to_scene()]
+    frame = tk.Frame(ctx, scenes[0])
+    frame.set_capture(True)
+    first = None
+    for scene in (scenes[0], scenes[1], scenes[0]):
+        frame.update(scene)
+        frame.render()
+        out = read_frame(frame, scene)
+        if first is None:
+            first = out
+        for key in ("raw_backdrops", "backdrops", "segment_counts", "segment_ranges", "segment_cursors", "segment_bumps",
+                    "tile_ptcl_counts", "tile_kinds", "ptcl", "image"):
+            assert np.array_equal(out[key], first[key]), key
+        assert np.array_equal(tile_sorted_segments(out["segments"], out["segment_ranges"]),
+                              tile_sorted_segments(first["segments"], first["segment_ranges"]))
+    assert np.array_equal(first["image"], oracle.render_frame(arrays)[0])
+
+
+def test_incremental_render_and_graph_replay_of_shared_rows(ctx):
+    canvas = _mixed_canvas()
+    scene = canvas.encode(0)
+    want = oracle.render_frame(canvas.arrays(0))[0]
+    frame = tk.Frame(ctx, scene)
+    frame.render()
+    assert np.array_equal(frame.image(), want)
+    T = scene.tiles_width * scene.tiles_height
+    for part in (np.arange(0, T, 7), np.array([T - 1]), np.arange(T)):
+        frame.render_tiles(part.astype(np.uint32))
+        assert np.array_equal(frame.image(), want)
+    frame.set_graph(True)
+    for _ in range(3):
+        frame.render()
+        assert np.array_equal(frame.image(), want)

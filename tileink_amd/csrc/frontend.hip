@@ -140,6 +140,7 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_fe_paths(tk_args_frontend
     }
     capacity = fe_wave_sum_u64(capacity);
     if (lane != 0u) return;
+    if (lines > TK_PATH_SCAN_LINES) atomicOr(a.status, 4u);  // scanned by the separate stages
     const uint32_t stride = tb[2] > tb[0] ? tb[2] - tb[0] : 0u, height = tb[3] > tb[1] ? tb[3] - tb[1] : 0u;
     const uint32_t data_len = stride * height;
     const uint32_t rows = stride && height ? height : 0u;

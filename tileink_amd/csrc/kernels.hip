@@ -2716,3 +2716,4 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_line_backward(tk_args_lin
 
 // The GPU front end of polygon scenes (tk_frame_set_polygons).
 #include "frontend.hip"
+#include "pathscan.hip"

@@ -73,7 +73,7 @@ struct tk_context {
     hipStream_t cur = nullptr;  // where launches go; null: `stream`
     hipEvent_t fork_a = nullptr, fork_b = nullptr, join = nullptr;
     hipFunction_t f_fill = nullptr, f_copy = nullptr, f_scan_clear = nullptr, f_scan_count = nullptr, f_scan_prefix = nullptr, f_scan_chunk_apply = nullptr,
-                  f_scan_emit = nullptr, f_cumsum = nullptr, f_coarse_count = nullptr,
+                  f_scan_emit = nullptr, f_cumsum = nullptr, f_path_scan = nullptr, f_path_scan_check = nullptr, f_coarse_count = nullptr,
                   f_coarse_scan = nullptr, f_coarse_emit = nullptr, f_layer_classes = nullptr, f_active_paths = nullptr,
                   f_draw_brush = nullptr,
                   f_fine = nullptr, f_coarse_count_scenes = nullptr, f_coarse_emit_scenes = nullptr,
@@ -97,6 +97,7 @@ struct tk_context {
                   f_flatten_count = nullptr, f_flatten_emit = nullptr;
     uint32_t compute_units = 0;
     // Scratch for the stage entry points (frames own their own).
+    uint32_t *refused = nullptr;  // pinned: tk_k_path_scan_check's answer
     uint32_t *tickets = nullptr;  // [0] scan prefix, [1] coarse scan
     unsigned long long *status = nullptr;
     size_t status_words = 0;
@@ -384,6 +385,7 @@ struct tk_frame {
     tk_scan_chunk *scan_chunks = nullptr;
     tk_scan_chunk_range *scan_chunk_ranges = nullptr;
     uint32_t *cs_offsets = nullptr, *cs_lens = nullptr, *cs_row_starts = nullptr, *cs_row_ends = nullptr;
+    bool path_scan = false;  // tk_k_path_scan takes the frame's scene
     // scan outputs
     int32_t *backdrops = nullptr, *raw_backdrops = nullptr;
     uint32_t *seg_counts = nullptr, *cursors = nullptr, *bumps = nullptr, *chunk_totals = nullptr,
@@ -556,9 +558,47 @@ uint64_t atlas_words(const tk_scene &s) {
     return s.atlas ? uint64_t(s.atlas_width) * s.atlas_height * s.atlas_pages : 0ull;
 }
 
+tk_scan_config frame_scan_config(const tk_scene &s) {
+    tk_scan_config c{};
+    c.clear_len = std::max({s.backdrop_len, s.path_count, s.scan_chunk_count});
+    c.backdrop_len = s.backdrop_len;
+    c.path_count = s.path_count;
+    c.scan_chunk_count = s.scan_chunk_count;
+    c.line_count = s.line_count;
+    c.segment_capacity = s.segment_capacity;
+    return c;
+}
+
+// Runs of tk_k_path_scan.
+uint32_t path_scan_runs(const tk_scene &s) {
+    return uint32_t((uint64_t(s.line_count) + s.backdrop_len) / TK_PATH_SCAN_RUN) + 1u;
+}
+
+// Whether tk_k_path_scan takes the scene whose records are in the frame's buffers:
+// *ctx->refused once the stream is idle.
+tk_status path_scan_check(tk_frame *f, const tk_scene &s) {
+    tk_args_path_scan_check a{};
+    a.cfg = frame_scan_config(s);
+    a.lines = f->lines;
+    a.paths = f->paths;
+    a.chunks = f->scan_chunks;
+    a.chunk_ranges = f->scan_chunk_ranges;
+    a.cs_offsets = f->cs_offsets;
+    a.cs_lens = f->cs_lens;
+    a.row_starts = f->cs_row_starts;
+    a.row_ends = f->cs_row_ends;
+    a.row_count = s.cumsum_row_count;
+    a.cs_chunk_count = s.cumsum_chunk_count;
+    *f->ctx->refused = 0u;
+    TK_HIP(hipHostGetDevicePointer(reinterpret_cast<void **>(&a.refused), f->ctx->refused, 0));
+    const uint32_t threads = std::max({1u, s.path_count, s.line_count, s.scan_chunk_count, s.cumsum_row_count});
+    return launch(f->ctx, f->ctx->f_path_scan_check, div_up(threads, 256), 1, 256, a);
+}
+
 tk_status frame_upload(tk_frame *f, const tk_scene *s) {
     f->diff_scene = diff_compatible(s);
     f->diff_ready = false;
+    f->path_scan = false;  // until the records are whole again
     TK_TRY(upload(f, f->lines, s->lines, s->line_count));
     TK_TRY(upload(f, f->paths, s->paths, s->path_count));
     TK_TRY(upload(f, f->draws, s->draws, s->draw_count));
@@ -575,6 +615,7 @@ tk_status frame_upload(tk_frame *f, const tk_scene *s) {
     TK_TRY(upload(f, f->cs_lens, s->cumsum_chunk_lens, s->cumsum_chunk_count));
     TK_TRY(upload(f, f->cs_row_starts, s->cumsum_row_starts, s->cumsum_row_count));
     TK_TRY(upload(f, f->cs_row_ends, s->cumsum_row_ends, s->cumsum_row_count));
+    TK_TRY(path_scan_check(f, *s));
     f->pair_count = 0;
     if (f->layer_bits && s->layer_count && s->layers) {
         const uint32_t pairs = layer_pairs(s, f->host_pair_of, f->host_pair_layer);
@@ -585,6 +626,7 @@ tk_status frame_upload(tk_frame *f, const tk_scene *s) {
         }
     }
     TK_HIP(hipStreamSynchronize(f->ctx->stream));
+    f->path_scan = *f->ctx->refused == 0u;
     return TK_OK;
 }
 
@@ -600,18 +642,6 @@ bool same_sizes(const tk_scene &a, const tk_scene &b, uint32_t index_capacity) {
            a.cumsum_row_count == b.cumsum_row_count && a.backdrop_len == b.backdrop_len &&
            a.segment_capacity == b.segment_capacity && a.ptcl_capacity <= b.ptcl_capacity &&
            a.max_clip_depth <= b.max_clip_depth;
-}
-
-tk_scan_config frame_scan_config(const tk_frame *f) {
-    const tk_scene &s = f->meta;
-    tk_scan_config c{};
-    c.clear_len = std::max({s.backdrop_len, s.path_count, s.scan_chunk_count});
-    c.backdrop_len = s.backdrop_len;
-    c.path_count = s.path_count;
-    c.scan_chunk_count = s.scan_chunk_count;
-    c.line_count = s.line_count;
-    c.segment_capacity = s.segment_capacity;
-    return c;
 }
 
 tk_coarse_config frame_coarse_config(const tk_frame *f) {
@@ -772,53 +802,31 @@ tk_status frame_render(tk_frame *f, uint32_t active_count = 0, const DiffTarget 
     const tk_tile_list list{active_count ? f->active_tiles : nullptr, active_count};
     const tk_scene_slots scenes{f->scene_slots, f->scene_of_column, f->scene_count, f->table_entries};
     const uint32_t *path_active = nullptr;
-    tk_scan_config scfg = frame_scan_config(f);
+    tk_scan_config scfg = frame_scan_config(s);
     const uint32_t T = s.tiles_width * s.tiles_height;
     f->epoch = (f->epoch + 1u) & 0x3FFFFFFFu;
     if (f->epoch == 0u) f->epoch = 1u;
 
+    const uint64_t status_words = 2ull * frame_scan_blocks(f, active_count);
     TK_TRY(record(f, 0));
-    // scan_clear: the deltas and counts accumulate; every other scan output is fully rewritten.
-    TK_TRY(fill_u32(ctx, f->backdrops, s.backdrop_len, 0u));
-    TK_TRY(fill_u32(ctx, f->seg_counts, s.backdrop_len, 0u));
-    TK_TRY(fill_u32(ctx, f->status, 4, 0u));
-    // The coarse scan's lookback words start each frame at zero, so a replayed
-    // graph (whose epoch argument is fixed) never sees the previous frame's flags.
-    TK_TRY(fill_u32(ctx, f->coarse_status, 2ull * frame_scan_blocks(f, active_count), 0u));
-    // The persistent launches' work counters (coarse count, coarse emit, fine) start at zero.
-    if (f->tuning.persistent) TK_TRY(fill_u32(ctx, f->queues, kQueueWords, 0u));
+    if (!f->path_scan) {
+        // scan_clear: the deltas and counts accumulate; every other scan output is fully rewritten.
+        TK_TRY(fill_u32(ctx, f->backdrops, s.backdrop_len, 0u));
+        TK_TRY(fill_u32(ctx, f->seg_counts, s.backdrop_len, 0u));
+        TK_TRY(fill_u32(ctx, f->status, 4, 0u));
+        // The coarse scan's lookback words start each frame at zero, so a replayed
+        // graph (whose epoch argument is fixed) never sees the previous frame's flags.
+        TK_TRY(fill_u32(ctx, f->coarse_status, status_words, 0u));
+        // The persistent launches' work counters (coarse count, coarse emit, fine) start at zero.
+        if (f->tuning.persistent) TK_TRY(fill_u32(ctx, f->queues, kQueueWords, 0u));
+    }
     if (active_count && s.path_count) {
         tk_args_active_paths ap{f->paths, s.path_count, s.tiles_width, s.tiles_height, f->damage_sat, f->path_active};
         TK_TRY(launch(ctx, ctx->f_active_paths, div_up(s.path_count, 256), 1, 256, ap));
         path_active = f->path_active;
     }
     TK_TRY(record(f, 1));
-    TK_TRY(run_scan_count(ctx, scfg, f->lines, f->paths, s.path_count, f->backdrops, f->seg_counts, path_active,
-                          f->tuning.scan_xcd_run, f->tuning.scan_block));
-    TK_TRY(record(f, 2));
-    // Fork A: the backdrop prefix needs only scan_count's deltas.
-    TK_HIP(hipEventRecord(ctx->fork_a, ctx->stream));
-    TK_HIP(hipStreamWaitEvent(ctx->side, ctx->fork_a, 0));
-    {
-        StreamScope on_side(ctx, ctx->side);
-        TK_TRY(record(f, 5));
-        if (f->capture_raw && s.backdrop_len)
-            TK_HIP(hipMemcpyAsync(f->raw_backdrops, f->backdrops, uint64_t(s.backdrop_len) * 4, hipMemcpyDeviceToDevice,
-                                  ctx->side));
-        tk_cumsum_config cc{s.cumsum_row_count, s.cumsum_chunk_count, 0u, 0u};
-        TK_TRY(run_cumsum(ctx, cc, f->cs_offsets, f->cs_lens, f->cs_row_starts, f->cs_row_ends, f->backdrops,
-                          f->cs_totals, f->cs_carries));
-        TK_TRY(record(f, 6));
-    }
-    TK_TRY(run_scan_prefix(ctx, scfg, f->scan_chunks, f->scan_chunk_ranges, f->paths, f->seg_counts, f->seg_ranges,
-                           f->cursors, f->bumps, f->chunk_totals, f->chunk_offsets));
-    TK_TRY(record(f, 3));
-    // Fork B: coarse needs the segment ranges (and the backdrops, earlier on the
-    // side stream), not the segments, so it overlaps scan_emit.
-    TK_HIP(hipEventRecord(ctx->fork_b, ctx->stream));
-    TK_HIP(hipStreamWaitEvent(ctx->side, ctx->fork_b, 0));
-    {
-        StreamScope on_side(ctx, ctx->side);
+    const auto coarse = [&]() -> tk_status {
         TK_TRY(record(f, 11));
         tk_coarse_config cc = frame_coarse_config(f);
         // Fields are set by name: the structs are part of the public ABI and may grow.
@@ -853,14 +861,65 @@ tk_status frame_render(tk_frame *f, uint32_t active_count = 0, const DiffTarget 
             TK_TRY(record(f, 7));
             TK_TRY(record(f, 8));
         }
-        TK_TRY(record(f, 9));
-        TK_HIP(hipEventRecord(ctx->join, ctx->side));
+        return record(f, 9);
+    };
+    if (f->path_scan) {
+        // One kernel, which also clears what the stages above clear; its time is scan_count's.
+        tk_args_path_scan a{};
+        a.cfg = scfg;
+        a.lines = f->lines;
+        a.paths = f->paths;
+        a.path_count = s.path_count;
+        a.path_active = path_active;
+        a.counts = f->seg_counts;
+        a.ranges = f->seg_ranges;
+        a.cursors = f->cursors;
+        a.bumps = f->bumps;
+        a.raw_backdrops = f->capture_raw ? f->raw_backdrops : nullptr;
+        a.backdrops = f->backdrops;
+        a.segments = f->segments;
+        a.clear[0] = {f->status, 4};
+        a.clear[1] = {reinterpret_cast<uint32_t *>(f->coarse_status), status_words};
+        a.clear[2] = {f->queues, f->tuning.persistent ? kQueueWords : 0};
+        TK_TRY(launch(ctx, ctx->f_path_scan, path_scan_runs(s), 1, 256, a));
+        for (int mark : {2, 3, 4, 5, 6}) TK_TRY(record(f, mark));
+        TK_TRY(coarse());
+    } else {
+        TK_TRY(run_scan_count(ctx, scfg, f->lines, f->paths, s.path_count, f->backdrops, f->seg_counts, path_active,
+                              f->tuning.scan_xcd_run, f->tuning.scan_block));
+        TK_TRY(record(f, 2));
+        // Fork A: the backdrop prefix needs only scan_count's deltas.
+        TK_HIP(hipEventRecord(ctx->fork_a, ctx->stream));
+        TK_HIP(hipStreamWaitEvent(ctx->side, ctx->fork_a, 0));
+        {
+            StreamScope on_side(ctx, ctx->side);
+            TK_TRY(record(f, 5));
+            if (f->capture_raw && s.backdrop_len)
+                TK_HIP(hipMemcpyAsync(f->raw_backdrops, f->backdrops, uint64_t(s.backdrop_len) * 4,
+                                      hipMemcpyDeviceToDevice, ctx->side));
+            tk_cumsum_config cc{s.cumsum_row_count, s.cumsum_chunk_count, 0u, 0u};
+            TK_TRY(run_cumsum(ctx, cc, f->cs_offsets, f->cs_lens, f->cs_row_starts, f->cs_row_ends, f->backdrops,
+                              f->cs_totals, f->cs_carries));
+            TK_TRY(record(f, 6));
+        }
+        TK_TRY(run_scan_prefix(ctx, scfg, f->scan_chunks, f->scan_chunk_ranges, f->paths, f->seg_counts, f->seg_ranges,
+                               f->cursors, f->bumps, f->chunk_totals, f->chunk_offsets));
+        TK_TRY(record(f, 3));
+        // Fork B: coarse needs the segment ranges (and the backdrops, earlier on the
+        // side stream), not the segments, so it overlaps scan_emit.
+        TK_HIP(hipEventRecord(ctx->fork_b, ctx->stream));
+        TK_HIP(hipStreamWaitEvent(ctx->side, ctx->fork_b, 0));
+        {
+            StreamScope on_side(ctx, ctx->side);
+            TK_TRY(coarse());
+            TK_HIP(hipEventRecord(ctx->join, ctx->side));
+        }
+        TK_TRY(run_scan_emit(ctx, scfg, f->lines, f->paths, s.path_count, f->cursors, f->segments, path_active,
+                             f->tuning.scan_xcd_run, f->tuning.scan_block));
+        TK_TRY(record(f, 4));
+        // Join: fine reads the segments and the PTCL.
+        TK_HIP(hipStreamWaitEvent(ctx->stream, ctx->join, 0));
     }
-    TK_TRY(run_scan_emit(ctx, scfg, f->lines, f->paths, s.path_count, f->cursors, f->segments, path_active,
-                         f->tuning.scan_xcd_run, f->tuning.scan_block));
-    TK_TRY(record(f, 4));
-    // Join: fine reads the segments and the PTCL.
-    TK_HIP(hipStreamWaitEvent(ctx->stream, ctx->join, 0));
     TK_TRY(record(f, 12));
     if (diff) {
         TK_TRY(fill_u32(ctx, f->diff_status, 1, 0u));
@@ -1113,6 +1172,8 @@ tk_status tk_context_create(int device, tk_context **out) {
         {&ctx->f_scan_chunk_apply, "tk_k_scan_chunk_apply"},
         {&ctx->f_scan_emit, "tk_k_scan_emit"},
         {&ctx->f_cumsum, "tk_k_cumsum"},
+        {&ctx->f_path_scan, "tk_k_path_scan"},
+        {&ctx->f_path_scan_check, "tk_k_path_scan_check"},
         {&ctx->f_coarse_count, "tk_k_coarse_count"},
         {&ctx->f_coarse_scan, "tk_k_coarse_scan"},
         {&ctx->f_coarse_emit, "tk_k_coarse_emit"},
@@ -1177,6 +1238,8 @@ tk_status tk_context_create(int device, tk_context **out) {
     }
     if (hipMalloc(&ctx->tickets, 16) != hipSuccess) return cleanup(fail(TK_ERR_OOM, "ticket allocation failed"));
     if (hipMemset(ctx->tickets, 0, 16) != hipSuccess) return cleanup(fail(TK_ERR_HIP, "ticket clear failed"));
+    if (hipHostMalloc(reinterpret_cast<void **>(&ctx->refused), sizeof(uint32_t)) != hipSuccess)
+        return cleanup(fail(TK_ERR_OOM, "pinned host allocation failed"));
     {
         void *scratch = nullptr;
         const tk_status st = scratch_address(device, &scratch);
@@ -1193,6 +1256,7 @@ void tk_context_destroy(tk_context *ctx) {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     if (ctx->status) (void)hipFree(ctx->status);
     if (ctx->tickets) (void)hipFree(ctx->tickets);
+    if (ctx->refused) (void)hipHostFree(ctx->refused);
     if (ctx->draw_brush) (void)hipFree(ctx->draw_brush);
     if (ctx->module) (void)hipModuleUnload(ctx->module);
     for (hipEvent_t e : {ctx->fork_a, ctx->fork_b, ctx->join})
@@ -1373,6 +1437,7 @@ tk_status frame_set_geometry(tk_frame *f, const FeInput &in) {
     uint32_t *line_vertex = in.line_vertex;
     tk_context *ctx = f->ctx;
     TK_TRY(fe_prepare(f));
+    f->path_scan = false;  // until the records are whole again
     tk_scene &s = f->meta;
     const uint32_t P = s.path_count, D = s.draw_count, Q = s.batch_count, R = f->fe_rows;
     const uint32_t C = s.tiles_width * s.tiles_height;  // table columns (a batch: all scenes' tiles)
@@ -1428,6 +1493,7 @@ tk_status frame_set_geometry(tk_frame *f, const FeInput &in) {
     TK_HIP(hipMemcpyAsync(f->fe_host, f->fe_totals, TK_FE_TOTALS * 8, hipMemcpyDeviceToHost, ctx->stream));
     TK_HIP(hipMemcpyAsync(f->fe_host + TK_FE_TOTALS, f->fe_status, 8, hipMemcpyDeviceToHost, ctx->stream));
     TK_HIP(hipStreamSynchronize(ctx->stream));
+    drop_graph(f);  // the streams are idle, and the path records already changed
     const unsigned long long *t = f->fe_host;
     const uint32_t flags = uint32_t(t[TK_FE_TOTALS]), overflow = uint32_t(t[TK_FE_TOTALS] >> 32);
     if (flags & 1u) return fail(TK_ERR_INVALID, "non-finite vertex: the frame needs valid vertices before it renders");
@@ -1437,7 +1503,6 @@ tk_status frame_set_geometry(tk_frame *f, const FeInput &in) {
     if (t[TK_FE_LINES] > point_count) return fail(TK_ERR_INVALID, "more lines than vertices");
 
     // Grow what the new geometry needs (the streams are idle).
-    drop_graph(f);
     const uint64_t lines = t[TK_FE_LINES], backdrops = t[TK_FE_BACKDROPS], segments = t[TK_FE_SEGMENTS];
     const uint64_t chunks = t[TK_FE_SCAN_CHUNKS], cs_rows = t[TK_FE_CUMSUM_ROWS], cs_chunks = t[TK_FE_CUMSUM_CHUNKS];
     if (grow(f->cap_lines, lines)) TK_TRY(reallocate(f, &f->lines, f->cap_lines));
@@ -1510,6 +1575,11 @@ tk_status frame_set_geometry(tk_frame *f, const FeInput &in) {
     s.tile_draw_index_count = uint32_t(t[TK_FE_TILE_REFS]);
     s.ptcl_capacity = t[TK_FE_PTCL];
     f->diff_ready = false;
+    // The front end lays paths out as the one-kernel scan takes them, unless one is too
+    // long (status bit 2) or too wide for it.
+    uint32_t widest = 0;
+    for (const tk_fe_scene &scene : f->fe_scenes_host) widest = std::max(widest, scene.tiles_width);
+    f->path_scan = !(flags & 4u) && widest <= TK_PATH_SCAN_RUN;
     return TK_OK;
 }
 
@@ -1991,6 +2061,7 @@ tk_status tk_frame_autotune(tk_frame *f, uint32_t repeats, tk_tuning *chosen) {
     tk_status st = TK_OK;
     for (const Axis &axis : axes) {
         if (st != TK_OK) break;
+        if (axis.stage == kScan && f->path_scan) continue;  // of the separate scan stages only
         float best_ms = 0.0f;
         tk_tuning axis_best = best;
         for (size_t i = 0; i < axis.values.size() && st == TK_OK; ++i) {

@@ -107,6 +107,39 @@ struct tk_args_scan_prefix {
     uint32_t wave_count;  // pass A: max(chunks, ceil(paths / 64)) waves
 };
 
+// The scan of a frame laid out path by path, in one kernel (pathscan.hip).
+#define TK_PATH_SCAN_RUN 1024u     // lines and tiles per run
+#define TK_PATH_SCAN_LINES 4096u   // lines of a path that one workgroup still scans
+struct tk_args_path_scan {
+    tk_scan_config cfg;
+    const tk_line *lines;
+    const tk_path_record *paths;
+    uint32_t path_count;
+    const uint32_t *path_active;  // incremental: as tk_args_scan_lines
+    uint32_t *counts;
+    tk_segment_range *ranges;
+    uint32_t *cursors;
+    uint32_t *bumps;
+    int32_t *raw_backdrops;       // the deltas before their prefix sums; null: not wanted
+    int32_t *backdrops;
+    tk_line_segment *segments;
+    struct {
+        uint32_t *words;
+        uint64_t count;
+    } clear[3];                   // words to clear on the way
+};
+
+struct tk_args_path_scan_check {
+    tk_scan_config cfg;
+    const tk_line *lines;
+    const tk_path_record *paths;
+    const tk_scan_chunk *chunks;
+    const tk_scan_chunk_range *chunk_ranges;
+    const uint32_t *cs_offsets, *cs_lens, *row_starts, *row_ends;
+    uint32_t row_count, cs_chunk_count;
+    uint32_t *refused;            // set to 1 when tk_k_path_scan does not take the scene
+};
+
 struct tk_args_cumsum {
     tk_cumsum_config cfg;
     const uint32_t *chunk_offsets_in;  // backdrop offset per chunk
