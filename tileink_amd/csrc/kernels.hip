@@ -358,6 +358,7 @@ struct CoarseCtx {
     const uint8_t *class_row;      // this tile's layer-pair classes, or null
     const uint32_t *class_pair_of; // per layer record: its pair
     uint32_t tw, th;               // the tile grid of this tile's canvas
+    uint32_t class_pairs;          // pairs of class_row
 };
 
 // Where a table column lives: its canvas's tile grid, its batches [q0, q1), and
@@ -442,6 +443,35 @@ __device__ Particle draw_particle(const CoarseCtx &c, uint32_t batch, uint32_t d
     return p;
 }
 
+// draw_particle of a draw from its table entry {box}, {tile, batch and kind words}.
+__device__ __forceinline__ Particle entry_particle(const CoarseCtx &c, uint32_t draw_index, uint4 box, uint4 words) {
+    Particle p{false, TK_PTCL_FILL, 0u, 0u, 0u, 0u, 0u};
+    const uint32_t kind = words.w & TK_ENTRY_KIND;
+    if (kind == TK_ENTRY_RECORD) return draw_particle(c, words.z, draw_index);
+    if (kind == TK_ENTRY_NONE || c.tx < box.x || c.ty < box.y || c.tx >= box.z || c.ty >= box.w) return p;
+    const uint32_t bd = words.x + c.ty * words.y + c.tx;
+    const tk_segment_range range = c.in->segment_ranges[bd];
+    const uint32_t winding = (uint32_t)c.in->backdrops[bd];
+    if (range.start == range.end && winding == 0u) return p;
+    p.valid = true;
+    p.winding = winding;
+    p.fill_rule = words.w >> 8;
+    p.seg_start = range.start;
+    p.seg_end = range.end;
+    p.color = draw_index;
+    if (kind == TK_ENTRY_CLIP) {
+        p.tag = TK_PTCL_BEGIN_CLIP;
+        p.color = 0u;
+    } else if (kind == TK_ENTRY_GLYPH) {
+        p.tag = kPtclPathGlyph;
+    } else if ((words.w & TK_ENTRY_SOLID_RECT) && range.start == range.end) {
+        p.tag = TK_PTCL_COLOR;
+        p.color = solid_color(constant(c.in->paint), c.cfg->paint_words, c.cfg->paint_brush_base,
+                              load_draw(c.in->draws, c.cfg->draw_count, draw_index));
+    }
+    return p;
+}
+
 __device__ __forceinline__ uint32_t particle_class_flags(const CoarseCtx &c, uint32_t draw_index, uint32_t tag) {
     if (tag == TK_PTCL_COLOR) return kClassColor;
     if (tag == kPtclImage) return kClassSdf;
@@ -499,8 +529,9 @@ __device__ __forceinline__ uint32_t layer_bits_at(const CoarseCtx &c, uint32_t i
 // The coarse view of table column `column`, whose tile is `tile` of its canvas.
 __device__ __forceinline__ CoarseCtx coarse_ctx(const tk_args_coarse &a, const SceneView &v, uint32_t tile,
                                                 uint32_t column) {
-    CoarseCtx c{&a.cfg, &a.in, tile % v.tw, tile / v.tw, nullptr, nullptr, v.tw, v.th};
+    CoarseCtx c{&a.cfg, &a.in, tile % v.tw, tile / v.tw, nullptr, nullptr, v.tw, v.th, 0u};
     if (a.classes.bits) {
+        c.class_pairs = a.classes.pair_count;
         c.class_row = a.classes.bits + (size_t)column * a.classes.pair_count;
         c.class_pair_of = a.classes.pair_of;
     }
@@ -1323,14 +1354,17 @@ __device__ uint32_t emit_stack_begins_wave(const CoarseCtx &c, uint32_t batch, E
 // kNone (and nothing is written) when a layer rejects the tile.  emitted and
 // end_tag keep what emit_stack_ends needs, so the END records are written
 // without loading the layers again (stack_ends_from_registers).
-__device__ uint32_t stack_begins_single_pass(const CoarseCtx &c, uint32_t batch, Emitter &e, uint32_t dst,
-                                             uint32_t lane, uint32_t &wrappers, uint64_t &emitted,
-                                             uint32_t &end_tag) {
+// class_lane: in lane k the tile's class of pair k, when the class table has at most
+// 64 pairs (one load less in the chain of every batch).
+__device__ uint32_t stack_begins_single_pass(const CoarseCtx &c, uint32_t first, uint32_t end, uint32_t class_lane,
+                                             Emitter &e, uint32_t dst, uint32_t lane, uint32_t &wrappers,
+                                             uint64_t &emitted, uint32_t &end_tag) {
     const tk_coarse_config &cfg = *c.cfg;
     const tk_coarse_inputs &in = *c.in;
-    const tk_batch_record br = in.batches[batch];
-    const uint32_t end = min(br.layer_end, cfg.layer_count);
-    const uint32_t i = br.layer_start + lane;
+    const uint32_t i = first + lane;
+    const bool in_lanes = c.class_row && c.class_pairs <= 64u;
+    uint32_t lane_bits = 0u;
+    if (in_lanes) lane_bits = (uint32_t)__shfl((int)class_lane, (int)(i < end ? c.class_pair_of[i] : 0u), 64);
     bool invalid = false, counted = false, emit = false;
     uint32_t tag = TK_PTCL_BEGIN_CLIP, winding = 0u, fill_rule = 0u, payload = 0u;
     tk_segment_range range{0u, 0u};
@@ -1338,7 +1372,7 @@ __device__ uint32_t stack_begins_single_pass(const CoarseCtx &c, uint32_t batch,
     if (i < end) {
         const tk_layer_record layer = in.layers[i];
         end_tag = layer.tag == 1u ? kPtclEndOpacity : (layer.tag == 2u ? kPtclEndBlend : TK_PTCL_END_CLIP);
-        const uint32_t bits = layer_bits_at(c, i, layer);
+        const uint32_t bits = in_lanes ? lane_bits : layer_bits_at(c, i, layer);
         invalid = (bits & kLayerInvalid) != 0u;
         counted = (bits & kLayerCounted) != 0u;
         emit = (bits & kLayerEmits) != 0u;
@@ -1405,20 +1439,35 @@ __device__ uint32_t emit_stack_ends_wave(const CoarseCtx &c, uint32_t batch, Emi
     return dst;
 }
 
-// One chunk of up to 64 list entries: lane's draw and batch (kNone when absent).
-__device__ __forceinline__ void load_list_entry(const tk_args_coarse &a, const tk_tile_draw_record &list, uint32_t base,
-                                                uint32_t lane, const SceneView &v, uint32_t &draw, uint32_t &batch) {
-    draw = kNone;
-    batch = kNone;
-    const uint32_t i = base + lane;
-    if (i < list.len) {
-        const uint32_t slot = list.start + i;
-        if (slot < a.cfg.tile_draw_index_count) {
-            draw = a.in.tile_draw_indices[slot];
-            if (draw < a.cfg.draw_count) batch = a.in.draw_batch_ids[draw];
-            if (batch < v.q0 || batch >= v.q1) batch = kNone;  // outside this canvas's batches
+// One chunk of up to 64 list entries: lane's draw and batch (kNone when absent), and
+// the draw's table entry where the frame has a table.
+struct ListEntry {
+    uint32_t draw, batch;
+    uint4 box, words;
+};
+__device__ __forceinline__ uint32_t list_draw(const tk_args_coarse &a, const tk_tile_draw_record &list, uint32_t len,
+                                              uint32_t i) {
+    if (i >= len) return kNone;
+    const uint32_t slot = list.start + i;
+    return slot < a.cfg.tile_draw_index_count ? a.in.tile_draw_indices[slot] : kNone;
+}
+__device__ __forceinline__ ListEntry list_entry(const tk_args_coarse &a, uint32_t draw, const SceneView &v) {
+    ListEntry e{draw, kNone, make_uint4(0u, 0u, 0u, 0u), make_uint4(0u, 0u, 0u, 0u)};
+    if (draw < a.cfg.draw_count) {
+        if (a.draw_entries) {
+            e.box = a.draw_entries[2u * (size_t)draw];
+            e.words = a.draw_entries[2u * (size_t)draw + 1u];
+            e.batch = e.words.z;
+        } else {
+            e.batch = a.in.draw_batch_ids[draw];
         }
     }
+    if (e.batch < v.q0 || e.batch >= v.q1) e.batch = kNone;  // outside this canvas's batches
+    return e;
+}
+__device__ __forceinline__ Particle list_particle(const tk_args_coarse &a, const CoarseCtx &c, const ListEntry &e) {
+    if (e.batch == kNone) return Particle{false, TK_PTCL_FILL, 0u, 0u, 0u, 0u, 0u};
+    return a.draw_entries ? entry_particle(c, e.draw, e.box, e.words) : draw_particle(c, e.batch, e.draw);
 }
 
 __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
@@ -1433,8 +1482,7 @@ __device__ uint32_t next_listed_batch(const tk_args_coarse &a, const tk_tile_dra
                                       uint32_t lane, const SceneView &v, uint32_t from) {
     uint32_t m = kNone;
     for (uint32_t base = 0; base < len; base += 64u) {
-        uint32_t d, b;
-        load_list_entry(a, list, base, lane, v, d, b);
+        const uint32_t b = list_entry(a, list_draw(a, list, len, base + lane), v).batch;
         if (b != kNone && b >= from) m = min(m, b);
     }
     return wave_min_u32(m);
@@ -1496,7 +1544,7 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_layer_classes(tk_args_lay
     if (pair >= a.pair_count || column >= a.list.columns) return;
     const uint32_t tile = a.list.tiles ? a.list.tiles[column] : column;
     const CoarseCtx c{&a.cfg,   &a.in,   tile % a.cfg.tiles_width, tile / a.cfg.tiles_width, nullptr, nullptr,
-                      a.cfg.tiles_width, a.cfg.tiles_height};
+                      a.cfg.tiles_width, a.cfg.tiles_height, 0u};
     a.bits[(uint64_t)column * a.pair_count + pair] = (uint8_t)layer_class_bits(c, a.in.layers[a.pair_layer[pair]]);
 }
 
@@ -1554,16 +1602,18 @@ __device__ __forceinline__ void coarse_count_tile(const tk_args_coarse &a, uint3
     bool disordered = false;
     uint32_t only = kNone;
     for (;;) {
+        uint32_t draw = list_draw(a, list, len, lane);
         for (uint32_t base = 0; base < len; base += 64u) {
-            uint32_t d, b;
-            load_list_entry(a, list, base, lane, v, d, b);
-            if (only != kNone && b != only) b = kNone;
-            const bool valid = b != kNone && draw_particle(c, b, d).valid;
+            ListEntry entry = list_entry(a, draw, v);
+            draw = list_draw(a, list, len, base + 64u + lane);  // the next chunk's, in flight meanwhile
+            if (only != kNone && entry.batch != only) entry.batch = kNone;
+            const uint32_t b = entry.batch;
+            const bool valid = list_particle(a, c, entry).valid;
             uint64_t pending_runs = __ballot(b != kNone);
             const uint64_t valid_mask = __ballot(valid);
             while (pending_runs) {
                 const uint32_t first = (uint32_t)__ffsll((unsigned long long)pending_runs) - 1u;
-                const uint32_t bb = (uint32_t)__shfl((int)b, (int)first, 64);
+                const uint32_t bb = (uint32_t)__builtin_amdgcn_readlane((int)b, (int)first);
                 const uint64_t run = __ballot(b == bb) & pending_runs;
                 pending_runs &= ~run;
                 if (bb != cur) {
@@ -1749,9 +1799,10 @@ __device__ __forceinline__ void coarse_emit_tile(const tk_args_coarse &a, uint32
         if (lane == 0u) kinds[table_index(v, cur)] = kind;
         next = cur + 1u;
     };
-    auto begin = [&](uint32_t bb) {
+    const uint32_t class_lane = c.class_row && lane < c.class_pairs ? c.class_row[lane] : 0u;
+    // r and br: the batch's table range and record
+    auto begin = [&](uint32_t bb, tk_segment_range r, tk_batch_record br) {
         cur = bb;
-        const tk_segment_range r = a.out.tile_ptcl_ranges[table_index(v, bb)];
         start = r.start;
         end = r.end;
         active = end > start;
@@ -1761,11 +1812,13 @@ __device__ __forceinline__ void coarse_emit_tile(const tk_args_coarse &a, uint32
         wrappers = 0u;
         dst = start;
         if (active) {
-            const tk_batch_record br = a.in.batches[bb];
             const uint32_t layer_end = min(br.layer_end, cfg.layer_count);
             single_pass = layer_end <= br.layer_start || layer_end - br.layer_start <= 64u;
-            if (single_pass) {
-                dst = stack_begins_single_pass(c, bb, e, start, lane, wrappers, stack_emitted, stack_end_tag);
+            if (layer_end <= br.layer_start) {
+                stack_emitted = 0ull;
+            } else if (single_pass) {
+                dst = stack_begins_single_pass(c, br.layer_start, layer_end, class_lane, e, start, lane, wrappers,
+                                               stack_emitted, stack_end_tag);
             } else {
                 wrappers = stack_wrapper_count_wave(c, bb, lane);
             }
@@ -1786,22 +1839,32 @@ __device__ __forceinline__ void coarse_emit_tile(const tk_args_coarse &a, uint32
     bool disordered = false;
     uint32_t only = kNone;
     for (;;) {
+        uint32_t draw = list_draw(a, list, len, lane);
         for (uint32_t base = 0; base < len; base += 64u) {
-            uint32_t d, b;
-            load_list_entry(a, list, base, lane, v, d, b);
-            if (only != kNone && b != only) b = kNone;
+            ListEntry entry = list_entry(a, draw, v);
+            draw = list_draw(a, list, len, base + 64u + lane);  // the next chunk's, in flight meanwhile
+            if (only != kNone && entry.batch != only) entry.batch = kNone;
+            const uint32_t b = entry.batch;
             // Every lane's particle and class at once (a lane's batch is its own b), so
-            // the particle code runs once per 64 entries however many batches they span.
-            Particle p{false, TK_PTCL_FILL, 0u, 0u, 0u, 0u, 0u};
-            if (b != kNone) p = draw_particle(c, b, d);
+            // the particle code runs once per 64 entries however many batches they span;
+            // likewise its batch's range and record, and the particles' stores.
+            tk_segment_range my_range{0u, 0u};
+            tk_batch_record my_record{0u, 0u};
+            if (b != kNone) {
+                my_range = a.out.tile_ptcl_ranges[table_index(v, b)];
+                my_record = a.in.batches[b];
+            }
+            uint32_t my_pos = kNone;
+            const Particle p = list_particle(a, c, entry);
             uint32_t cls = 0u;
-            if (p.valid) cls = particle_class_flags(c, d, p.tag);
+            if (p.valid) cls = particle_class_flags(c, entry.draw, p.tag);
             const bool p_opaque = p.valid && p.tag == TK_PTCL_COLOR && (p.color >> 24) == 255u;
             const bool p_begins = p.valid && is_begin_tag(p.tag);
             uint64_t pending = __ballot(b != kNone);
             while (pending) {
                 const uint32_t first = (uint32_t)__ffsll((unsigned long long)pending) - 1u;
-                const uint32_t bb = (uint32_t)__shfl((int)b, (int)first, 64);
+                const auto value = [&](uint32_t x) { return (uint32_t)__builtin_amdgcn_readlane((int)x, (int)first); };
+                const uint32_t bb = value(b);
                 const uint64_t run = __ballot(b == bb) & pending;
                 pending &= ~run;
                 if (bb != cur) {
@@ -1811,7 +1874,8 @@ __device__ __forceinline__ void coarse_emit_tile(const tk_args_coarse &a, uint32
                     }
                     finish();
                     empty_until(bb);
-                    begin(bb);
+                    begin(bb, tk_segment_range{value(my_range.start), value(my_range.end)},
+                          tk_batch_record{value(my_record.layer_start), value(my_record.layer_end)});
                 }
                 if (!active) continue;
                 const bool mine = (run >> lane) & 1ull;
@@ -1820,7 +1884,7 @@ __device__ __forceinline__ void coarse_emit_tile(const tk_args_coarse &a, uint32
                 const uint32_t pos = dst + (uint32_t)__popcll(valid & lanes_below(lane));
                 const uint32_t my_cls = emits ? cls : 0u;
                 const bool opaque = emits && p_opaque, begins = emits && p_begins;
-                if (emits && pos < end) e.store(pos, p.tag, p.winding, p.fill_rule, p.seg_start, p.seg_end, p.color);
+                if (emits && pos < end) my_pos = pos;
                 if (__ballot(my_cls & kClassColor)) flags |= kClassColor;
                 if (__ballot(my_cls & kClassSdf)) flags |= kClassSdf;
                 if (__ballot(my_cls & kClassOther)) flags |= kClassOther;
@@ -1835,6 +1899,7 @@ __device__ __forceinline__ void coarse_emit_tile(const tk_args_coarse &a, uint32
                 }
                 dst += (uint32_t)__popcll(valid);
             }
+            if (my_pos != kNone) e.store(my_pos, p.tag, p.winding, p.fill_rule, p.seg_start, p.seg_end, p.color);
         }
         if (!disordered) break;
         uint32_t from = only + 1u;
@@ -1863,27 +1928,54 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_coarse_emit_scenes_persis
     coarse_tiles<true>(a, 8u, [&](uint32_t column) { coarse_emit_tile<true>(a, column); });
 }
 
-// The colour sample_draw_brush returns for a draw whose brush does not depend on
-// the pixel (solid, and the kinds sample_brush maps to the header colour or to
-// 0), so that a fill reads one table entry instead of the draw record and then
-// its brush header (shared/brush/sample.hlsli:15-42); the entry holds the colour's
-// bytes as floats too, which the blend takes from scalar registers.
-extern "C" __global__ __launch_bounds__(256) void tk_k_draw_brush(tk_args_draw_brush a) {
+// The per-draw tables of a frame.  Brush: the colour sample_draw_brush returns for a
+// draw whose brush does not depend on the pixel (solid, and the kinds sample_brush
+// maps to the header colour or to 0), so that a fill reads one table entry instead of
+// the draw record and then its brush header (shared/brush/sample.hlsli:15-42); the
+// entry holds the colour's bytes as floats too, which the blend takes from scalar
+// registers.  Entry: what draw_particle reads of the draw and path records (200 bytes
+// over three or four cache lines) for every (tile, draw) pair, in 32 bytes.
+extern "C" __global__ __launch_bounds__(256) void tk_k_draw_tables(tk_args_draw_tables a) {
     const uint32_t d = blockIdx.x * 256u + threadIdx.x;
     if (d >= a.draw_count) return;
-    const uint32_t offset = a.draws[d].brush_offset;
-    const uint32_t kind = blob_word(constant(a.paint), a.paint_words, a.paint_brush_base, offset);
-    const uint32_t color = blob_word(constant(a.paint), a.paint_words, a.paint_brush_base, offset + 4u);
-    uint32_t flag = 1u, value = color;
-    if (kind == TK_BRUSH_LINEAR || kind == TK_BRUSH_RADIAL || kind == TK_BRUSH_SWEEP || kind == TK_BRUSH_FOUR_CORNER ||
-        kind == TK_BRUSH_IMAGE)
-        flag = 0u, value = 0u;
-    else if (kind == 6u)  // BRUSH_PATTERN
-        value = 0u;
-    uint4 *entry = reinterpret_cast<uint4 *>(a.table + (size_t)d * TK_DRAW_BRUSH_WORDS);
-    entry[0] = make_uint4(flag, value, 0u, 0u);
-    entry[1] = make_uint4(__float_as_uint((float)(value & 255u)), __float_as_uint((float)((value >> 8) & 255u)),
-                          __float_as_uint((float)((value >> 16) & 255u)), __float_as_uint((float)(value >> 24)));
+    if (a.brushes) {
+        const uint32_t offset = a.draws[d].brush_offset;
+        const uint32_t kind = blob_word(constant(a.paint), a.paint_words, a.paint_brush_base, offset);
+        const uint32_t color = blob_word(constant(a.paint), a.paint_words, a.paint_brush_base, offset + 4u);
+        uint32_t flag = 1u, value = color;
+        if (kind == TK_BRUSH_LINEAR || kind == TK_BRUSH_RADIAL || kind == TK_BRUSH_SWEEP ||
+            kind == TK_BRUSH_FOUR_CORNER || kind == TK_BRUSH_IMAGE)
+            flag = 0u, value = 0u;
+        else if (kind == 6u)  // BRUSH_PATTERN
+            value = 0u;
+        uint4 *entry = reinterpret_cast<uint4 *>(a.brushes + (size_t)d * TK_DRAW_BRUSH_WORDS);
+        entry[0] = make_uint4(flag, value, 0u, 0u);
+        entry[1] = make_uint4(__float_as_uint((float)(value & 255u)), __float_as_uint((float)((value >> 8) & 255u)),
+                              __float_as_uint((float)((value >> 16) & 255u)), __float_as_uint((float)(value >> 24)));
+    }
+    if (a.entries) {
+        const DrawData draw = load_draw(a.draws, a.draw_count, d);
+        uint32_t kind = TK_ENTRY_NONE, base = 0u, stride = 0u;
+        uint4 box = make_uint4(0u, 0u, 0u, 0u);
+        if (draw_has_sdf(draw) || draw.fill_rule > 0xFFFFu) {
+            kind = TK_ENTRY_RECORD;
+        } else if (draw.path_id < a.path_count && draw.path_id != kNone &&
+                   (draw.tag == TK_DRAW_BRUSH || draw.tag == TK_DRAW_PATH_GLYPH || draw.tag == TK_DRAW_CLIP)) {
+            const tk_path_record &p = a.paths[draw.path_id];
+            // the draw's box (draw_hits_tile; a tile is inside its grid, so no limits) within the path's
+            box = make_uint4(max(tile_min_of(draw.pb[0], ~0u), p.tile_x0), max(tile_min_of(draw.pb[1], ~0u), p.tile_y0),
+                             min(tile_max_of(draw.pb[2], ~0u), p.tile_x1), min(tile_max_of(draw.pb[3], ~0u), p.tile_y1));
+            kind = draw.tag == TK_DRAW_BRUSH ? TK_ENTRY_FILL : (draw.tag == TK_DRAW_CLIP ? TK_ENTRY_CLIP : TK_ENTRY_GLYPH);
+            if (draw.tag == TK_DRAW_BRUSH && draw.solid_rect != 0u && draw.lb == 0.0f && draw.lc == 0.0f &&
+                nontransparent_solid(constant(a.paint), a.paint_words, a.paint_brush_base, draw))
+                kind |= TK_ENTRY_SOLID_RECT;
+            kind |= draw.fill_rule << 8;
+            stride = p.tile_x1 - p.tile_x0;
+            base = p.data_offset - p.tile_y0 * stride - p.tile_x0;
+        }
+        a.entries[2u * (size_t)d] = box;
+        a.entries[2u * (size_t)d + 1u] = make_uint4(base, stride, a.batch_ids[d], kind);
+    }
 }
 
 // Marks of fine's walk.

@@ -75,7 +75,7 @@ struct tk_context {
     hipFunction_t f_fill = nullptr, f_copy = nullptr, f_scan_clear = nullptr, f_scan_count = nullptr, f_scan_prefix = nullptr, f_scan_chunk_apply = nullptr,
                   f_scan_emit = nullptr, f_cumsum = nullptr, f_path_scan = nullptr, f_path_scan_check = nullptr, f_coarse_count = nullptr,
                   f_coarse_scan = nullptr, f_coarse_emit = nullptr, f_layer_classes = nullptr, f_active_paths = nullptr,
-                  f_draw_brush = nullptr,
+                  f_draw_tables = nullptr,
                   f_fine = nullptr, f_coarse_count_scenes = nullptr, f_coarse_emit_scenes = nullptr,
                   f_fine_scenes = nullptr, f_fine_diff = nullptr, f_fine_diff_scenes = nullptr,
                   f_fine_backward = nullptr, f_fine_backward_scenes = nullptr, f_line_backward = nullptr,
@@ -288,13 +288,13 @@ tk_status run_coarse(tk_context *ctx, const tk_coarse_config &cfg, const tk_coar
                      hipEvent_t *marks, const LayerClassPlan &plan = LayerClassPlan{},
                      tk_tile_list list = tk_tile_list{nullptr, 0u},
                      tk_scene_slots scenes = tk_scene_slots{nullptr, nullptr, 0u, 0ull},
-                     TileLaunch shape = TileLaunch{TK_XCD_CHUNK_COARSE}) {
+                     TileLaunch shape = TileLaunch{TK_XCD_CHUNK_COARSE}, const uint4 *draw_entries = nullptr) {
     if (!list.tiles) list.columns = cfg.tile_count;
     if (cfg.batch_count == 0 || list.columns == 0) return TK_OK;
     const uint32_t blocks = scenes.slots ? coarse_scan_blocks_for(scenes.table_entries, shape.scan_items)
                                          : coarse_scan_blocks(cfg, list.columns, shape.scan_items);
     tk_args_coarse a{cfg, in, out, status, ticket, epoch, blocks, tk_layer_classes{nullptr, nullptr, 0u}, list, scenes,
-                     shape.xcd_run, shape.queue};
+                     shape.xcd_run, shape.queue, draw_entries};
     if (plan.bits && plan.pair_count) {
         tk_args_layer_classes b{cfg, in, plan.pair_layer, plan.pair_count, plan.bits, list};
         // pair-major: div_up(columns, 256) workgroups per pair (the table is at most
@@ -329,8 +329,13 @@ tk_status run_coarse(tk_context *ctx, const tk_coarse_config &cfg, const tk_coar
     return TK_OK;
 }
 
-// `draw_brush` holds TK_DRAW_BRUSH_WORDS * cfg.draw_count words; it is rebuilt here from the draws
-// and paint before fine reads it.
+// Fine's brush words and coarse's entries of every draw (either may be null).
+tk_status run_draw_tables(tk_context *ctx, const tk_args_draw_tables &a) {
+    if (!a.draw_count) return TK_OK;
+    return launch(ctx, ctx->f_draw_tables, div_up(a.draw_count, 256), 1, 256, a);
+}
+
+// `draw_brush`: run_draw_tables' brush words.
 tk_status run_fine(tk_context *ctx, const tk_fine_config &cfg, const tk_fine_inputs &in, uint32_t *rgba,
                    uint32_t *draw_brush, tk_tile_list list = tk_tile_list{nullptr, 0u},
                    tk_scene_slots scenes = tk_scene_slots{nullptr, nullptr, 0u, 0ull},
@@ -339,10 +344,6 @@ tk_status run_fine(tk_context *ctx, const tk_fine_config &cfg, const tk_fine_inp
     if (cfg.clip_spill_depth > TK_FINE_MAX_CLIP_SPILL) {
         set_error("clip nesting deeper than %u is not supported", 4u + TK_FINE_MAX_CLIP_SPILL);
         return TK_ERR_INVALID;
-    }
-    if (cfg.draw_count) {
-        tk_args_draw_brush b{in.draws, cfg.draw_count, in.paint, cfg.paint_words, cfg.paint_brush_base, draw_brush};
-        TK_TRY(launch(ctx, ctx->f_draw_brush, div_up(cfg.draw_count, 256), 1, 256, b));
     }
     tk_args_fine a{cfg, in, rgba, draw_brush, list, scenes, xcd_run, queue};
     if (list.columns == 0) return TK_OK;
@@ -398,6 +399,7 @@ struct tk_frame {
     tk_ptcl_record *ptcl = nullptr;
     uint64_t ptcl_capacity = 0;
     uint32_t *draw_brush = nullptr;  // fine's per-draw brush words
+    uint4 *draw_entries = nullptr;   // coarse's per-draw entries
     // per-tile layer classes (coarse): see LayerClassPlan
     uint32_t *layer_pair_of = nullptr, *pair_layer = nullptr;
     uint8_t *layer_bits = nullptr;
@@ -820,6 +822,9 @@ tk_status frame_render(tk_frame *f, uint32_t active_count = 0, const DiffTarget 
         // The persistent launches' work counters (coarse count, coarse emit, fine) start at zero.
         if (f->tuning.persistent) TK_TRY(fill_u32(ctx, f->queues, kQueueWords, 0u));
     }
+    TK_TRY(run_draw_tables(ctx, tk_args_draw_tables{f->draws, s.draw_count, f->paint, s.paint_words, s.paint_brush_base,
+                                                    diff ? nullptr : f->draw_brush, f->draw_entries, f->paths,
+                                                    s.path_count, f->batch_ids}));
     if (active_count && s.path_count) {
         tk_args_active_paths ap{f->paths, s.path_count, s.tiles_width, s.tiles_height, f->damage_sat, f->path_active};
         TK_TRY(launch(ctx, ctx->f_active_paths, div_up(s.path_count, 256), 1, 256, ap));
@@ -856,7 +861,7 @@ tk_status frame_render(tk_frame *f, uint32_t active_count = 0, const DiffTarget 
             plan.bits = f->layer_bits;
         }
         TK_TRY(run_coarse(ctx, cc, in, out, f->coarse_status, &f->tickets[1], f->epoch, f->timing ? &f->ev[7] : nullptr,
-                          plan, list, scenes, coarse_launch(f)));
+                          plan, list, scenes, coarse_launch(f), f->draw_entries));
         if (cc.batch_count == 0 && f->timing) {
             TK_TRY(record(f, 7));
             TK_TRY(record(f, 8));
@@ -1049,7 +1054,8 @@ tk_status frame_create(tk_context *ctx, const tk_scene *s, const BatchLayout *ba
     ALLOC(status, 4);
     ALLOC(diff_status, 1);
     ALLOC(ptcl, f->ptcl_capacity);
-    ALLOC(draw_brush, TK_DRAW_BRUSH_WORDS * std::max<uint64_t>(s->draw_count, 1));
+    ALLOC(draw_brush, (TK_DRAW_BRUSH_WORDS + TK_DRAW_ENTRY_WORDS) * std::max<uint64_t>(s->draw_count, 1));
+    f->draw_entries = reinterpret_cast<uint4 *>(f->draw_brush + TK_DRAW_BRUSH_WORDS * std::max<uint64_t>(s->draw_count, 1));
     ALLOC(active_tiles, T);
     ALLOC(damage_sat, uint64_t(s->tiles_width + 1) * (s->tiles_height + 1));
     ALLOC(path_active, std::max<uint64_t>(s->path_count, 1));
@@ -1179,7 +1185,7 @@ tk_status tk_context_create(int device, tk_context **out) {
         {&ctx->f_coarse_emit, "tk_k_coarse_emit"},
         {&ctx->f_layer_classes, "tk_k_layer_classes"},
         {&ctx->f_active_paths, "tk_k_active_paths"},
-        {&ctx->f_draw_brush, "tk_k_draw_brush"},
+        {&ctx->f_draw_tables, "tk_k_draw_tables"},
         {&ctx->f_fine, "tk_k_fine"},
         {&ctx->f_coarse_count_scenes, "tk_k_coarse_count_scenes"},
         {&ctx->f_coarse_emit_scenes, "tk_k_coarse_emit_scenes"},
@@ -2462,6 +2468,8 @@ tk_status tk_fine(tk_context *ctx, const tk_fine_config *cfg, const tk_fine_inpu
     if (uint64_t(cfg->tiles_width) * cfg->tiles_height != cfg->tile_count)
         return fail(TK_ERR_INVALID, "tile_count must equal tiles_width * tiles_height");
     TK_TRY(ensure_draw_brush(ctx, TK_DRAW_BRUSH_WORDS * size_t(cfg->draw_count)));
+    TK_TRY(run_draw_tables(ctx, tk_args_draw_tables{in->draws, cfg->draw_count, in->paint, cfg->paint_words,
+                                                    cfg->paint_brush_base, ctx->draw_brush, nullptr, nullptr, 0u, nullptr}));
     return run_fine(ctx, *cfg, *in, rgba, ctx->draw_brush);
 }
 

@@ -175,6 +175,7 @@ struct tk_args_coarse {
     uint32_t xcd_run;  // XCD run length in four-tile workgroups (a power of two; 0: launch order)
     uint32_t *queue;   // 16 per-XCD work counters (count, emit), zero at launch: persistent count and emit
                        // launches, each wave taking tiles; null: one four-tile workgroup per launch item
+    const uint4 *draw_entries;  // tk_args_draw_tables::entries; null: the draw and path records are read
 };
 
 struct tk_args_layer_classes {
@@ -186,23 +187,40 @@ struct tk_args_layer_classes {
     tk_tile_list list;
 };
 
-// Per-draw brush words for fine, eight per draw: {1, colour, 0, 0, the colour's
-// four bytes as floats} when the draw's brush colour does not depend on the pixel,
-// zeros when it must be sampled.
+// Per-draw words for fine and coarse, built from the records in front of a frame.
+// Brush (fine), eight per draw: {1, colour, 0, 0, the colour's four bytes as floats}
+// when the draw's brush colour does not depend on the pixel, zeros when it must be
+// sampled.  Entry (coarse), eight per draw: the tile box {x0, y0, x1, y1} in which the
+// draw may cover tiles, then {base, stride, batch, kind | fill rule << 8}: the
+// backdrop tile of (x, y) is base + y * stride + x, modulo 2^32.
 #define TK_DRAW_BRUSH_WORDS 8u
-struct tk_args_draw_brush {
+#define TK_DRAW_ENTRY_WORDS 8u
+enum tk_draw_entry_kind : uint32_t {
+    TK_ENTRY_NONE = 0,       // never a particle
+    TK_ENTRY_FILL = 1,       // a brush over its path
+    TK_ENTRY_GLYPH = 2,
+    TK_ENTRY_CLIP = 3,
+    TK_ENTRY_RECORD = 4,     // by its record: SDF draws
+    TK_ENTRY_KIND = 7,
+    TK_ENTRY_SOLID_RECT = 8, // with FILL: a COLOR particle on tiles without segments
+};
+struct tk_args_draw_tables {
     const tk_draw_record *draws;
     uint32_t draw_count;
     const uint32_t *paint;
     uint32_t paint_words, paint_brush_base;
-    uint32_t *table;
+    uint32_t *brushes;                // null: not wanted
+    uint4 *entries;                   // null: not wanted
+    const tk_path_record *paths;      // the rest for entries only
+    uint32_t path_count;
+    const uint32_t *batch_ids;
 };
 
 struct tk_args_fine {
     tk_fine_config cfg;
     tk_fine_inputs in;
     uint32_t *rgba;
-    const uint32_t *draw_brush;  // tk_args_draw_brush::table, draw_count entries
+    const uint32_t *draw_brush;  // tk_args_draw_tables::brushes, draw_count entries
     tk_tile_list list;
     tk_scene_slots scenes;
     uint32_t xcd_run;  // XCD run length in tiles (a power of two; 0: launch order)
