@@ -12,8 +12,8 @@ from helpers import channel_diff, compare_frame, read_frame, tile_sorted_segment
 
 pytestmark = pytest.mark.gpu
 
-RUN = 1024    # lines and tiles per run (TK_PATH_SCAN_RUN)
-LINES = 4096  # lines of the longest path it takes (TK_PATH_SCAN_LINES)
+RUN = 928     # lines, tiles and paths (four each) per run, at most (TK_PATH_SCAN_RUN)
+LINES = 8192  # lines of the longest path it takes (TK_PATH_SCAN_LINES)
 
 
 def _box(canvas, x0, y0, tiles_x, tiles_y, rng):
@@ -40,13 +40,15 @@ def _matches(ctx, canvas):
     assert not bad, (bad, channel_diff(gpu["image"], ref["image"]))
 
 
-# tile boxes: single tiles, a table's last row, one tile past 2 RUN (the first shared
-# size, one band), past 3 RUN, and many bands of uneven rows
-@pytest.mark.parametrize("tiles", [(1, 1), (64, 32), (683, 3), (64, 48), (96, 33), (131, 67), (1024, 5)])
+# tile boxes on canvases little larger, in runs of 128 or the canvas's width: single
+# tiles, two runs' tiles and one more (the first size that is shared out), past three,
+# many bands of uneven rows, and the widest canvas
+@pytest.mark.parametrize("tiles", [(1, 1), (16, 16), (1, 256), (1, 257), (20, 13), (16, 24), (35, 11), (128, 2), (131, 67),
+                                   (RUN - 2, 4)])
 def test_path_sizes_match_oracle(ctx, tiles):
     rng = np.random.default_rng(tiles[0])
     tw, th = max(tiles[0] + 2, 20), max(tiles[1] + 2, 12)
-    canvas = tk.Canvas(16 * min(tw, 1024), 16 * th)
+    canvas = tk.Canvas(16 * tw, 16 * th)
     for k in range(5):
         for _ in range(40):
             _box(canvas, int(rng.integers(0, 15)), int(rng.integers(0, 8)), *rng.integers(1, 5, 2), rng)
@@ -74,6 +76,22 @@ def test_long_and_wide_paths_match_oracle(ctx, lines, width, height):
     _zigzag(canvas, 50, width, height, rng)
     _zigzag(canvas, lines, width, height, rng)
     _zigzag(canvas, 30, width, height, rng)
+    _matches(ctx, canvas)
+
+
+def test_lines_within_one_tile_match_the_general_traversal(ctx):
+    """Short lines, which skip the traversal: ends on tile corners and edges, level
+    lines on and off a tile's top, lines a hair long, at every side of the canvas."""
+    rng = np.random.default_rng(3)
+    canvas = tk.Canvas(100, 70)
+    for k in range(300):
+        at = rng.choice([0.0, 16.0, 32.0, 48.0, 63.9999, 64.0, 95.0, 96.0, 100.0], 2) * (1.0, 0.7)
+        path = tk.BezPath().move_to(*at)
+        for _ in range(int(rng.integers(2, 9))):
+            step = rng.choice([0.0, 1e-6, 1e-3, 0.5, 3.0, 15.9999, 16.0], 2) * rng.choice([-1.0, 1.0], 2)
+            at = at + step
+            path.line_to(*at)
+        canvas.push_path(path.close_path(), tk.Color(*rng.uniform(0, 1, 3), 0.5), rule=tk.FillRule(k % 2))
     _matches(ctx, canvas)
 
 

@@ -11,18 +11,25 @@
 // with LDS cursors.  Memory sees the lines twice, the tables once (no clear before,
 // no atomics on them) and the segments.
 //
-// Run r covers the positions [r, r + 1) * TK_PATH_SCAN_RUN of the line and tile
-// counts summed over the paths: it takes the paths that start there, the last of
-// which may reach beyond.  So the paths before the last hold fewer than one RUN of
-// tiles, and a path of up to two more is counted in the same tables, three RUNs
-// long.  A larger path leaves runs behind it in which no path starts; these share its
-// tile rows out among them.  Each reads all the path's lines, tables its own rows,
-// and finds where its segments start by counting the visits above them, so no
-// workgroup waits on another.
+// Run r covers the positions [r, r + 1) * RUN of the paths laid end to end, each as
+// long as its lines, its tiles and four: it takes the paths that start there (a
+// quarter of RUN at most), the last of which may reach beyond.  So the paths
+// before the last hold fewer than one RUN of tiles, and a path of up to two more is
+// counted in the same tables, three RUNs long.  A larger path leaves runs behind it in
+// which no path starts; these share its tile rows out among them.  Each reads all the
+// path's lines, tables its own rows, and finds where its segments start by counting
+// the visits above them, so no workgroup waits on another.
+//
+// Most lines of flattened curves stay in one tile and need neither the traversal's
+// quotients nor the clipping's, so each wave handles those as they come and queues
+// the others, to take them 64 at a time.  A line's loads stand one step ahead, and
+// its path comes from LDS: by the records, a step was a chain of three loads.
+// Bound by VALU issue (two thirds of the time) and, below a thousand runs, by the chain
+// of loads from a run's search to its segments.  11.3 M lines of 50,000 paths, 2.3 M
+// tiles, 14.8 M segments: 0.32 ms (the separate stages 0.80 ms, 0.45 ms of it beside
+// coarse); 27 lines of an icon: 14 us (six launches before, 36 us with their gaps).
 
 namespace {
-
-constexpr uint32_t kPathScanTiles = 3u * TK_PATH_SCAN_RUN;
 
 // What a workgroup carries: paths [first, end), their lines, and the tiles
 // [tile0, tile0 + tiles) of their slabs.
@@ -32,7 +39,7 @@ struct PathRun {
 };
 
 __device__ __forceinline__ uint64_t path_scan_position(const tk_args_path_scan &a, uint32_t p) {
-    return (uint64_t)a.paths[p].line_start + a.paths[p].data_offset;
+    return (uint64_t)a.paths[p].line_start + a.paths[p].data_offset + 4ull * p;
 }
 
 // Run r; false when nothing is left to it.  Its paths are found by a search, 64 probes
@@ -40,7 +47,7 @@ __device__ __forceinline__ uint64_t path_scan_position(const tk_args_path_scan &
 // table of them would be one more kernel and buffer in front of every scene.
 __device__ __forceinline__ bool path_run(const tk_args_path_scan &a, uint32_t r, PathRun &u) {
     const Const<tk_path_record> paths = constant(a.paths);
-    const uint64_t begin = (uint64_t)r * TK_PATH_SCAN_RUN, end = begin + TK_PATH_SCAN_RUN;
+    const uint64_t begin = (uint64_t)r * a.run, end = begin + a.run;
     const uint32_t lane = threadIdx.x & 63u;
     uint32_t lo = 0u, hi = a.path_count;  // the first path at or past `begin` is in [lo, hi]
     while (lo < hi) {
@@ -56,22 +63,23 @@ __device__ __forceinline__ bool path_run(const tk_args_path_scan &a, uint32_t r,
     }
     u.band = u.first >= u.end;
     if (!u.band) {
-        if (paths[u.end - 1u].data_len > 2u * TK_PATH_SCAN_RUN) u.end -= 1u;  // the runs after this one
+        if (paths[u.end - 1u].data_len > 2u * a.run) u.end -= 1u;  // the runs after this one
         if (u.first >= u.end) return false;
         const __attribute__((address_space(4))) tk_path_record &p = paths[u.first], &q = paths[u.end - 1u];
         u.line0 = p.line_start;
         u.line1 = q.line_start + q.line_count;
         u.tile0 = p.data_offset;
         u.tiles = q.data_offset + q.data_len - p.data_offset;
-        return u.tiles <= kPathScanTiles;
+        return u.tiles <= 3u * a.run;
     }
     if (u.first == 0u) return false;
     u.end = u.first;
     u.first -= 1u;
     const __attribute__((address_space(4))) tk_path_record &p = paths[u.first];
-    if (p.data_len <= 2u * TK_PATH_SCAN_RUN) return false;
-    const uint32_t k0 = (uint32_t)(((uint64_t)p.line_start + p.data_offset) / TK_PATH_SCAN_RUN);
-    const uint32_t k1 = (uint32_t)(((uint64_t)p.line_start + p.line_count + p.data_offset + p.data_len) / TK_PATH_SCAN_RUN);
+    if (p.data_len <= 2u * a.run) return false;
+    const uint64_t at = (uint64_t)p.line_start + p.data_offset + 4ull * u.first;
+    const uint32_t k0 = (uint32_t)(at / a.run);
+    const uint32_t k1 = (uint32_t)((at + p.line_count + p.data_len + 4u) / a.run);
     const uint32_t bands = k1 - k0 - 1u, rows = p.tile_y1 - p.tile_y0, width = p.tile_x1 - p.tile_x0;
     const uint32_t share = (rows + bands - 1u) / bands, row = (r - k0 - 1u) * share;
     if (row >= rows) return false;
@@ -79,125 +87,258 @@ __device__ __forceinline__ bool path_run(const tk_args_path_scan &a, uint32_t r,
     u.line1 = p.line_start + p.line_count;
     u.tile0 = p.data_offset + row * width;
     u.tiles = min(share, rows - row) * width;
-    return u.tiles <= kPathScanTiles;
+    return u.tiles <= 3u * a.run;
 }
 
-// The traversal of line `id`, unless an incremental render leaves its path out.
-__device__ __forceinline__ bool path_scan_line(const tk_args_path_scan &a, uint32_t id, ScanTraversal &s) {
-    if (a.path_active) {
-        const uint32_t path = a.lines[id].path_id;
-        if (path < a.path_count && a.path_active[path] == 0u) return false;
+// What a run keeps of each of its paths in LDS: its first tile less the run's, its
+// box {x0 | y0 << 16, x1 | flags | y1 << 16}, and its segments' start less the slots
+// before it in the run (once those are known).
+constexpr uint32_t kPathIdentity = 1u << 15, kPathLeftOut = 1u << 14;
+struct alignas(16) RunPath {
+    uint32_t first, low, high, offset;
+};
+static_assert(TK_PATH_SCAN_RUN < kPathLeftOut, "x1 and the flags share 16 bits");
+
+__device__ __forceinline__ bool is_identity(const tk_affine &t) {
+    return t.a == 1.0f && t.b == 0.0f && t.c == 0.0f && t.d == 1.0f && t.e == 0.0f && t.f == 0.0f;
+}
+
+// A line's box and end points; false when an incremental render leaves its path out
+// or the box is empty.  data_offset is relative to the run.
+__device__ __forceinline__ bool path_scan_line(const tk_args_path_scan &a, const tk_line &line, const RunPath &p,
+                                               ScanTraversal &s) {
+    s = ScanTraversal{};
+    s.data_offset = p.first;
+    s.bx = p.low & 0xFFFFu;
+    s.by = p.low >> 16;
+    s.bz = p.high & (kPathLeftOut - 1u);
+    s.bw = p.high >> 16;
+    if ((p.high & kPathLeftOut) || s.bx >= s.bz || s.by >= s.bw) return false;
+    tk_affine t{1.0f, 0.0f, 0.0f, 1.0f, 0.0f, 0.0f};
+    if (!(p.high & kPathIdentity)) t = a.paths[line.path_id].transform;
+    scan_endpoints(line, t, s);
+    return true;
+}
+
+// Passes the workgroup's lines: one(s, path, tx, ty) for a line in one tile, many(s,
+// path) for any other that visits tiles; `path` is its RunPath.  `queue`: the wave's,
+// 128 entries.
+template <class One, class Many>
+__device__ __forceinline__ void path_scan_lines(const tk_args_path_scan &a, const PathRun &u, const RunPath *paths,
+                                                uint16_t *queue, One one, Many many) {
+    const uint32_t lane = threadIdx.x & 63u, n = u.line1 - u.line0;
+    const auto load = [&](uint32_t index) { return index < n ? a.lines[u.line0 + index] : tk_line{}; };
+    const auto order = [] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    const auto general = [&](uint32_t index) {
+        const tk_line line = load(index);
+        const RunPath path = paths[line.path_id - u.first];
+        ScanTraversal s;
+        if (path_scan_line(a, line, path, s) && scan_traverse(s)) many(s, path);
+    };
+    uint32_t held = 0u;  // fewer than 64 queued between steps
+    const uint32_t wave_base = uniform(threadIdx.x & ~63u);
+    tk_line next = load(wave_base + lane);
+    for (uint32_t base = wave_base; base < n; base += 256u) {
+        const uint32_t index = base + lane;
+        const tk_line line = next;
+        next = load(index + 256u);
+        bool queued = false;
+        if (index < n) {
+            const RunPath path = paths[line.path_id - u.first];
+            ScanTraversal s;
+            if (path_scan_line(a, line, path, s)) {
+                int32_t tx, ty;
+                const ScanSingle single = scan_single_tile(s, tx, ty);
+                if (single == kScanOne) one(s, path, tx, ty);
+                queued = single == kScanGeneral;
+            }
+        }
+        const uint64_t mask = __ballot(queued);
+        if (queued) queue[held + (uint32_t)__popcll(mask & lanes_below(lane))] = (uint16_t)index;
+        held += (uint32_t)__popcll(mask);
+        order();
+        if (held >= 64u) {
+            held -= 64u;
+            general(queue[held + lane]);
+            order();
+        }
     }
-    return scan_geometry(a.lines, a.paths, a.path_count, id, s);
+    if (lane < held) general(queue[lane]);
+    order();
 }
 
 }  // namespace
 
 extern "C" __global__ __launch_bounds__(256) void tk_k_path_scan(tk_args_path_scan a) {
-    __shared__ uint32_t counts[kPathScanTiles], deltas[kPathScanTiles];
-    __shared__ uint32_t s_before;
+    // Its paths, at most RUN / 4; per tile the visits, then the slots before it among
+    // the run's (one word past the end for the last's); per tile the backdrop delta,
+    // then the deltas' running sum.
+    extern __shared__ uint32_t path_scan_lds[];  // TK_PATH_SCAN_LDS(run)
+    RunPath *paths = reinterpret_cast<RunPath *>(path_scan_lds);
+    uint32_t *slots = path_scan_lds + 4u * ((a.run + 3u) / 4u), *deltas = slots + 3u * a.run + 1u;
+    __shared__ uint16_t queues[4][128];
+    __shared__ uint32_t sums[2][2][4], s_before;
+    static_assert(TK_PATH_SCAN_LINES + TK_PATH_SCAN_RUN < 65536u, "the queues hold line numbers in 16 bits");
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = uniform(tid >> 6);
 #pragma unroll
     for (uint32_t k = 0; k < 3u; ++k)  // words that later kernels of the frame start from zero
-        for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < a.clear[k].count; i += gridDim.x * 256ull)
+        for (uint64_t i = blockIdx.x * 256ull + tid; i < a.clear[k].count; i += gridDim.x * 256ull)
             a.clear[k].words[i] = 0u;
     PathRun u;
     if (!path_run(a, blockIdx.x, u)) return;
-    for (uint32_t t = threadIdx.x; t < u.tiles; t += 256u) {
-        counts[t] = 0u;
+    const uint32_t path_count = u.end - u.first;  // at most RUN / 4
+    uint32_t path_end = 0u;                       // thread j: path j's tiles end here
+    bool last_part = true;                        // and with them the path
+    if (tid < path_count) {
+        const tk_path_record &p = a.paths[u.first + tid];
+        const bool left_out = a.path_active && a.path_active[u.first + tid] == 0u;
+        paths[tid] = RunPath{p.data_offset - u.tile0, p.tile_x0 | (p.tile_y0 << 16),
+                             p.tile_x1 | (is_identity(p.transform) ? kPathIdentity : 0u) |
+                                 (left_out ? kPathLeftOut : 0u) | (p.tile_y1 << 16),
+                             p.segment_start};
+        path_end = p.data_offset - u.tile0 + p.data_len;
+        last_part = path_end <= u.tiles;
+        path_end = min(path_end, u.tiles);
+    }
+    for (uint32_t t = tid; t < u.tiles; t += 256u) {
+        slots[t] = 0u;
         deltas[t] = 0u;
     }
-    if (threadIdx.x == 0u) s_before = 0u;
+    if (tid == 0u) s_before = 0u;
     __syncthreads();
 
     uint32_t before = 0u;  // visits above a band
-    for (uint32_t id = u.line0 + threadIdx.x; id < u.line1; id += 256u) {
-        ScanTraversal s;
-        if (!path_scan_line(a, id, s)) continue;
-        const uint32_t step = s.down ? ~0u : 1u, stride = s.bz - s.bx, base = s.data_offset - u.tile0;
-        for (int32_t y = s.ymin; y < s.ymax; y++) {
-            const uint32_t t = base + (uint32_t)(y - (int32_t)s.by) * stride;
-            if (t < u.tiles) atomicAdd(&deltas[t], step);
-        }
-        float last_z = floorf(s.a * ((float)s.imin - 1.0f) + s.b);
-        for (uint32_t i = s.imin; i < s.imax; i++) {
-            const float z = floorf(s.a * (float)i + s.b);
-            int32_t tx, ty;
-            scan_tile(s, i, z, tx, ty);
-            if (scan_tile_inside(s, tx, ty)) {
-                const uint32_t offset = scan_tile_offset(s, tx, ty), t = offset - u.tile0;
-                if (t < u.tiles) {
-                    bool top = last_z == z;
-                    if (i == 0u) top = fabsf(s.y0 - s.py0 * (1.0f / 16.0f)) <= kScanEpsilon;
-                    // the tile to the right is of the same row, so of the same band
-                    if (top && tx + 1 < (int32_t)s.bz) atomicAdd(&deltas[t + 1u], step);
-                    atomicAdd(&counts[t], 1u);
-                } else if (offset < u.tile0) {
-                    ++before;
-                }
+    path_scan_lines(
+        a, u, paths, queues[wave],
+        [&](const ScanTraversal &s, const RunPath &, int32_t tx, int32_t ty) {
+            const uint32_t t = scan_tile_offset(s, tx, ty);
+            if (t < u.tiles) {
+                const bool top = fabsf((float)ty - s.py0 * (1.0f / 16.0f)) <= kScanEpsilon;
+                if (top && tx + 1 < (int32_t)s.bz) atomicAdd(&deltas[t + 1u], s.down ? ~0u : 1u);
+                atomicAdd(&slots[t], 1u);
+            } else if ((int32_t)t < 0) {
+                ++before;
             }
-            last_z = z;
-        }
-    }
+        },
+        [&](const ScanTraversal &s, const RunPath &) {
+            const uint32_t step = s.down ? ~0u : 1u, stride = s.bz - s.bx;
+            for (int32_t y = s.ymin; y < s.ymax; y++) {
+                const uint32_t t = s.data_offset + (uint32_t)(y - (int32_t)s.by) * stride;
+                if (t < u.tiles) atomicAdd(&deltas[t], step);
+            }
+            float last_z = floorf(s.a * ((float)s.imin - 1.0f) + s.b);
+            for (uint32_t i = s.imin; i < s.imax; i++) {
+                const float z = floorf(s.a * (float)i + s.b);
+                int32_t tx, ty;
+                scan_tile(s, i, z, tx, ty);
+                if (scan_tile_inside(s, tx, ty)) {
+                    const uint32_t t = scan_tile_offset(s, tx, ty);
+                    if (t < u.tiles) {
+                        bool top = last_z == z;
+                        if (i == 0u) top = fabsf(s.y0 - s.py0 * (1.0f / 16.0f)) <= kScanEpsilon;
+                        // the tile to the right is of the same row, so of the same band
+                        if (top && tx + 1 < (int32_t)s.bz) atomicAdd(&deltas[t + 1u], step);
+                        atomicAdd(&slots[t], 1u);
+                    } else if ((int32_t)t < 0) {
+                        ++before;
+                    }
+                }
+                last_z = z;
+            }
+        });
     if (u.band) {
         before = wave_sum_u32(before);
-        if (__lane_id() == 0u && before) atomicAdd(&s_before, before);
+        if (lane == 0u && before) atomicAdd(&s_before, before);
     }
     __syncthreads();
 
-    // One wave per path, its tiles in order, 64 at a time: the slots before each tile
-    // and the running sum of the deltas.
-    const uint32_t lane = threadIdx.x & 63u;
-    for (uint32_t p = u.first + uniform(threadIdx.x >> 6); p < u.end; p += 4u) {
-        const __attribute__((address_space(4))) tk_path_record &r = constant(a.paths)[p];
-        const uint32_t first = u.band ? u.tile0 : r.data_offset, n = u.band ? u.tiles : r.data_len;
-        const uint32_t o = first - u.tile0, stride = r.tile_x1 - r.tile_x0, start = r.segment_start;
-        uint32_t slot = start + (u.band ? s_before : 0u), sum = 0u;
-        for (uint32_t c = 0u; c < n; c += 64u) {
-            const uint32_t i = c + lane;
-            const uint32_t v = i < n ? counts[o + i] : 0u, d = i < n ? deltas[o + i] : 0u;
-            const uint32_t end = slot + wave_inclusive_scan_dpp(v), total = sum + wave_inclusive_scan_dpp(d);
-            if (i < n) {
-                a.counts[first + i] = v;
-                a.ranges[first + i] = tk_segment_range{end - v, end};
-                a.cursors[first + i] = end;  // as emission leaves it
-                if (a.raw_backdrops) a.raw_backdrops[first + i] = (int32_t)d;
-                counts[o + i] = end - v;
-                deltas[o + i] = total;
+    // Both tables' prefix sums over the whole run; what belongs to one path or row
+    // alone is a difference of two of them.
+    uint32_t slot_carry = 0u, delta_carry = 0u;
+    for (uint32_t base = 0u, buffer = 0u; base < u.tiles; base += 256u, buffer ^= 1u) {
+        const uint32_t t = base + tid;
+        const uint32_t v = t < u.tiles ? slots[t] : 0u, d = t < u.tiles ? deltas[t] : 0u;
+        const uint32_t vi = wave_inclusive_scan_dpp(v), di = wave_inclusive_scan_dpp(d);
+        if (lane == 63u) {
+            sums[buffer][0][wave] = vi;
+            sums[buffer][1][wave] = di;
+        }
+        __syncthreads();
+        uint32_t v_before = slot_carry, d_before = delta_carry;
+#pragma unroll
+        for (uint32_t w = 0; w < 4u; ++w) {
+            const uint32_t vs = sums[buffer][0][w], ds = sums[buffer][1][w];
+            if (w < wave) v_before += vs, d_before += ds;
+            slot_carry += vs;
+            delta_carry += ds;
+        }
+        if (t < u.tiles) {
+            slots[t] = v_before + vi - v;
+            deltas[t] = d_before + di;
+        }
+    }
+    if (tid == 0u) slots[u.tiles] = slot_carry;
+    __syncthreads();
+    if (tid < path_count) {
+        const uint32_t first = u.band ? 0u : slots[paths[tid].first], above = u.band ? s_before : 0u;
+        if (last_part) a.bumps[u.first + tid] = slots[path_end] - first + above;
+        paths[tid].offset += above - first;
+    }
+    __syncthreads();
+    for (uint32_t t = tid; t < u.tiles; t += 256u) {
+        uint32_t lo = 0u, hi = path_count;  // the last path whose first tile is at or before t
+        while (hi - lo > 1u) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (paths[mid].first <= t) lo = mid;
+            else hi = mid;
+        }
+        const RunPath p = paths[lo];
+        const uint32_t first = u.band ? 0u : p.first, stride = (p.high & (kPathLeftOut - 1u)) - (p.low & 0xFFFFu);
+        const uint32_t start = p.offset + slots[t], end = p.offset + slots[t + 1u];
+        // exact: below 2^12 over at most 2^10, half a step from the nearest whole number
+        const uint32_t row = first + (uint32_t)(((float)(t - first) + 0.5f) * (1.0f / (float)stride)) * stride;
+        const uint32_t tile = u.tile0 + t;
+        a.counts[tile] = end - start;
+        a.ranges[tile] = tk_segment_range{start, end};
+        a.cursors[tile] = end;  // as emission leaves it
+        if (a.raw_backdrops) a.raw_backdrops[tile] = (int32_t)(deltas[t] - (t ? deltas[t - 1u] : 0u));
+        a.backdrops[tile] = (int32_t)(deltas[t] - (row ? deltas[row - 1u] : 0u));
+    }
+    __syncthreads();
+
+    path_scan_lines(
+        a, u, paths, queues[wave],
+        [&](const ScanTraversal &s, const RunPath &path, int32_t tx, int32_t ty) {
+            const uint32_t t = scan_tile_offset(s, tx, ty);
+            if (t >= u.tiles) return;
+            const uint32_t slot = path.offset + atomicAdd(&slots[t], 1u);
+            if (slot < a.cfg.segment_capacity)
+                a.segments[slot] = tile_segment(s.px0, s.py0, s.px1, s.py1, (float)tx * kTileSize, (float)ty * kTileSize, s.down);
+        },
+        [&](const ScanTraversal &s, const RunPath &path) {
+            for (uint32_t i = s.imin; i < s.imax; i++) {
+                const float z = floorf(s.a * (float)i + s.b);
+                int32_t tx, ty;
+                scan_tile(s, i, z, tx, ty);
+                if (!scan_tile_inside(s, tx, ty)) continue;
+                const uint32_t t = scan_tile_offset(s, tx, ty);
+                if (t >= u.tiles) continue;
+                const uint32_t slot = path.offset + atomicAdd(&slots[t], 1u);
+                if (slot < a.cfg.segment_capacity) a.segments[slot] = clipped_segment(s, i, z, tx, ty);
             }
-            slot = (uint32_t)__builtin_amdgcn_readlane((int)end, 63);
-            sum = (uint32_t)__builtin_amdgcn_readlane((int)total, 63);
-        }
-        if (lane == 0u && first + n == r.data_offset + r.data_len) a.bumps[p] = slot - start;
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        // A tile's backdrop: the sum up to it less the sum before its row.
-        for (uint32_t i = lane; i < n; i += 64u) {
-            const uint32_t row = i - i % stride;
-            a.backdrops[first + i] = (int32_t)(deltas[o + i] - (row ? deltas[o + row - 1u] : 0u));
-        }
-    }
-    __syncthreads();
-
-    for (uint32_t id = u.line0 + threadIdx.x; id < u.line1; id += 256u) {
-        ScanTraversal s;
-        if (!path_scan_line(a, id, s)) continue;
-        for (uint32_t i = s.imin; i < s.imax; i++) {
-            const float z = floorf(s.a * (float)i + s.b);
-            int32_t tx, ty;
-            scan_tile(s, i, z, tx, ty);
-            if (!scan_tile_inside(s, tx, ty)) continue;
-            const uint32_t t = scan_tile_offset(s, tx, ty) - u.tile0;
-            if (t >= u.tiles) continue;
-            const uint32_t slot = atomicAdd(&counts[t], 1u);
-            if (slot < a.cfg.segment_capacity) a.segments[slot] = clipped_segment(s, i, z, tx, ty);
-        }
-    }
+        });
 }
 
 // Whether a scene is laid out as tk_k_path_scan takes it: lines and slabs path by
 // path without gaps, slabs as large as their tile boxes, scan chunks and cumsum rows
-// that cut every slab as the recorder does, and no path too long or too wide.
-// Anything else is left to the separate stages, whose result for it is the
+// that cut every slab as the recorder does, no path of more than TK_PATH_SCAN_LINES
+// lines and no box beyond the canvas or, where that is wider, beyond TK_PATH_SCAN_RUN.
+// (One path of 4096, 8192 and 16384 lines on 1024x1024, scan and coarse: 118, 142 and
+// 187 us here, 159, 167 and 188 us by the stages; eight such paths: 131, 156 and 202,
+// 208, 223 and 236.)  Anything else is left to the separate stages, whose result for it is the
 // reference's.  One thread per line, path, chunk and row.
 extern "C" __global__ __launch_bounds__(256) void tk_k_path_scan_check(tk_args_path_scan_check a) {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
@@ -211,7 +352,7 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_path_scan_check(tk_args_p
              p.line_count <= cfg.line_count - min(p.line_start, cfg.line_count) &&
              p.data_len <= cfg.backdrop_len - min(p.data_offset, cfg.backdrop_len) &&
              (!last || (p.line_start + p.line_count == cfg.line_count && p.data_offset + p.data_len == cfg.backdrop_len)) &&
-             p.tile_x0 <= p.tile_x1 && p.tile_y0 <= p.tile_y1 && p.tile_x1 - p.tile_x0 <= TK_PATH_SCAN_RUN &&
+             p.tile_x0 <= p.tile_x1 && p.tile_y0 <= p.tile_y1 && p.tile_x1 <= a.widest && p.tile_y1 <= 0xFFFFu &&
              (uint64_t)(p.tile_x1 - p.tile_x0) * (p.tile_y1 - p.tile_y0) == p.data_len &&
              p.line_count <= TK_PATH_SCAN_LINES;
         const tk_scan_chunk_range r = a.chunk_ranges[i];

@@ -74,20 +74,8 @@ TKD uint32_t scan_span(float a, float b) {
     return f2u(value);
 }
 
-TKD bool scan_geometry(const tk_line *lines, const tk_path_record *paths, uint32_t path_count,
-                       uint32_t line_index, ScanTraversal &s) {
-    s = ScanTraversal{};
-    const tk_line line = lines[line_index];
-    uint32_t path_id = line.path_id;
-    if (path_id >= path_count) return false;
-    const tk_path_record &path = paths[path_id];
-    s.bx = path.tile_x0;
-    s.by = path.tile_y0;
-    s.bz = path.tile_x1;
-    s.bw = path.tile_y1;
-    s.data_offset = path.data_offset;
-    if (s.bz - s.bx == 0u || s.by >= s.bw) return false;
-    const tk_affine t = path.transform;
+// The line's end points in device space, the upper one first.
+TKD void scan_endpoints(const tk_line &line, const tk_affine &t, ScanTraversal &s) {
     float p0x = t.a * line.p0[0] + t.c * line.p0[1] + t.e;
     float p0y = t.b * line.p0[0] + t.d * line.p0[1] + t.f;
     float p1x = t.a * line.p1[0] + t.c * line.p1[1] + t.e;
@@ -98,6 +86,10 @@ TKD bool scan_geometry(const tk_line *lines, const tk_path_record *paths, uint32
     } else {
         s.px0 = p1x; s.py0 = p1y; s.px1 = p0x; s.py1 = p0y;
     }
+}
+
+// The tiles a line with these end points visits; false when it visits none.
+TKD bool scan_traverse(ScanTraversal &s) {
     float sx = s.px0 * kTileScale, sy = s.py0 * kTileScale;
     float sz = s.px1 * kTileScale, sw = s.py1 * kTileScale;
     uint32_t count_x = scan_span(sx, sz) - 1u;
@@ -174,6 +166,43 @@ TKD bool scan_geometry(const tk_line *lines, const tk_path_record *paths, uint32
     return true;
 }
 
+TKD bool scan_geometry(const tk_line *lines, const tk_path_record *paths, uint32_t path_count,
+                       uint32_t line_index, ScanTraversal &s) {
+    s = ScanTraversal{};
+    const tk_line line = lines[line_index];
+    uint32_t path_id = line.path_id;
+    if (path_id >= path_count) return false;
+    const tk_path_record &path = paths[path_id];
+    s.bx = path.tile_x0;
+    s.by = path.tile_y0;
+    s.bz = path.tile_x1;
+    s.bw = path.tile_y1;
+    s.data_offset = path.data_offset;
+    if (s.bz - s.bx == 0u || s.by >= s.bw) return false;
+    scan_endpoints(line, path.transform, s);
+    return scan_traverse(s);
+}
+
+// What scan_traverse finds for a line within one tile of its box, without its
+// quotients: no tile, or the tile (tx, ty) alone, as visit 0 with z = 0.  The span of
+// both axes is one cell, so count is 1 and b, a fraction, has floor 0; no cut at the
+// box applies; and x0 is the cell for either slope (a falling line that starts on a
+// cell's left edge ends in the cell before it).  Lines so short that the general
+// code's reciprocal may overflow are left to it.
+enum ScanSingle : uint32_t { kScanNone, kScanOne, kScanGeneral };
+TKD ScanSingle scan_single_tile(const ScanTraversal &s, int32_t &tx, int32_t &ty) {
+    const float sx = s.px0 * kTileScale, sy = s.py0 * kTileScale;
+    const float sz = s.px1 * kTileScale, sw = s.py1 * kTileScale;
+    const float cx = floorf(sx), cy = floorf(sy);
+    const float dx = fabsf(sz - sx), dy = sw - sy;
+    tx = f2i(cx);
+    ty = f2i(cy);
+    const bool inside = tx >= (int32_t)s.bx && tx < (int32_t)s.bz && ty >= (int32_t)s.by && ty < (int32_t)s.bw;
+    if (!(cx == floorf(sz) && cy == floorf(sw) && inside && dx + dy >= 1.0e-30f)) return kScanGeneral;
+    if ((dy == 0.0f && cy == sy) || sw <= (float)s.by + kTopTouchEpsilon) return kScanNone;
+    return kScanOne;
+}
+
 TKD void scan_tile(const ScanTraversal &s, uint32_t index, float z, int32_t &tx, int32_t &ty) {
     tx = f2i(s.x0 + s.sign * z);
     ty = f2i(s.y0 + (float)index - z);
@@ -203,6 +232,50 @@ TKD float clip_y_at_x(const ScanTraversal &s, float x, float tmin, float tmax) {
         return tmin + kTileClipNudge;
     }
     return clampf(y, tmin + kTileClipNudge, tmax);
+}
+
+// The part (qx0, qy0) - (qx1, qy1) of a line, upper end first, in the coordinates of
+// the tile whose corner is (tminx, tminy).
+TKD tk_line_segment tile_segment(float qx0, float qy0, float qx1, float qy1, float tminx, float tminy, bool down) {
+    const float tile_size = kTileSize;
+    float edge = 1000000000.0f;
+    float p0x = clampf(qx0 - tminx, 0.0f, tile_size);
+    float p0y = clampf(qy0 - tminy, 0.0f, tile_size);
+    float p1x = clampf(qx1 - tminx, 0.0f, tile_size);
+    float p1y = clampf(qy1 - tminy, 0.0f, tile_size);
+    if (p0x <= kScanEpsilon) p0x = 0.0f; else if (tile_size - p0x <= kScanEpsilon) p0x = tile_size;
+    if (p0y <= kScanEpsilon) p0y = 0.0f; else if (tile_size - p0y <= kScanEpsilon) p0y = tile_size;
+    if (p1x <= kScanEpsilon) p1x = 0.0f; else if (tile_size - p1x <= kScanEpsilon) p1x = tile_size;
+    if (p1y <= kScanEpsilon) p1y = 0.0f; else if (tile_size - p1y <= kScanEpsilon) p1y = tile_size;
+    if (p0x == 0.0f) {
+        if (p1x == 0.0f) {
+            p0x = kScanEpsilon;
+            if (p0y == 0.0f) {
+                p1x = kScanEpsilon;
+                p1y = tile_size;
+            } else {
+                p1x = 2.0f * kScanEpsilon;
+                p1y = p0y;
+            }
+        } else if (p0y == 0.0f) {
+            p0x = kScanEpsilon;
+        } else {
+            edge = p0y;
+        }
+    } else if (p1x == 0.0f) {
+        if (p1y == 0.0f) p1x = kScanEpsilon;
+        else edge = p1y;
+    }
+    if (floorf(p0x) == p0x && p0x != 0.0f) p0x -= kScanEpsilon;
+    if (floorf(p1x) == p1x && p1x != 0.0f) p1x -= kScanEpsilon;
+    tk_line_segment out;
+    if (!down) {
+        out.p0x = p1x; out.p0y = p1y; out.p1x = p0x; out.p1y = p0y;
+    } else {
+        out.p0x = p0x; out.p0y = p0y; out.p1x = p1x; out.p1y = p1y;
+    }
+    out.y_edge = edge;
+    return out;
 }
 
 TKD tk_line_segment clipped_segment(const ScanTraversal &s, uint32_t sub_index, float z, int32_t tx, int32_t ty) {
@@ -236,44 +309,7 @@ TKD tk_line_segment clipped_segment(const ScanTraversal &s, uint32_t sub_index, 
             qy1 = clip_y_at_x(s, x_clip, tminy, tmaxy);
         }
     }
-    float edge = 1000000000.0f;
-    float p0x = clampf(qx0 - tminx, 0.0f, tile_size);
-    float p0y = clampf(qy0 - tminy, 0.0f, tile_size);
-    float p1x = clampf(qx1 - tminx, 0.0f, tile_size);
-    float p1y = clampf(qy1 - tminy, 0.0f, tile_size);
-    if (p0x <= kScanEpsilon) p0x = 0.0f; else if (tile_size - p0x <= kScanEpsilon) p0x = tile_size;
-    if (p0y <= kScanEpsilon) p0y = 0.0f; else if (tile_size - p0y <= kScanEpsilon) p0y = tile_size;
-    if (p1x <= kScanEpsilon) p1x = 0.0f; else if (tile_size - p1x <= kScanEpsilon) p1x = tile_size;
-    if (p1y <= kScanEpsilon) p1y = 0.0f; else if (tile_size - p1y <= kScanEpsilon) p1y = tile_size;
-    if (p0x == 0.0f) {
-        if (p1x == 0.0f) {
-            p0x = kScanEpsilon;
-            if (p0y == 0.0f) {
-                p1x = kScanEpsilon;
-                p1y = tile_size;
-            } else {
-                p1x = 2.0f * kScanEpsilon;
-                p1y = p0y;
-            }
-        } else if (p0y == 0.0f) {
-            p0x = kScanEpsilon;
-        } else {
-            edge = p0y;
-        }
-    } else if (p1x == 0.0f) {
-        if (p1y == 0.0f) p1x = kScanEpsilon;
-        else edge = p1y;
-    }
-    if (floorf(p0x) == p0x && p0x != 0.0f) p0x -= kScanEpsilon;
-    if (floorf(p1x) == p1x && p1x != 0.0f) p1x -= kScanEpsilon;
-    tk_line_segment out;
-    if (!s.down) {
-        out.p0x = p1x; out.p0y = p1y; out.p1x = p0x; out.p1y = p0y;
-    } else {
-        out.p0x = p0x; out.p0y = p0y; out.p1x = p1x; out.p1y = p1y;
-    }
-    out.y_edge = edge;
-    return out;
+    return tile_segment(qx0, qy0, qx1, qy1, tminx, tminy, s.down);
 }
 
 // ---------------------------------------------------------------------------

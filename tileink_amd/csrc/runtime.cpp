@@ -571,9 +571,27 @@ tk_scan_config frame_scan_config(const tk_scene &s) {
     return c;
 }
 
-// Runs of tk_k_path_scan.
-uint32_t path_scan_runs(const tk_scene &s) {
-    return uint32_t((uint64_t(s.line_count) + s.backdrop_len) / TK_PATH_SCAN_RUN) + 1u;
+// The widest tile grid of the frame's canvases.
+uint32_t frame_tiles_width(const tk_frame *f) {
+    uint32_t widest = 0;
+    for (const tk_fe_scene &scene : f->fe_scenes_host) widest = std::max(widest, scene.tiles_width);
+    return widest;
+}
+
+// Positions of tk_k_path_scan.
+uint64_t path_scan_positions(const tk_scene &s) {
+    return uint64_t(s.line_count) + s.backdrop_len + 4ull * s.path_count;
+}
+// How many make a run: in a large frame 640, which balances what a run costs to set up
+// against the LDS it holds (50,000 paths, 13.9 M positions: runs of 256, 384, 512, 640
+// and 912 take 442, 374, 344, 324 and 330 us); in a smaller one fewer, so that about
+// as many workgroups run as are resident at once (an icon: 14 us, in runs of 960 26 us).
+// A run is never shorter than the widest canvas, whose rows its tables must hold.
+constexpr uint32_t kPathScanRun = 640;
+uint32_t path_scan_run(const tk_frame *f) {
+    const uint64_t even = path_scan_positions(f->meta) / (6u * f->ctx->compute_units);
+    const uint64_t run = std::max<uint64_t>({std::min<uint64_t>(even, kPathScanRun), 128u, frame_tiles_width(f)});
+    return uint32_t(std::min<uint64_t>(run, TK_PATH_SCAN_RUN));
 }
 
 // Whether tk_k_path_scan takes the scene whose records are in the frame's buffers:
@@ -591,6 +609,7 @@ tk_status path_scan_check(tk_frame *f, const tk_scene &s) {
     a.row_ends = f->cs_row_ends;
     a.row_count = s.cumsum_row_count;
     a.cs_chunk_count = s.cumsum_chunk_count;
+    a.widest = std::min<uint32_t>(frame_tiles_width(f), TK_PATH_SCAN_RUN);
     *f->ctx->refused = 0u;
     TK_HIP(hipHostGetDevicePointer(reinterpret_cast<void **>(&a.refused), f->ctx->refused, 0));
     const uint32_t threads = std::max({1u, s.path_count, s.line_count, s.scan_chunk_count, s.cumsum_row_count});
@@ -875,6 +894,7 @@ tk_status frame_render(tk_frame *f, uint32_t active_count = 0, const DiffTarget 
         a.lines = f->lines;
         a.paths = f->paths;
         a.path_count = s.path_count;
+        a.run = path_scan_run(f);
         a.path_active = path_active;
         a.counts = f->seg_counts;
         a.ranges = f->seg_ranges;
@@ -886,7 +906,8 @@ tk_status frame_render(tk_frame *f, uint32_t active_count = 0, const DiffTarget 
         a.clear[0] = {f->status, 4};
         a.clear[1] = {reinterpret_cast<uint32_t *>(f->coarse_status), status_words};
         a.clear[2] = {f->queues, f->tuning.persistent ? kQueueWords : 0};
-        TK_TRY(launch(ctx, ctx->f_path_scan, path_scan_runs(s), 1, 256, a));
+        TK_TRY(launch(ctx, ctx->f_path_scan, uint32_t(path_scan_positions(s) / a.run) + 1u, 1, 256, a,
+                      TK_PATH_SCAN_LDS(a.run)));
         for (int mark : {2, 3, 4, 5, 6}) TK_TRY(record(f, mark));
         TK_TRY(coarse());
     } else {
@@ -1583,9 +1604,9 @@ tk_status frame_set_geometry(tk_frame *f, const FeInput &in) {
     f->diff_ready = false;
     // The front end lays paths out as the one-kernel scan takes them, unless one is too
     // long (status bit 2) or too wide for it.
-    uint32_t widest = 0;
-    for (const tk_fe_scene &scene : f->fe_scenes_host) widest = std::max(widest, scene.tiles_width);
-    f->path_scan = !(flags & 4u) && widest <= TK_PATH_SCAN_RUN;
+    uint32_t highest = 0;
+    for (const tk_fe_scene &scene : f->fe_scenes_host) highest = std::max(highest, scene.tiles_height);
+    f->path_scan = !(flags & 4u) && frame_tiles_width(f) <= TK_PATH_SCAN_RUN && highest <= 0xFFFFu;
     return TK_OK;
 }
 

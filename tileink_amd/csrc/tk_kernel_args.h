@@ -108,13 +108,15 @@ struct tk_args_scan_prefix {
 };
 
 // The scan of a frame laid out path by path, in one kernel (pathscan.hip).
-#define TK_PATH_SCAN_RUN 1024u     // lines and tiles per run
-#define TK_PATH_SCAN_LINES 4096u   // lines of a path that one workgroup still scans
+#define TK_PATH_SCAN_RUN 928u      // lines, tiles and paths (four each) per run, at most
+#define TK_PATH_SCAN_LDS(run) (16u * (((run) + 3u) / 4u) + 24u * (run) + 4u)  // bytes of LDS for a run's tables
+#define TK_PATH_SCAN_LINES 8192u   // lines of the longest path it takes
 struct tk_args_path_scan {
     tk_scan_config cfg;
     const tk_line *lines;
     const tk_path_record *paths;
     uint32_t path_count;
+    uint32_t run;                 // lines, tiles and paths (four each) per run: the widest tile box at least
     const uint32_t *path_active;  // incremental: as tk_args_scan_lines
     uint32_t *counts;
     tk_segment_range *ranges;
@@ -137,6 +139,7 @@ struct tk_args_path_scan_check {
     const tk_scan_chunk_range *chunk_ranges;
     const uint32_t *cs_offsets, *cs_lens, *row_starts, *row_ends;
     uint32_t row_count, cs_chunk_count;
+    uint32_t widest;              // tiles of the widest canvas, TK_PATH_SCAN_RUN at most
     uint32_t *refused;            // set to 1 when tk_k_path_scan does not take the scene
 };
 
