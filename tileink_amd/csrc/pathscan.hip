@@ -187,6 +187,10 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_path_scan(tk_args_path_sc
     for (uint32_t k = 0; k < 3u; ++k)  // words that later kernels of the frame start from zero
         for (uint64_t i = blockIdx.x * 256ull + tid; i < a.clear[k].count; i += gridDim.x * 256ull)
             a.clear[k].words[i] = 0u;
+    if (blockIdx.x >= a.runs) {  // the workgroups behind the runs build the draw tables, a launch less
+        draw_tables(a.tables, (blockIdx.x - a.runs) * 256u + tid);
+        return;
+    }
     PathRun u;
     if (!path_run(a, blockIdx.x, u)) return;
     const uint32_t path_count = u.end - u.first;  // at most RUN / 4

@@ -85,6 +85,7 @@ struct tk_context {
                   f_fine_diff_keep[4] = {}, f_fine_backward_keep[4] = {},
                   f_fill_coverage = nullptr, f_pixel_math = nullptr, f_brush_words = nullptr;
     // Persistent forms (work queues) and the coarse scan's other block sizes.
+    hipFunction_t f_coarse_count_stage = nullptr, f_coarse_emit_stage = nullptr;
     hipFunction_t f_fine_persistent = nullptr, f_fine_scenes_persistent = nullptr,
                   f_coarse_count_persistent = nullptr, f_coarse_count_scenes_persistent = nullptr,
                   f_coarse_emit_persistent = nullptr, f_coarse_emit_scenes_persistent = nullptr,
@@ -281,6 +282,7 @@ struct LayerClassPlan {
     const uint32_t *pair_layer = nullptr, *pair_of = nullptr;
     uint32_t pair_count = 0;
     uint8_t *bits = nullptr;
+    const uint4 *batch_pairs = nullptr;
 };
 
 tk_status run_coarse(tk_context *ctx, const tk_coarse_config &cfg, const tk_coarse_inputs &in,
@@ -293,7 +295,7 @@ tk_status run_coarse(tk_context *ctx, const tk_coarse_config &cfg, const tk_coar
     if (cfg.batch_count == 0 || list.columns == 0) return TK_OK;
     const uint32_t blocks = scenes.slots ? coarse_scan_blocks_for(scenes.table_entries, shape.scan_items)
                                          : coarse_scan_blocks(cfg, list.columns, shape.scan_items);
-    tk_args_coarse a{cfg, in, out, status, ticket, epoch, blocks, tk_layer_classes{nullptr, nullptr, 0u}, list, scenes,
+    tk_args_coarse a{cfg, in, out, status, ticket, epoch, blocks, tk_layer_classes{nullptr, nullptr, 0u, nullptr}, list, scenes,
                      shape.xcd_run, shape.queue, draw_entries};
     if (plan.bits && plan.pair_count) {
         tk_args_layer_classes b{cfg, in, plan.pair_layer, plan.pair_count, plan.bits, list};
@@ -301,7 +303,7 @@ tk_status run_coarse(tk_context *ctx, const tk_coarse_config &cfg, const tk_coar
         // 64 MiB, so the grid fits 32 bits)
         TK_TRY(launch(ctx, ctx->f_layer_classes, uint32_t(div_up(list.columns, 256) * uint64_t(plan.pair_count)), 1,
                       256, b));
-        a.classes = tk_layer_classes{plan.bits, plan.pair_of, plan.pair_count};
+        a.classes = tk_layer_classes{plan.bits, plan.pair_of, plan.pair_count, plan.batch_pairs};
     }
     const uint32_t block = 64u * shape.coarse_block;
     hipFunction_t count_fn, emit_fn;
@@ -313,8 +315,9 @@ tk_status run_coarse(tk_context *ctx, const tk_coarse_config &cfg, const tk_coar
         TK_TRY(resident_grid(ctx, count_fn, block, 0u, groups, &count_grid));
         TK_TRY(resident_grid(ctx, emit_fn, block, 0u, groups, &emit_grid));
     } else {
-        count_fn = scenes.slots ? ctx->f_coarse_count_scenes : ctx->f_coarse_count;
-        emit_fn = scenes.slots ? ctx->f_coarse_emit_scenes : ctx->f_coarse_emit;
+        // the stage entry points have no frame's tables
+        count_fn = scenes.slots ? ctx->f_coarse_count_scenes : draw_entries ? ctx->f_coarse_count : ctx->f_coarse_count_stage;
+        emit_fn = scenes.slots ? ctx->f_coarse_emit_scenes : draw_entries ? ctx->f_coarse_emit : ctx->f_coarse_emit_stage;
         count_grid = emit_grid = xcd_grid(div_up(list.columns, shape.coarse_block), shape.xcd_run);
     }
     hipFunction_t scan_fn = shape.scan_items == 1024u   ? ctx->f_coarse_scan_1k
@@ -404,7 +407,9 @@ struct tk_frame {
     uint32_t *layer_pair_of = nullptr, *pair_layer = nullptr;
     uint8_t *layer_bits = nullptr;
     uint32_t pair_capacity = 0, pair_count = 0;
+    uint4 *batch_pairs = nullptr;
     std::vector<uint32_t> host_pair_of, host_pair_layer;
+    std::vector<uint4> host_batch_pairs;
     // incremental renders: the listed tiles, the damage summed-area table, per-path flags
     uint32_t *active_tiles = nullptr, *damage_sat = nullptr, *path_active = nullptr;
     std::vector<uint32_t> host_active, host_sat;
@@ -560,6 +565,31 @@ uint64_t atlas_words(const tk_scene &s) {
     return s.atlas ? uint64_t(s.atlas_width) * s.atlas_height * s.atlas_pages : 0ull;
 }
 
+// tk_layer_classes::batch_pairs of the scene's batches, whose layers' pairs are in
+// host_pair_of.
+void batch_pairs(const tk_frame &f, const tk_scene &s, std::vector<uint4> &out) {
+    const std::vector<uint32_t> &scene_of = f.fe_scene_of_batch_host;
+    const auto scene = [&](uint32_t b) { return b < scene_of.size() ? scene_of[b] : 0u; };
+    const auto layers = [&](uint32_t b, auto body) {
+        for (uint32_t i = s.batches[b].layer_start; i < std::min(s.batches[b].layer_end, s.layer_count); ++i)
+            body(f.host_pair_of[i]);
+    };
+    std::vector<uint32_t> first(std::max<size_t>(f.scene_count, 1), 0xFFFFFFFFu), last(first.size(), 0u);
+    for (uint32_t b = 0; b < s.batch_count; ++b)
+        layers(b, [&](uint32_t pair) {
+            first[scene(b)] = std::min(first[scene(b)], pair);
+            last[scene(b)] = std::max(last[scene(b)], pair);
+        });
+    out.assign(s.batch_count, uint4{0u, 0u, 0u, 0u});
+    for (uint32_t b = 0; b < s.batch_count; ++b) {
+        const uint32_t base = first[scene(b)] == 0xFFFFFFFFu ? 0u : first[scene(b)];
+        if (last[scene(b)] - base >= 64u && last[scene(b)] >= base) continue;
+        uint64_t pairs = 0;
+        layers(b, [&](uint32_t pair) { pairs |= 1ull << (pair - base); });
+        out[b] = uint4{uint32_t(pairs), uint32_t(pairs >> 32), base, 1u};
+    }
+}
+
 tk_scan_config frame_scan_config(const tk_scene &s) {
     tk_scan_config c{};
     c.clear_len = std::max({s.backdrop_len, s.path_count, s.scan_chunk_count});
@@ -643,6 +673,8 @@ tk_status frame_upload(tk_frame *f, const tk_scene *s) {
         if (pairs <= f->pair_capacity) {  // else: no table for this scene
             TK_TRY(upload(f, f->layer_pair_of, f->host_pair_of.data(), s->layer_count));
             TK_TRY(upload(f, f->pair_layer, f->host_pair_layer.data(), pairs));
+            batch_pairs(*f, *s, f->host_batch_pairs);
+            TK_TRY(upload(f, f->batch_pairs, f->host_batch_pairs.data(), s->batch_count));
             f->pair_count = pairs;
         }
     }
@@ -841,9 +873,9 @@ tk_status frame_render(tk_frame *f, uint32_t active_count = 0, const DiffTarget 
         // The persistent launches' work counters (coarse count, coarse emit, fine) start at zero.
         if (f->tuning.persistent) TK_TRY(fill_u32(ctx, f->queues, kQueueWords, 0u));
     }
-    TK_TRY(run_draw_tables(ctx, tk_args_draw_tables{f->draws, s.draw_count, f->paint, s.paint_words, s.paint_brush_base,
-                                                    diff ? nullptr : f->draw_brush, f->draw_entries, f->paths,
-                                                    s.path_count, f->batch_ids}));
+    const tk_args_draw_tables tables{f->draws, s.draw_count, f->paint, s.paint_words, s.paint_brush_base,
+                                     diff ? nullptr : f->draw_brush, f->draw_entries, f->paths, s.path_count, f->batch_ids};
+    if (!f->path_scan) TK_TRY(run_draw_tables(ctx, tables));
     if (active_count && s.path_count) {
         tk_args_active_paths ap{f->paths, s.path_count, s.tiles_width, s.tiles_height, f->damage_sat, f->path_active};
         TK_TRY(launch(ctx, ctx->f_active_paths, div_up(s.path_count, 256), 1, 256, ap));
@@ -878,6 +910,7 @@ tk_status frame_render(tk_frame *f, uint32_t active_count = 0, const DiffTarget 
             plan.pair_of = f->layer_pair_of;
             plan.pair_count = f->pair_count;
             plan.bits = f->layer_bits;
+            plan.batch_pairs = f->batch_pairs;
         }
         TK_TRY(run_coarse(ctx, cc, in, out, f->coarse_status, &f->tickets[1], f->epoch, f->timing ? &f->ev[7] : nullptr,
                           plan, list, scenes, coarse_launch(f), f->draw_entries));
@@ -906,8 +939,9 @@ tk_status frame_render(tk_frame *f, uint32_t active_count = 0, const DiffTarget 
         a.clear[0] = {f->status, 4};
         a.clear[1] = {reinterpret_cast<uint32_t *>(f->coarse_status), status_words};
         a.clear[2] = {f->queues, f->tuning.persistent ? kQueueWords : 0};
-        TK_TRY(launch(ctx, ctx->f_path_scan, uint32_t(path_scan_positions(s) / a.run) + 1u, 1, 256, a,
-                      TK_PATH_SCAN_LDS(a.run)));
+        a.runs = uint32_t(path_scan_positions(s) / a.run) + 1u;
+        a.tables = tables;
+        TK_TRY(launch(ctx, ctx->f_path_scan, a.runs + div_up(s.draw_count, 256), 1, 256, a, TK_PATH_SCAN_LDS(a.run)));
         for (int mark : {2, 3, 4, 5, 6}) TK_TRY(record(f, mark));
         TK_TRY(coarse());
     } else {
@@ -1093,6 +1127,7 @@ tk_status frame_create(tk_context *ctx, const tk_scene *s, const BatchLayout *ba
         if (pairs * T <= kMaxLayerClassBytes) {
             ALLOC(layer_pair_of, s->layer_count);
             ALLOC(pair_layer, pairs);
+            ALLOC(batch_pairs, s->batch_count);
             ALLOC(layer_bits, pairs * T);
             f->pair_capacity = uint32_t(pairs);
         }
@@ -1203,6 +1238,8 @@ tk_status tk_context_create(int device, tk_context **out) {
         {&ctx->f_path_scan_check, "tk_k_path_scan_check"},
         {&ctx->f_coarse_count, "tk_k_coarse_count"},
         {&ctx->f_coarse_scan, "tk_k_coarse_scan"},
+        {&ctx->f_coarse_count_stage, "tk_k_coarse_count_stage"},
+        {&ctx->f_coarse_emit_stage, "tk_k_coarse_emit_stage"},
         {&ctx->f_coarse_emit, "tk_k_coarse_emit"},
         {&ctx->f_layer_classes, "tk_k_layer_classes"},
         {&ctx->f_active_paths, "tk_k_active_paths"},

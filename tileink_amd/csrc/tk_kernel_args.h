@@ -107,6 +107,37 @@ struct tk_args_scan_prefix {
     uint32_t wave_count;  // pass A: max(chunks, ceil(paths / 64)) waves
 };
 
+// Per-draw words for fine and coarse, built from the records in front of a frame.
+// Brush (fine), eight per draw: {1, colour, 0, 0, the colour's four bytes as floats}
+// when the draw's brush colour does not depend on the pixel, zeros when it must be
+// sampled.  Entry (coarse), eight per draw: the tile box {x0, y0, x1, y1} in which the
+// draw may cover tiles, then {base, stride, batch, kind | fill rule << 8}: the
+// backdrop tile of (x, y) is base + y * stride + x, modulo 2^32.
+#define TK_DRAW_BRUSH_WORDS 8u
+#define TK_DRAW_ENTRY_WORDS 8u
+enum tk_draw_entry_kind : uint32_t {
+    TK_ENTRY_NONE = 0,       // never a particle
+    TK_ENTRY_FILL = 1,       // a brush over its path
+    TK_ENTRY_GLYPH = 2,
+    TK_ENTRY_CLIP = 3,
+    TK_ENTRY_SDF = 4,        // by its record
+    TK_ENTRY_KIND = 7,
+    TK_ENTRY_SOLID_RECT = 8, // with FILL: a COLOR particle on tiles without segments
+    TK_ENTRY_RECORD_RULE = 16, // a fill rule too large for the entry
+    TK_ENTRY_RULE_SHIFT = 8,
+};
+struct tk_args_draw_tables {
+    const tk_draw_record *draws;
+    uint32_t draw_count;
+    const uint32_t *paint;
+    uint32_t paint_words, paint_brush_base;
+    uint32_t *brushes;                // null: not wanted
+    uint4 *entries;                   // null: not wanted
+    const tk_path_record *paths;      // the rest for entries only
+    uint32_t path_count;
+    const uint32_t *batch_ids;
+};
+
 // The scan of a frame laid out path by path, in one kernel (pathscan.hip).
 #define TK_PATH_SCAN_RUN 928u      // lines, tiles and paths (four each) per run, at most
 #define TK_PATH_SCAN_LDS(run) (16u * (((run) + 3u) / 4u) + 24u * (run) + 4u)  // bytes of LDS for a run's tables
@@ -116,6 +147,7 @@ struct tk_args_path_scan {
     const tk_line *lines;
     const tk_path_record *paths;
     uint32_t path_count;
+    uint32_t runs;
     uint32_t run;                 // lines, tiles and paths (four each) per run: the widest tile box at least
     const uint32_t *path_active;  // incremental: as tk_args_scan_lines
     uint32_t *counts;
@@ -129,6 +161,7 @@ struct tk_args_path_scan {
         uint32_t *words;
         uint64_t count;
     } clear[3];                   // words to clear on the way
+    tk_args_draw_tables tables;   // built by the workgroups after the runs
 };
 
 struct tk_args_path_scan_check {
@@ -162,6 +195,9 @@ struct tk_layer_classes {
     const uint8_t *bits;        // columns * pair_count (one row of pair_count bytes per table column)
     const uint32_t *pair_of;    // per layer record: its pair
     uint32_t pair_count;
+    // Per batch {pairs of its layers, low and high word, less base; base, the first pair
+    // of its scene; 1, or 0 when the scene has more than 64}.
+    const uint4 *batch_pairs;
 };
 
 struct tk_args_coarse {
@@ -178,7 +214,7 @@ struct tk_args_coarse {
     uint32_t xcd_run;  // XCD run length in four-tile workgroups (a power of two; 0: launch order)
     uint32_t *queue;   // 16 per-XCD work counters (count, emit), zero at launch: persistent count and emit
                        // launches, each wave taking tiles; null: one four-tile workgroup per launch item
-    const uint4 *draw_entries;  // tk_args_draw_tables::entries; null: the draw and path records are read
+    const uint4 *draw_entries;  // tk_args_draw_tables::entries (a frame's kernels only)
 };
 
 struct tk_args_layer_classes {
@@ -188,35 +224,6 @@ struct tk_args_layer_classes {
     uint32_t pair_count;
     uint8_t *bits;               // columns * pair_count, column-major
     tk_tile_list list;
-};
-
-// Per-draw words for fine and coarse, built from the records in front of a frame.
-// Brush (fine), eight per draw: {1, colour, 0, 0, the colour's four bytes as floats}
-// when the draw's brush colour does not depend on the pixel, zeros when it must be
-// sampled.  Entry (coarse), eight per draw: the tile box {x0, y0, x1, y1} in which the
-// draw may cover tiles, then {base, stride, batch, kind | fill rule << 8}: the
-// backdrop tile of (x, y) is base + y * stride + x, modulo 2^32.
-#define TK_DRAW_BRUSH_WORDS 8u
-#define TK_DRAW_ENTRY_WORDS 8u
-enum tk_draw_entry_kind : uint32_t {
-    TK_ENTRY_NONE = 0,       // never a particle
-    TK_ENTRY_FILL = 1,       // a brush over its path
-    TK_ENTRY_GLYPH = 2,
-    TK_ENTRY_CLIP = 3,
-    TK_ENTRY_RECORD = 4,     // by its record: SDF draws
-    TK_ENTRY_KIND = 7,
-    TK_ENTRY_SOLID_RECT = 8, // with FILL: a COLOR particle on tiles without segments
-};
-struct tk_args_draw_tables {
-    const tk_draw_record *draws;
-    uint32_t draw_count;
-    const uint32_t *paint;
-    uint32_t paint_words, paint_brush_base;
-    uint32_t *brushes;                // null: not wanted
-    uint4 *entries;                   // null: not wanted
-    const tk_path_record *paths;      // the rest for entries only
-    uint32_t path_count;
-    const uint32_t *batch_ids;
 };
 
 struct tk_args_fine {
