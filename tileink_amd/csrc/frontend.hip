@@ -202,11 +202,21 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_fe_batch_clips(tk_args_fr
 
 // Phase 1, one thread per draw of a batch: its tile box, its share of the PTCL
 // bound, its rows, and the visible runs of each row (the box minus its cover).
+// Bound by atomics on few words (a scene's draws meet in its batches and tile rows),
+// so a wave adds up each batch's areas first and a workgroup its rows' entries, in LDS
+// for frames of up to kFeRows rows: 6000 draws over 45 rows 84 -> 9 us.
+constexpr uint32_t kFeRows = 4096u;
 extern "C" __global__ __launch_bounds__(256) void tk_k_fe_draw_count(tk_args_frontend a) {
+    __shared__ uint32_t s_rows[kFeRows];
+    const bool local = a.row_count <= kFeRows;
+    if (local) {
+        for (uint32_t r = threadIdx.x; r < a.row_count; r += 256u) s_rows[r] = 0u;
+        __syncthreads();
+    }
     const uint32_t d = blockIdx.x * 256u + threadIdx.x;
-    if (d >= a.draw_count) return;
-    const uint32_t b = a.batch_ids[d];
+    const uint32_t b = d < a.draw_count ? a.batch_ids[d] : kNone;
     uint32_t tb[4] = {0u, 0u, 0u, 0u};
+    unsigned long long area = 0ull;
     if (b < a.batch_count) {
         const tk_fe_scene sc = a.scenes[fe_scene_of(a.scene_of_draw, d)];
         const tk_pixel_bounds pb = a.draws[d].pixel_bounds;
@@ -215,15 +225,15 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_fe_draw_count(tk_args_fro
             const uint32_t *clip = a.batch_clip + 4u * b;
             const uint32_t cx0 = max(tb[0], clip[0]), cy0 = max(tb[1], clip[1]);
             const uint32_t cx1 = min(tb[2], clip[2]), cy1 = min(tb[3], clip[3]);
-            if (cx1 > cx0 && cy1 > cy0)
-                atomicAdd(&a.batch_area[b], (unsigned long long)(cx1 - cx0) * (unsigned long long)(cy1 - cy0));
+            if (cx1 > cx0 && cy1 > cy0) area = (unsigned long long)(cx1 - cx0) * (unsigned long long)(cy1 - cy0);
             const uint32_t *cv = a.covers + 4u * d;
             const uint32_t hx0 = max(tb[0], cv[0]), hy0 = max(tb[1], cv[1]);
             const uint32_t hx1 = min(tb[2], cv[2]), hy1 = min(tb[3], cv[3]);
             const bool hides = hx1 > hx0 && hy1 > hy0;
             const uint64_t base = (uint64_t)sc.column_start + sc.row_start;
             for (uint32_t y = tb[1]; y < tb[3]; ++y) {
-                atomicAdd(&a.row_counts[sc.row_start + y], 1u);
+                if (local) atomicAdd(&s_rows[sc.row_start + y], 1u);
+                else atomicAdd(&a.row_counts[sc.row_start + y], 1u);
                 int32_t *row = a.diff + base + (uint64_t)y * (sc.tiles_width + 1u);
                 if (hides && y >= hy0 && y < hy1) {
                     if (hx0 > tb[0]) {
@@ -243,7 +253,19 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_fe_draw_count(tk_args_fro
             tb[0] = tb[1] = tb[2] = tb[3] = 0u;
         }
     }
-    for (int k = 0; k < 4; ++k) a.draw_box[4u * d + k] = tb[k];
+    for (uint64_t pending = __ballot(area != 0ull); pending;) {
+        const uint32_t first = (uint32_t)__builtin_ctzll(pending);
+        const uint32_t bb = (uint32_t)__builtin_amdgcn_readlane((int)b, (int)first);
+        const unsigned long long sum = fe_wave_sum_u64(b == bb ? area : 0ull);
+        if ((threadIdx.x & 63u) == first) atomicAdd(&a.batch_area[bb], sum);
+        pending &= ~__ballot(b == bb);
+    }
+    if (d < a.draw_count)
+        for (int k = 0; k < 4; ++k) a.draw_box[4u * d + k] = tb[k];
+    if (!local) return;
+    __syncthreads();
+    for (uint32_t r = threadIdx.x; r < a.row_count; r += 256u)
+        if (s_rows[r]) atomicAdd(&a.row_counts[r], s_rows[r]);
 }
 
 // Phase 1, one thread per batch: per batch, its particles plus (2 depth + 1)
@@ -261,18 +283,64 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_fe_batch_caps(tk_args_fro
     atomicAdd(&a.totals[TK_FE_PTCL], area + (2ull * depth + 1ull) * (clip_area < area ? clip_area : area));
 }
 
-// Phase 1, one thread per tile row: the row's tile list lengths from its runs.
+// Phase 1, one wave per tile row: the row's tile list lengths from its runs.  (One
+// thread per row, a chain of loads: 80 tiles a row 21 us; a wave: 3.5.)
 extern "C" __global__ __launch_bounds__(256) void tk_k_fe_tile_counts(tk_args_frontend a) {
-    const uint32_t r = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t r = blockIdx.x * 4u + uniform(threadIdx.x >> 6), lane = threadIdx.x & 63u;
     if (r >= a.row_count) return;
     const tk_fe_scene sc = a.scenes[fe_scene_of(a.scene_of_row, r)];
     const uint32_t y = r - sc.row_start;
     const int32_t *row = a.diff + (uint64_t)sc.column_start + sc.row_start + (uint64_t)y * (sc.tiles_width + 1u);
     uint32_t *counts = a.tile_counts + sc.column_start + (uint64_t)y * sc.tiles_width;
-    int32_t run = 0;
-    for (uint32_t x = 0; x < sc.tiles_width; ++x) {
-        run += row[x];
-        counts[x] = (uint32_t)run;
+    uint32_t run = 0u;
+    for (uint32_t base = 0; base < sc.tiles_width; base += 64u) {
+        const uint32_t x = base + lane;
+        const uint32_t upto = run + wave_inclusive_scan_dpp(x < sc.tiles_width ? (uint32_t)row[x] : 0u);
+        if (x < sc.tiles_width) counts[x] = upto;
+        run = (uint32_t)__builtin_amdgcn_readlane((int)upto, 63);
+    }
+}
+
+// In-place exclusive scans of short columns, one workgroup each: a launch where the
+// three kernels below take three per table.
+extern "C" __global__ __launch_bounds__(256) void tk_k_fe_scan_short(tk_args_fe_scan_short a) {
+    __shared__ unsigned long long s_wave[2][4];
+    uint32_t *v = a.columns[blockIdx.x].values;
+    const uint32_t count = a.columns[blockIdx.x].count, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    unsigned long long carry = 0ull;
+    for (uint32_t base = 0u, buffer = 0u; base < count; base += 2048u, buffer ^= 1u) {
+        const uint32_t first = base + threadIdx.x * 8u;
+        uint32_t x[8];
+        unsigned long long sum = 0ull;
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; ++k) {
+            x[k] = first + k < count ? v[first + k] : 0u;
+            sum += x[k];
+        }
+        unsigned long long upto = sum;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const unsigned long long y = (unsigned long long)__shfl_up((long long)upto, off, 64);
+            if (lane >= (uint32_t)off) upto += y;
+        }
+        if (lane == 63u) s_wave[buffer][wave] = upto;
+        __syncthreads();
+        unsigned long long before = carry;
+#pragma unroll
+        for (uint32_t w = 0; w < 4u; ++w) {
+            if (w < wave) before += s_wave[buffer][w];
+            carry += s_wave[buffer][w];
+        }
+        uint32_t run = (uint32_t)(before + upto - sum);
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; ++k) {
+            if (first + k < count) v[first + k] = run;
+            run += x[k];
+        }
+    }
+    if (threadIdx.x == 0u) {
+        *a.columns[blockIdx.x].total = carry;
+        if (carry > 0xFFFFFFFFull) atomicOr(a.overflow, 1u);
     }
 }
 
@@ -447,36 +515,48 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_fe_rows(tk_args_frontend 
     }
 }
 
-// Phase 2, one workgroup per tile row, one lane per tile: each lane walks the
-// row's draws in order and appends those visible in its tile to its list.
+// Phase 2, one wave per tile: the row's draws in order, 64 at a time; those visible in
+// the tile are appended to its list.  (A lane per tile and a workgroup per row
+// walked the row's draws one by one: 45 rows of 80 tiles and some 500 draws 139 us;
+// a wave per tile 6.4.)
 extern "C" __global__ __launch_bounds__(256) void tk_k_fe_tiles(tk_args_frontend a) {
-    const uint32_t r = blockIdx.x;
+    const uint32_t r = blockIdx.x, x = blockIdx.y * 4u + uniform(threadIdx.x >> 6), lane = threadIdx.x & 63u;
     if (r >= a.row_count) return;
     const tk_fe_scene sc = a.scenes[fe_scene_of(a.scene_of_row, r)];
+    if (x >= sc.tiles_width) return;
     const uint32_t y = r - sc.row_start;
     const uint32_t first = a.row_counts[r];
     const uint32_t last = r + 1u < a.row_count ? a.row_counts[r + 1u] : (uint32_t)a.totals[TK_FE_ROW_ENTRIES];
-    for (uint32_t xb = 0; xb < sc.tiles_width; xb += 256u) {
-        const uint32_t x = xb + threadIdx.x;
-        const bool mine = x < sc.tiles_width;
-        const uint64_t column = (uint64_t)sc.column_start + (uint64_t)y * sc.tiles_width + x;
-        uint64_t dst = mine ? a.tile_counts[column] : 0u;
-        for (uint32_t k = first; k < last && (uint64_t)k < a.row_capacity; ++k) {
-            const uint4 e = a.row_entries[k];
-            const uint32_t hx0 = e.w & 0xFFFFu, hx1 = e.w >> 16;
-            if (mine && x >= e.y && x < e.z && !(x >= hx0 && x < hx1)) {
-                if (dst < a.index_capacity) a.tile_draw_indices[dst] = e.x;
-                ++dst;
-            }
-        }
+    const uint64_t end = min((uint64_t)last, a.row_capacity);
+    uint64_t dst = a.tile_counts[(uint64_t)sc.column_start + (uint64_t)y * sc.tiles_width + x];
+    for (uint64_t base = first; base < end; base += 64u) {
+        uint4 e = make_uint4(0u, 0u, 0u, 0u);
+        if (base + lane < end) e = a.row_entries[base + lane];
+        const bool visible = x >= e.y && x < e.z && !(x >= (e.w & 0xFFFFu) && x < (e.w >> 16));
+        const uint64_t mask = __ballot(visible), at = dst + (uint32_t)__popcll(mask & lanes_below(lane));
+        if (visible && at < a.index_capacity) a.tile_draw_indices[at] = e.x;
+        dst += (uint32_t)__popcll(mask);
     }
 }
 
-// GPU flattening: one thread per path, whose closed contour of cubics goes
-// through the shared flattener (flatten.h) exactly as push_path records it: the
-// start point, then each cubic's points after its start; the path's bounds are
-// the cubics' exact bounds (add_cubic_bounds).  Pass 1 counts and bounds,
-// pass 2 (after a scan of the counts) writes the points.
+// Clears several tables in one launch.
+extern "C" __global__ __launch_bounds__(256) void tk_k_clear(tk_args_clear a) {
+    for (uint32_t k = 0; k < a.count; ++k)
+        for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < a.tables[k].count; i += gridDim.x * 256ull)
+            a.tables[k].words[i] = 0u;
+}
+
+// GPU flattening: every cubic of a path's closed contour goes through the shared
+// flattener (flatten.h) exactly as push_path records it: the start point, then each
+// cubic's points after its start; the path's bounds are the cubics' exact bounds
+// (add_cubic_bounds).  Pass 1 counts and bounds, pass 2 (after a scan of the
+// counts) writes the points.
+//
+// Bound by the chain of FP64 divisions and roots along a cubic.  Eight lanes take a
+// path, a cubic each in turn, since a path has few; pass 2 counts a cubic again before
+// it writes it, to place it behind its neighbours.  One thread per path: 94 waves for
+// 6000 paths of six cubics, 119 us a pass; eight: 26 and 47 us.
+constexpr uint32_t kFlattenLanes = 8u;
 __device__ __forceinline__ bool fl_contour(const tk_args_flatten &a, uint32_t p, uint32_t &first, uint32_t &cubics) {
     first = a.starts[p];
     const uint32_t end = a.starts[p + 1u];
@@ -485,47 +565,62 @@ __device__ __forceinline__ bool fl_contour(const tk_args_flatten &a, uint32_t p,
     return n >= 4u && (n - 1u) % 3u == 0u;
 }
 
+__device__ __forceinline__ bool fl_cubic(const double *c, uint32_t cubics, uint32_t k, tk::FPt *p) {
+    if (k >= cubics) return false;
+    for (uint32_t i = 0; i < 4u; ++i) p[i] = tk::FPt{c[6u * k + 2u * i], c[6u * k + 2u * i + 1u]};
+    return true;
+}
+
 extern "C" __global__ __launch_bounds__(256) void tk_k_flatten_count(tk_args_flatten a) {
-    const uint32_t p = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t p = blockIdx.x * (256u / kFlattenLanes) + threadIdx.x / kFlattenLanes;
+    const uint32_t member = threadIdx.x % kFlattenLanes;
     if (p >= a.path_count) return;
     uint32_t first, cubics;
     uint32_t count = 0u;
     double x0 = __builtin_inf(), y0 = __builtin_inf(), x1 = -__builtin_inf(), y1 = -__builtin_inf();
     if (!fl_contour(a, p, first, cubics)) {
-        atomicOr(a.status, 2u);
+        if (member == 0u) atomicOr(a.status, 2u);
     } else {
         const double *c = a.ctrl + 2u * first;
-        bool finite = true;
-        for (uint32_t i = 0; i < 2u * (3u * cubics + 1u); ++i) finite = finite && isfinite(c[i]);
+        uint32_t finite = 1u;
+        for (uint32_t i = member; i < 2u * (3u * cubics + 1u); i += kFlattenLanes) finite = finite && isfinite(c[i]) ? 1u : 0u;
+        for (uint32_t off = 1u; off < kFlattenLanes; off <<= 1) finite &= (uint32_t)__shfl_xor((int)finite, (int)off, kFlattenLanes);
         if (!finite) {
-            atomicOr(a.status, 1u);
+            if (member == 0u) atomicOr(a.status, 1u);
         } else {
-            count = 1u;
             auto add = [&](tk::FPt q) {
                 x0 = fmin(x0, q.x);
                 y0 = fmin(y0, q.y);
                 x1 = fmax(x1, q.x);
                 y1 = fmax(y1, q.y);
             };
-            for (uint32_t k = 0; k < cubics; ++k) {
-                const tk::FPt p0{c[6u * k], c[6u * k + 1u]}, p1{c[6u * k + 2u], c[6u * k + 3u]},
-                    p2{c[6u * k + 4u], c[6u * k + 5u]}, p3{c[6u * k + 6u], c[6u * k + 7u]};
-                tk::flatten_cubic(p0, p1, p2, p3, a.tolerance, [&](tk::FPt) { ++count; });
-                add(p0);
-                add(p3);
+            tk::FPt q[4];
+            for (uint32_t k = member; fl_cubic(c, cubics, k, q); k += kFlattenLanes) {
+                tk::flatten_cubic(q[0], q[1], q[2], q[3], a.tolerance, [&](tk::FPt) { ++count; });
+                add(q[0]);
+                add(q[3]);
                 double ts[2];
                 int nt;
-                tk::cubic_axis_extrema(p0.x, p1.x, p2.x, p3.x, ts, &nt);
+                tk::cubic_axis_extrema(q[0].x, q[1].x, q[2].x, q[3].x, ts, &nt);
                 for (int i = 0; i < nt; ++i)
-                    add(tk::FPt{tk::cubic_coord(p0.x, p1.x, p2.x, p3.x, ts[i]),
-                                tk::cubic_coord(p0.y, p1.y, p2.y, p3.y, ts[i])});
-                tk::cubic_axis_extrema(p0.y, p1.y, p2.y, p3.y, ts, &nt);
+                    add(tk::FPt{tk::cubic_coord(q[0].x, q[1].x, q[2].x, q[3].x, ts[i]),
+                                tk::cubic_coord(q[0].y, q[1].y, q[2].y, q[3].y, ts[i])});
+                tk::cubic_axis_extrema(q[0].y, q[1].y, q[2].y, q[3].y, ts, &nt);
                 for (int i = 0; i < nt; ++i)
-                    add(tk::FPt{tk::cubic_coord(p0.x, p1.x, p2.x, p3.x, ts[i]),
-                                tk::cubic_coord(p0.y, p1.y, p2.y, p3.y, ts[i])});
+                    add(tk::FPt{tk::cubic_coord(q[0].x, q[1].x, q[2].x, q[3].x, ts[i]),
+                                tk::cubic_coord(q[0].y, q[1].y, q[2].y, q[3].y, ts[i])});
             }
+            for (uint32_t off = 1u; off < kFlattenLanes; off <<= 1) {
+                count += (uint32_t)__shfl_xor((int)count, (int)off, kFlattenLanes);
+                x0 = fmin(x0, __shfl_xor(x0, (int)off, kFlattenLanes));
+                y0 = fmin(y0, __shfl_xor(y0, (int)off, kFlattenLanes));
+                x1 = fmax(x1, __shfl_xor(x1, (int)off, kFlattenLanes));
+                y1 = fmax(y1, __shfl_xor(y1, (int)off, kFlattenLanes));
+            }
+            ++count;  // the start point
         }
     }
+    if (member != 0u) return;
     a.counts[p] = count;
     a.bounds[4u * p] = x0;
     a.bounds[4u * p + 1u] = y0;
@@ -534,7 +629,8 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_flatten_count(tk_args_fla
 }
 
 extern "C" __global__ __launch_bounds__(256) void tk_k_flatten_emit(tk_args_flatten a) {
-    const uint32_t p = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t p = blockIdx.x * (256u / kFlattenLanes) + threadIdx.x / kFlattenLanes;
+    const uint32_t member = threadIdx.x % kFlattenLanes;
     if (p >= a.path_count) return;
     const uint32_t at = a.counts[p];
     const uint32_t next = p + 1u < a.path_count ? a.counts[p + 1u] : 0xFFFFFFFFu;
@@ -550,10 +646,20 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_flatten_emit(tk_args_flat
         }
         ++w;
     };
-    put(tk::FPt{c[0], c[1]});
-    for (uint32_t k = 0; k < cubics; ++k) {
-        const tk::FPt p0{c[6u * k], c[6u * k + 1u]}, p1{c[6u * k + 2u], c[6u * k + 3u]},
-            p2{c[6u * k + 4u], c[6u * k + 5u]}, p3{c[6u * k + 6u], c[6u * k + 7u]};
-        tk::flatten_cubic(p0, p1, p2, p3, a.tolerance, put);
+    if (member == 0u) put(tk::FPt{c[0], c[1]});
+    uint64_t done = (uint64_t)at + 1u;
+    for (uint32_t base = 0u; base < cubics; base += kFlattenLanes) {
+        tk::FPt q[4];
+        const bool mine = fl_cubic(c, cubics, base + member, q);
+        uint32_t count = 0u;
+        if (mine) tk::flatten_cubic(q[0], q[1], q[2], q[3], a.tolerance, [&](tk::FPt) { ++count; });
+        uint32_t upto = count;
+        for (uint32_t off = 1u; off < kFlattenLanes; off <<= 1) {
+            const uint32_t below = (uint32_t)__shfl_up((int)upto, off, kFlattenLanes);
+            if (member >= off) upto += below;
+        }
+        w = done + upto - count;
+        if (mine) tk::flatten_cubic(q[0], q[1], q[2], q[3], a.tolerance, put);
+        done += (uint32_t)__shfl((int)upto, (int)kFlattenLanes - 1, kFlattenLanes);
     }
 }

@@ -385,6 +385,25 @@ struct tk_args_fe_scan {
     uint32_t *overflow;               // set when a prefix exceeds u32
 };
 
+// The same of up to eight columns of their own lengths, each by one workgroup.
+#define TK_FE_SHORT_SCAN 16384u
+struct tk_args_fe_scan_short {
+    struct {
+        uint32_t *values;
+        uint32_t count;
+        unsigned long long *total;
+    } columns[TK_FE_PATH_COLUMNS + 2];
+    uint32_t *overflow;               // set when a prefix exceeds u32
+};
+
+struct tk_args_clear {
+    struct {
+        uint32_t *words;
+        uint64_t count;
+    } tables[6];
+    uint32_t count;
+};
+
 // GPU flattening of closed cubic contours, one per path: path p's control
 // points are ctrl[starts[p] .. starts[p+1]) = the start point, then three per
 // cubic (the two control points and the end point).
