@@ -410,6 +410,8 @@ tk_status tk_frame_render_tiles(tk_frame *frame, const uint32_t *tiles, uint32_t
  *    plain launch would deal it; an XCD whose queue is used up takes from the
  *    others) until all are used up.
  *  - scan_block: lines per scan count / emit workgroup: 64, 128, 256, 512, 1024.
+ *    (This and scan_xcd_run are of the separate scan stages: a frame that scans in
+ *    one kernel keeps them unused, and the search leaves them as they are.)
  *  - coarse_block: tiles (one 64-lane wave each) per coarse workgroup: 1, 2, 4.
  *  - coarse_scan_items: counts per workgroup of the coarse exclusive scan
  *    (decoupled lookback): 1024, 2048, 4096, 8192.
@@ -605,7 +607,9 @@ typedef struct tk_stage_times {
     float scan_clear, scan_count, scan_prefix, scan_emit, cumsum;
     float coarse_count, coarse_prefix, coarse_emit, fine, total;
 } tk_stage_times;
-/* Enables hipEvent timestamps around each stage of later renders. */
+/* Enables hipEvent timestamps around each stage of later renders.  A frame that
+ * scans in one kernel reports its time as scan_count, and the other scan stages
+ * as about zero. */
 tk_status tk_frame_enable_timing(tk_frame *frame, int enable);
 tk_status tk_frame_stage_times(tk_frame *frame, tk_stage_times *out);
 

@@ -543,7 +543,7 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_fe_tiles(tk_args_frontend
 extern "C" __global__ __launch_bounds__(256) void tk_k_clear(tk_args_clear a) {
     for (uint32_t k = 0; k < a.count; ++k)
         for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < a.tables[k].count; i += gridDim.x * 256ull)
-            a.tables[k].words[i] = 0u;
+            a.tables[k].words[i] = a.tables[k].value;
 }
 
 // GPU flattening: every cubic of a path's closed contour goes through the shared

@@ -248,11 +248,12 @@ __device__ __forceinline__ bool rounded_corner_covers(float px, float py, float 
     return !in_square || (inner > 0.0f && dx * dx + dy * dy <= inner * inner);
 }
 
-__device__ bool rect_covers_tile(const float rect[4], const float radii_in[4], const DrawData &d, uint32_t tx,
+// (te, tf): the draw's translation.
+__device__ bool rect_covers_tile(const float rect[4], const float radii_in[4], float te, float tf, uint32_t tx,
                                  uint32_t ty, float inset) {
     float lx = fminf(rect[0], rect[2]), ly = fminf(rect[1], rect[3]);
     float ux = fmaxf(rect[0], rect[2]), uy = fmaxf(rect[1], rect[3]);
-    float tlx = (float)(tx * 16u) + 0.5f - d.te, tly = (float)(ty * 16u) + 0.5f - d.tf;
+    float tlx = (float)(tx * 16u) + 0.5f - te, tly = (float)(ty * 16u) + 0.5f - tf;
     float tux = tlx + 15.0f, tuy = tly + 15.0f;
     float sx = ux - lx, sy = uy - ly;
     float need = 15.0f + 2.0f * inset;
@@ -261,7 +262,7 @@ __device__ bool rect_covers_tile(const float rect[4], const float radii_in[4], c
     float limit = fminf(sx, sy) * 0.5f;
     for (int i = 0; i < 4; ++i)
         if (!(fabsf(rect[i]) <= 65536.0f) || !(fabsf(radii_in[i]) <= 65536.0f)) return false;
-    if (!(fabsf(d.te) <= 65536.0f) || !(fabsf(d.tf) <= 65536.0f)) return false;
+    if (!(fabsf(te) <= 65536.0f) || !(fabsf(tf) <= 65536.0f)) return false;
     float r[4];
     for (int i = 0; i < 4; ++i) r[i] = fminf(fmaxf(radii_in[i], 0.0f), limit);
     return rounded_corner_covers(tlx, tly, lx, ly, lx + r[0], ly + r[0], r[0], inset) &&
@@ -274,22 +275,31 @@ __device__ __forceinline__ bool identity_linear(const DrawData &d) {
     return d.la == 1.0f && d.lb == 0.0f && d.lc == 0.0f && d.ld == 1.0f;
 }
 
-__device__ bool sdf_clip_covers(Const<uint32_t> paint, uint32_t pc, const DrawData &d, uint32_t tx, uint32_t ty) {
-    if (d.sdf_offset == kNone || d.shadow_offset != kNone || d.sdf_len < 9u) return false;
-    uint32_t base = d.sdf_offset;
-    if (paint_word(paint, pc, base) != TK_SDF_KIND_RECT || !identity_linear(d)) return false;
+// sdf_clip_covers: the draws that may cover a tile, and whether such a one does.
+__device__ __forceinline__ bool sdf_covers_some(Const<uint32_t> paint, uint32_t pc, const DrawData &d) {
+    return d.sdf_offset != kNone && d.shadow_offset == kNone && d.sdf_len >= 9u &&
+           paint_word(paint, pc, d.sdf_offset) == TK_SDF_KIND_RECT && identity_linear(d);
+}
+__device__ bool sdf_rect_covers(Const<uint32_t> paint, uint32_t pc, uint32_t base, float te, float tf, uint32_t tx,
+                                uint32_t ty) {
     float rect[4], radii[4];
     for (int i = 0; i < 4; ++i) {
         rect[i] = asfloat(paint_word(paint, pc, base + 1u + (uint32_t)i));
         radii[i] = asfloat(paint_word(paint, pc, base + 5u + (uint32_t)i));
     }
-    return rect_covers_tile(rect, radii, d, tx, ty, 0.5f);
+    return rect_covers_tile(rect, radii, te, tf, tx, ty, 0.5f);
+}
+__device__ bool sdf_clip_covers(Const<uint32_t> paint, uint32_t pc, const DrawData &d, uint32_t tx, uint32_t ty) {
+    return sdf_covers_some(paint, pc, d) && sdf_rect_covers(paint, pc, d.sdf_offset, d.te, d.tf, tx, ty);
 }
 
-__device__ bool sdf_stroke_empty(Const<uint32_t> paint, uint32_t pc, const DrawData &d, uint32_t tx, uint32_t ty) {
-    if (d.sdf_offset == kNone || d.shadow_offset != kNone || d.sdf_len < 13u || !identity_linear(d)) return false;
-    uint32_t base = d.sdf_offset;
-    if (paint_word(paint, pc, base) != 3u) return false;  // SDF_KIND_RECT_STROKE
+// sdf_stroke_empty: likewise.
+__device__ __forceinline__ bool sdf_stroke_some(Const<uint32_t> paint, uint32_t pc, const DrawData &d) {
+    return d.sdf_offset != kNone && d.shadow_offset == kNone && d.sdf_len >= 13u && identity_linear(d) &&
+           paint_word(paint, pc, d.sdf_offset) == 3u;  // SDF_KIND_RECT_STROKE
+}
+__device__ bool sdf_rect_stroke_empty(Const<uint32_t> paint, uint32_t pc, uint32_t base, float te, float tf, uint32_t tx,
+                                      uint32_t ty) {
     float rect[4], radii[4], stroke[4];
     for (int i = 0; i < 4; ++i) {
         rect[i] = asfloat(paint_word(paint, pc, base + 1u + (uint32_t)i));
@@ -308,7 +318,10 @@ __device__ bool sdf_stroke_empty(Const<uint32_t> paint, uint32_t pc, const DrawD
     float corner[4] = {fmaxf(hw[0], hw[3]), fmaxf(hw[0], hw[1]), fmaxf(hw[2], hw[3]), fmaxf(hw[2], hw[1])};
     float r[4];
     for (int i = 0; i < 4; ++i) r[i] = fmaxf(radii[i] - corner[i], 0.0f);
-    return rect_covers_tile(inner, r, d, tx, ty, 1.0f);
+    return rect_covers_tile(inner, r, te, tf, tx, ty, 1.0f);
+}
+__device__ bool sdf_stroke_empty(Const<uint32_t> paint, uint32_t pc, const DrawData &d, uint32_t tx, uint32_t ty) {
+    return sdf_stroke_some(paint, pc, d) && sdf_rect_stroke_empty(paint, pc, d.sdf_offset, d.te, d.tf, tx, ty);
 }
 
 __device__ __forceinline__ uint32_t brush_base_of(uint32_t paint_brush_base, const DrawData &d) {
@@ -333,12 +346,14 @@ __device__ __forceinline__ uint32_t full_tile_solid(Const<uint32_t> paint, uint3
     return nontransparent_solid(paint, pc, pbb, d) && sdf_clip_covers(paint, pc, d, tx, ty) ? solid_color(paint, pc, pbb, d)
                                                                                             : 0u;
 }
-__device__ __forceinline__ bool full_tile_image(Const<uint32_t> paint, uint32_t pc, uint32_t pbb, const DrawData &d,
-                                                uint32_t tx, uint32_t ty) {
+__device__ __forceinline__ bool opaque_image(Const<uint32_t> paint, uint32_t pc, uint32_t pbb, const DrawData &d) {
     if (d.brush_offset == kNone) return false;
     uint32_t base = brush_base_of(pbb, d);
-    return paint_word(paint, pc, base) == 7u && paint_word(paint, pc, base + 7u) == 255u &&
-           sdf_clip_covers(paint, pc, d, tx, ty);
+    return paint_word(paint, pc, base) == 7u && paint_word(paint, pc, base + 7u) == 255u;
+}
+__device__ __forceinline__ bool full_tile_image(Const<uint32_t> paint, uint32_t pc, uint32_t pbb, const DrawData &d,
+                                                uint32_t tx, uint32_t ty) {
+    return opaque_image(paint, pc, pbb, d) && sdf_clip_covers(paint, pc, d, tx, ty);
 }
 
 constexpr uint32_t kClassColor = 1u, kClassSdf = 2u, kClassOther = 4u;
@@ -453,7 +468,21 @@ __device__ Particle draw_particle(const CoarseCtx &c, uint32_t batch, uint32_t d
 __device__ __forceinline__ Particle entry_particle(const CoarseCtx &c, uint32_t draw_index, uint4 box, uint4 words) {
     Particle p{false, TK_PTCL_FILL, 0u, 0u, 0u, 0u, 0u};
     const uint32_t kind = words.w & TK_ENTRY_KIND;
-    if (kind == TK_ENTRY_SDF) return sdf_particle(c, load_draw(c.in->draws, c.cfg->draw_count, draw_index), draw_index);
+    if (kind == TK_ENTRY_SDF) {  // sdf_particle, from {SDF offset, translation} and the brush's colour
+        const Const<uint32_t> paint = constant(c.in->paint);
+        const float te = asfloat(box.y), tf = asfloat(box.z);
+        if ((words.w & TK_ENTRY_STROKE) && sdf_rect_stroke_empty(paint, c.cfg->paint_words, box.x, te, tf, c.tx, c.ty)) return p;
+        p.valid = true;
+        p.color = draw_index;
+        if ((words.w & TK_ENTRY_COVERS) && sdf_rect_covers(paint, c.cfg->paint_words, box.x, te, tf, c.tx, c.ty)) {
+            p.tag = (words.w & TK_ENTRY_SOLID_RECT) ? (uint32_t)TK_PTCL_COLOR : kPtclImage;
+            if (words.w & TK_ENTRY_SOLID_RECT) p.color = words.x;
+        } else {
+            p.tag = TK_PTCL_SDF;
+            p.seg_start = draw_index;
+        }
+        return p;
+    }
     if (kind == TK_ENTRY_NONE || c.tx < box.x || c.ty < box.y || c.tx >= box.z || c.ty >= box.w) return p;
     const uint32_t bd = words.x + c.ty * words.y + c.tx;
     const tk_segment_range range = c.in->segment_ranges[bd];
@@ -472,8 +501,8 @@ __device__ __forceinline__ Particle entry_particle(const CoarseCtx &c, uint32_t 
         p.tag = kPtclPathGlyph;
     } else if ((words.w & TK_ENTRY_SOLID_RECT) && range.start == range.end) {
         p.tag = TK_PTCL_COLOR;
-        p.color = solid_color(constant(c.in->paint), c.cfg->paint_words, c.cfg->paint_brush_base,
-                              load_draw(c.in->draws, c.cfg->draw_count, draw_index));
+        p.color = paint_word(constant(c.in->paint), c.cfg->paint_words,
+                             c.cfg->paint_brush_base + c.in->draws[draw_index].brush_offset + 4u);
     }
     return p;
 }
@@ -1508,7 +1537,6 @@ struct ChunkRuns {
     uint64_t heads;    // lanes that begin a run (not lane 0 when it goes on with `cur`)
     uint32_t head;     // this lane's run's first lane; 64: of the open run
     uint64_t run;      // a head's run's lanes
-    uint32_t previous; // a head's batch before
     bool closed;       // a head's run is closed
     uint64_t rest;     // lanes of the runs that are not
 };
@@ -1520,7 +1548,6 @@ __device__ __forceinline__ ChunkRuns chunk_runs(const tk_args_coarse &a, const T
     r.head = mine ? 63u - (uint32_t)__clzll((long long)mine) : 64u;
     const uint32_t end = above ? (uint32_t)__builtin_ctzll(above) : n;
     r.run = lanes_below(end) & ~lanes_below(lane);
-    r.previous = before;
     bool acts = false;
     if (a.cfg.layer_count && lane < n) {
         acts = true;
@@ -1661,8 +1688,9 @@ __device__ __forceinline__ void coarse_count_tile(const tk_args_coarse &a, uint3
         }
         if (++pending == 64u) resolve();
     };
-    auto empty_until = [&](uint32_t stop) {
-        for (uint32_t bb = next + lane; bb < stop; bb += 64u) counts[table_index(v, bb)] = 0u;
+    auto empty_until = [&](uint32_t stop) {  // a frame's table is cleared in front
+        if constexpr (!kFrame)
+            for (uint32_t bb = next + lane; bb < stop; bb += 64u) counts[table_index(v, bb)] = 0u;
         next = max(next, stop);
     };
     // A list out of batch order (the recorder never produces one; the stage entry
@@ -1689,12 +1717,9 @@ __device__ __forceinline__ void coarse_count_tile(const tk_args_coarse &a, uint3
                           !__ballot(lane < n && (b == kNone || (b < before && (lane || cur != kNone))));
             if (ordered) {
                 const ChunkRuns r = chunk_runs(a, layers, n, base + 64u >= len, b, before, cur, lane);
-                if ((r.heads >> lane) & 1ull) {
-                    for (uint32_t bb = r.previous + 1u; bb < b; ++bb) counts[table_index(v, bb)] = 0u;
-                    if (r.closed) {
-                        const uint32_t k = (uint32_t)__popcll(valid_mask & r.run);
-                        counts[table_index(v, b)] = k ? k + 1u : 0u;
-                    }
+                if (r.closed) {
+                    const uint32_t k = (uint32_t)__popcll(valid_mask & r.run);
+                    counts[table_index(v, b)] = k ? k + 1u : 0u;
                 }
                 pending_runs = r.rest;
                 next = (uint32_t)__builtin_amdgcn_readlane((int)b, (int)(n - 1u)) + 1u;
@@ -1776,35 +1801,54 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_coarse_count_scenes_persi
 // coarse_prefix_chunks + coarse_chunk_offsets + coarse_apply_chunk_offsets for
 // every batch: one wrapping exclusive scan over the batch-major count table.
 // A batch's reference (per-batch) offsets are start - batch_ptcl_bases[batch].
-// kItems consecutive counts per lane, 256 * kItems per workgroup (a.scan_blocks
-// workgroups): the scan block size is a launch choice among 1024-8192 counts.
+// 256 * kItems counts per workgroup (a.scan_blocks workgroups): the scan block size is
+// a launch choice among 1024-8192 counts.  Bound by the table's bytes and by launch
+// and lookback: a lane takes four counts in a row of every 1024, 16 bytes read and 32
+// written, so that a wave's accesses run on.  (kItems counts in a row per lane, a wave
+// 128 bytes apart in its reads and 256 in its writes: 1.06 M counts 18.3 us; now 15.4, half of it lookback.)
 template <uint32_t kItems>
 __device__ __forceinline__ void coarse_scan(const tk_args_coarse &a) {
+    constexpr uint32_t kRounds = kItems / 4u;
     __shared__ uint32_t s_ticket, s_base;
-    __shared__ uint32_t s_wave[4];
+    __shared__ uint32_t s_sum[kRounds][4];
     const uint32_t k = draw_ticket(a.ticket, a.scan_blocks, &s_ticket);
     const uint64_t n = a.scenes.slots ? a.scenes.table_entries : (uint64_t)a.cfg.batch_count * a.list.columns;
-    const uint64_t first = ((uint64_t)k * 256u + threadIdx.x) * kItems;
-    uint32_t v[kItems];
-    uint32_t sum = 0u;
-    if (first + kItems <= n && ((uintptr_t)a.out.tile_ptcl_counts & 15u) == 0u) {
-        const uint4 *src = reinterpret_cast<const uint4 *>(a.out.tile_ptcl_counts + first);
+    const uint64_t first = (uint64_t)k * (256u * kItems) + threadIdx.x * 4u;  // plus 1024 per round
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const bool aligned = (((uintptr_t)a.out.tile_ptcl_counts | (uintptr_t)a.out.tile_ptcl_ranges) & 15u) == 0u;
+    uint32_t v[kRounds][4], upto[kRounds];
 #pragma unroll
-        for (uint32_t q = 0; q < kItems / 4u; ++q) {
-            const uint4 w = src[q];
-            v[4 * q] = w.x;
-            v[4 * q + 1] = w.y;
-            v[4 * q + 2] = w.z;
-            v[4 * q + 3] = w.w;
+    for (uint32_t r = 0; r < kRounds; ++r) {
+        const uint64_t at = first + r * 1024u;
+        if (aligned && at + 4u <= n) {
+            const uint4 w = *reinterpret_cast<const uint4 *>(a.out.tile_ptcl_counts + at);
+            v[r][0] = w.x;
+            v[r][1] = w.y;
+            v[r][2] = w.z;
+            v[r][3] = w.w;
+        } else {
+#pragma unroll
+            for (uint32_t i = 0; i < 4u; ++i) v[r][i] = at + i < n ? a.out.tile_ptcl_counts[at + i] : 0u;
         }
-    } else {
-#pragma unroll
-        for (uint32_t i = 0; i < kItems; ++i) v[i] = first + i < n ? a.out.tile_ptcl_counts[first + i] : 0u;
     }
 #pragma unroll
-    for (uint32_t i = 0; i < kItems; ++i) sum += v[i];
-    uint32_t total;
-    const uint32_t excl = block_exclusive_scan_256(sum, s_wave, total);
+    for (uint32_t r = 0; r < kRounds; ++r) {
+        upto[r] = wave_inclusive_scan_dpp(v[r][0] + v[r][1] + v[r][2] + v[r][3]);
+        if (lane == 63u) s_sum[r][wave] = upto[r];
+    }
+    __syncthreads();
+    uint32_t total = 0u;
+#pragma unroll
+    for (uint32_t r = 0; r < kRounds; ++r) {
+        uint32_t before = total;
+#pragma unroll
+        for (uint32_t w = 0; w < 4u; ++w) {
+            const uint32_t sum = s_sum[r][w];
+            if (w < wave) before += sum;
+            total += sum;
+        }
+        upto[r] += before - (v[r][0] + v[r][1] + v[r][2] + v[r][3]);  // now the slots before the lane's four
+    }
     if (threadIdx.x < 64u) {
         uint32_t base = 0u;
         if (k > 0u) {
@@ -1821,21 +1865,34 @@ __device__ __forceinline__ void coarse_scan(const tk_args_coarse &a) {
         }
     }
     __syncthreads();
-    if (first >= n) return;
-    uint32_t running = s_base + excl;
-    uint64_t batch = first / a.list.columns;
-    uint32_t offset = (uint32_t)(first - batch * a.list.columns);
 #pragma unroll
-    for (uint32_t i = 0; i < kItems; ++i) {
-        const uint64_t idx = first + i;
-        if (idx < n) {
-            a.out.tile_ptcl_ranges[idx] = tk_segment_range{running, running + v[i]};
-            if (offset == 0u && !a.scenes.slots) a.out.batch_ptcl_bases[batch] = running;
+    for (uint32_t r = 0; r < kRounds; ++r) {
+        const uint64_t at = first + r * 1024u;
+        if (at >= n) return;
+        uint32_t slot[5] = {s_base + upto[r]};
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i) slot[i + 1u] = slot[i] + v[r][i];
+        if (aligned && at + 4u <= n) {
+            uint4 *dst = reinterpret_cast<uint4 *>(a.out.tile_ptcl_ranges + at);
+            dst[0] = make_uint4(slot[0], slot[1], slot[1], slot[2]);
+            dst[1] = make_uint4(slot[2], slot[3], slot[3], slot[4]);
+        } else {
+#pragma unroll
+            for (uint32_t i = 0; i < 4u; ++i)
+                if (at + i < n) a.out.tile_ptcl_ranges[at + i] = tk_segment_range{slot[i], slot[i + 1u]};
         }
-        running += v[i];
-        if (++offset == a.list.columns) {
-            offset = 0u;
-            ++batch;
+        if (a.scenes.slots) continue;
+        // where a batch begins
+        const bool narrow = (at >> 32) == 0ull;
+        uint64_t batch = narrow ? (uint64_t)((uint32_t)at / a.list.columns) : at / a.list.columns;
+        uint32_t offset = (uint32_t)(at - batch * a.list.columns);
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i) {
+            if (offset == 0u && at + i < n) a.out.batch_ptcl_bases[batch] = slot[i];
+            if (++offset == a.list.columns) {
+                offset = 0u;
+                ++batch;
+            }
         }
     }
 }
@@ -1875,8 +1932,9 @@ __device__ __forceinline__ void coarse_emit_tile(const tk_args_coarse &a, uint32
     bool single_pass = false;  // the batch's stack is at most 64 layers: ENDs come from registers
     uint64_t stack_emitted = 0ull;
     uint32_t stack_end_tag = TK_PTCL_END_CLIP;
-    auto empty_until = [&](uint32_t stop) {
-        for (uint32_t bb = next + lane; bb < stop; bb += 64u) kinds[table_index(v, bb)] = TK_TILE_KIND_EMPTY;
+    auto empty_until = [&](uint32_t stop) {  // a frame's table is cleared in front
+        if constexpr (!kFrame)
+            for (uint32_t bb = next + lane; bb < stop; bb += 64u) kinds[table_index(v, bb)] = TK_TILE_KIND_EMPTY;
         next = max(next, stop);
     };
     auto finish = [&]() {
@@ -1951,7 +2009,14 @@ __device__ __forceinline__ void coarse_emit_tile(const tk_args_coarse &a, uint32
             uint32_t my_pos = kNone;
             const Particle p = list_particle<kFrame>(c, entry);
             uint32_t cls = 0u;
-            if (p.valid) cls = particle_class_flags(c, entry.draw, p.tag);
+            if constexpr (kFrame)
+                cls = !p.valid                      ? 0u
+                      : p.tag == TK_PTCL_COLOR      ? kClassColor
+                      : p.tag == kPtclImage         ? kClassSdf
+                      : p.tag != TK_PTCL_SDF        ? kClassOther
+                      : (entry.words.w & TK_ENTRY_SDF_CLASS) ? kClassSdf : kClassOther;
+            else if (p.valid)
+                cls = particle_class_flags(c, entry.draw, p.tag);
             const bool p_opaque = p.valid && p.tag == TK_PTCL_COLOR && (p.color >> 24) == 255u;
             const bool p_begins = p.valid && is_begin_tag(p.tag);
             uint64_t pending = __ballot(b != kNone);
@@ -1970,24 +2035,18 @@ __device__ __forceinline__ void coarse_emit_tile(const tk_args_coarse &a, uint32
                     const uint32_t pos = my_range.start + (uint32_t)__popcll(valid & lanes_below(lane) & ~lanes_below(r.head));
                     if (pos < my_range.end) my_pos = pos;
                 }
-                if ((r.heads >> lane) & 1ull) {
-                    for (uint32_t bb = r.previous + 1u; bb < b; ++bb) kinds[table_index(v, bb)] = TK_TILE_KIND_EMPTY;
-                    if (r.closed) {  // what begin, the loop below and finish do for one run without layers
-                        uint32_t kind = TK_TILE_KIND_EMPTY;
-                        if (my_range.end > my_range.start) {
-                            const uint64_t drawn = valid & r.run, covers = opaque & r.run;
-                            const uint32_t set = ((color & r.run) ? kClassColor : 0u) | ((sdf & r.run) ? kClassSdf : 0u) |
-                                                 ((other & r.run) ? kClassOther : 0u);
-                            uint32_t skip = 0u;
-                            if ((covers & ~(drawn & (0ull - drawn))) && my_range.end - my_range.start > 2u) {
-                                const uint32_t h = 63u - (uint32_t)__clzll((long long)covers);
-                                if (!((begins & r.run) >> h)) skip = (uint32_t)__popcll(drawn & lanes_below(h));
-                            }
-                            kind = classify_tile_flags(set) | (skip << TK_TILE_PREFIX_SHIFT);
-                            e.store(my_range.start + (uint32_t)__popcll(drawn), TK_PTCL_END, 0u, 0u, 0u, 0u, 0u);
-                        }
-                        kinds[table_index(v, b)] = kind;
+                // what begin, the loop below and finish do for one run without layers
+                if (r.closed && my_range.end > my_range.start) {
+                    const uint64_t drawn = valid & r.run, covers = opaque & r.run;
+                    const uint32_t set = ((color & r.run) ? kClassColor : 0u) | ((sdf & r.run) ? kClassSdf : 0u) |
+                                         ((other & r.run) ? kClassOther : 0u);
+                    uint32_t skip = 0u;
+                    if ((covers & ~(drawn & (0ull - drawn))) && my_range.end - my_range.start > 2u) {
+                        const uint32_t h = 63u - (uint32_t)__clzll((long long)covers);
+                        if (!((begins & r.run) >> h)) skip = (uint32_t)__popcll(drawn & lanes_below(h));
                     }
+                    kinds[table_index(v, b)] = classify_tile_flags(set) | (skip << TK_TILE_PREFIX_SHIFT);
+                    e.store(my_range.start + (uint32_t)__popcll(drawn), TK_PTCL_END, 0u, 0u, 0u, 0u, 0u);
                 }
                 pending = r.rest;
                 next = (uint32_t)__builtin_amdgcn_readlane((int)b, (int)(n - 1u)) + 1u;
@@ -2091,8 +2150,19 @@ __device__ __forceinline__ void draw_tables(const tk_args_draw_tables &a, uint32
         const DrawData draw = load_draw(a.draws, a.draw_count, d);
         uint32_t kind = TK_ENTRY_NONE, base = 0u, stride = 0u;
         uint4 box = make_uint4(0u, 0u, 0u, 0u);
+        const Const<uint32_t> paint = constant(a.paint);
         if (draw_has_sdf(draw)) {
-            kind = TK_ENTRY_SDF;
+            if (draw.tag == TK_DRAW_BRUSH) {
+                const bool solid = nontransparent_solid(paint, a.paint_words, a.paint_brush_base, draw);
+                kind = TK_ENTRY_SDF | (solid ? TK_ENTRY_SOLID_RECT : 0u);
+                if (sdf_stroke_some(paint, a.paint_words, draw)) kind |= TK_ENTRY_STROKE;
+                if (sdf_covers_some(paint, a.paint_words, draw) &&
+                    (solid || opaque_image(paint, a.paint_words, a.paint_brush_base, draw)))
+                    kind |= TK_ENTRY_COVERS;
+                if (solid_supported_sdf(paint, a.paint_words, a.paint_brush_base, draw)) kind |= TK_ENTRY_SDF_CLASS;
+                if (solid) base = solid_color(paint, a.paint_words, a.paint_brush_base, draw);
+                box = make_uint4(draw.sdf_offset, asuint(draw.te), asuint(draw.tf), 0u);
+            }
         } else if (draw.path_id < a.path_count && draw.path_id != kNone &&
                    (draw.tag == TK_DRAW_BRUSH || draw.tag == TK_DRAW_PATH_GLYPH || draw.tag == TK_DRAW_CLIP)) {
             const tk_path_record &p = a.paths[draw.path_id];
@@ -2101,7 +2171,7 @@ __device__ __forceinline__ void draw_tables(const tk_args_draw_tables &a, uint32
                              min(tile_max_of(draw.pb[2], ~0u), p.tile_x1), min(tile_max_of(draw.pb[3], ~0u), p.tile_y1));
             kind = draw.tag == TK_DRAW_BRUSH ? TK_ENTRY_FILL : (draw.tag == TK_DRAW_CLIP ? TK_ENTRY_CLIP : TK_ENTRY_GLYPH);
             if (draw.tag == TK_DRAW_BRUSH && draw.solid_rect != 0u && draw.lb == 0.0f && draw.lc == 0.0f &&
-                nontransparent_solid(constant(a.paint), a.paint_words, a.paint_brush_base, draw))
+                nontransparent_solid(paint, a.paint_words, a.paint_brush_base, draw))
                 kind |= TK_ENTRY_SOLID_RECT;
             if (draw.fill_rule >> (32u - TK_ENTRY_RULE_SHIFT)) kind |= TK_ENTRY_RECORD_RULE;
             else kind |= draw.fill_rule << TK_ENTRY_RULE_SHIFT;

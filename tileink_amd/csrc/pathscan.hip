@@ -184,9 +184,9 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_path_scan(tk_args_path_sc
     static_assert(TK_PATH_SCAN_LINES + TK_PATH_SCAN_RUN < 65536u, "the queues hold line numbers in 16 bits");
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = uniform(tid >> 6);
 #pragma unroll
-    for (uint32_t k = 0; k < 3u; ++k)  // words that later kernels of the frame start from zero
+    for (uint32_t k = 0; k < 5u; ++k)  // tables that later kernels of the frame start from
         for (uint64_t i = blockIdx.x * 256ull + tid; i < a.clear[k].count; i += gridDim.x * 256ull)
-            a.clear[k].words[i] = 0u;
+            a.clear[k].words[i] = a.clear[k].value;
     if (blockIdx.x >= a.runs) {  // the workgroups behind the runs build the draw tables, a launch less
         draw_tables(a.tables, (blockIdx.x - a.runs) * 256u + tid);
         return;

@@ -5,10 +5,12 @@
 // The frame pipeline replaces the reference's per-frame dispatch list
 // (src/native/runtime/program/scene_scan.rs:73-325, program/cumsum.rs:171-269,
 // program/coarse.rs:29-129, program/fine.rs:26-67, one coarse+fine pair per
-// DrawBatch) with a fixed sequence of gfx950 kernels on one stream:
-//   clear -> scan_count -> scan_prefix -> scan_emit -> cumsum
-//   -> coarse_count -> coarse_scan -> coarse_emit -> fine
-// where coarse and fine process every DrawBatch in a single launch.
+// DrawBatch) with a fixed sequence of gfx950 kernels:
+//   path_scan -> layer_classes -> coarse_count -> coarse_scan -> coarse_emit -> fine
+// where path_scan does all scan stages and coarse and fine process every DrawBatch
+// in a single launch.  Frames whose records do not lie path by path run
+//   clear -> draw_tables -> scan_count -> scan_prefix -> scan_emit
+// in its place, with cumsum and coarse on a second stream beside them.
 
 #include <hip/hip_runtime.h>
 
@@ -200,12 +202,13 @@ tk_status fill_u32(tk_context *ctx, void *dst, uint64_t count, uint32_t value) {
 struct ClearTable {
     void *words;
     uint64_t count;
+    uint32_t value = 0;
 };
 tk_status clear_tables(tk_context *ctx, std::initializer_list<ClearTable> tables) {
     tk_args_clear a{};
     uint64_t most = 1;
     for (const ClearTable &t : tables) {
-        a.tables[a.count++] = {static_cast<uint32_t *>(t.words), t.count};
+        a.tables[a.count++] = {static_cast<uint32_t *>(t.words), t.count, t.value};
         most = std::max(most, t.count);
     }
     return launch(ctx, ctx->f_clear, uint32_t(std::min<uint64_t>(div_up(most, 256), 65536)), 1, 256, a);
@@ -422,7 +425,7 @@ struct tk_frame {
     uint32_t *layer_pair_of = nullptr, *pair_layer = nullptr;
     uint8_t *layer_bits = nullptr;
     uint32_t pair_capacity = 0, pair_count = 0;
-    uint4 *batch_pairs = nullptr;
+    uint4 *batch_pairs = nullptr;  // with layer_pair_of and pair_layer behind it
     std::vector<uint32_t> host_pair_of, host_pair_layer;
     std::vector<uint4> host_batch_pairs;
     // incremental renders: the listed tiles, the damage summed-area table, per-path flags
@@ -686,10 +689,16 @@ tk_status frame_upload(tk_frame *f, const tk_scene *s) {
     if (f->layer_bits && s->layer_count && s->layers) {
         const uint32_t pairs = layer_pairs(s, f->host_pair_of, f->host_pair_layer);
         if (pairs <= f->pair_capacity) {  // else: no table for this scene
-            TK_TRY(upload(f, f->layer_pair_of, f->host_pair_of.data(), s->layer_count));
-            TK_TRY(upload(f, f->pair_layer, f->host_pair_layer.data(), pairs));
+            // one buffer, one copy: the batches' pairs, the layers', and the pairs' layers
             batch_pairs(*f, *s, f->host_batch_pairs);
-            TK_TRY(upload(f, f->batch_pairs, f->host_batch_pairs.data(), s->batch_count));
+            const size_t batches = f->host_batch_pairs.size();
+            f->host_batch_pairs.resize(batches + (uint64_t(s->layer_count) + pairs + 3) / 4);
+            uint32_t *words = reinterpret_cast<uint32_t *>(f->host_batch_pairs.data() + batches);
+            std::copy(f->host_pair_of.begin(), f->host_pair_of.end(), words);
+            std::copy(f->host_pair_layer.begin(), f->host_pair_layer.end(), words + s->layer_count);
+            TK_TRY(upload(f, f->batch_pairs, f->host_batch_pairs.data(), f->host_batch_pairs.size()));
+            f->layer_pair_of = reinterpret_cast<uint32_t *>(f->batch_pairs + batches);
+            f->pair_layer = f->layer_pair_of + s->layer_count;
             f->pair_count = pairs;
         }
     }
@@ -875,18 +884,21 @@ tk_status frame_render(tk_frame *f, uint32_t active_count = 0, const DiffTarget 
     f->epoch = (f->epoch + 1u) & 0x3FFFFFFFu;
     if (f->epoch == 0u) f->epoch = 1u;
 
-    const uint64_t status_words = 2ull * frame_scan_blocks(f, active_count);
+    // What the frame starts from: the status; the coarse scan's lookback words (a
+    // replayed graph, whose epoch argument is fixed, must not see the previous frame's
+    // flags); the persistent launches' work counters (coarse count, coarse emit, fine);
+    // and the batch tables, most of whose entries a scene of many batches leaves empty
+    // (a tile's entries lie a canvas apart: 1 M entries by tiles 10 us, in order 3).
+    const ClearTable clear[5] = {{f->status, 4},
+                                 {f->coarse_status, 2ull * frame_scan_blocks(f, active_count)},
+                                 {f->queues, f->tuning.persistent ? kQueueWords : 0},
+                                 {f->tile_counts, frame_table_entries(f, active_count)},
+                                 {f->tile_kinds, frame_table_entries(f, active_count), TK_TILE_KIND_EMPTY}};
     TK_TRY(record(f, 0));
     if (!f->path_scan) {
         // scan_clear: the deltas and counts accumulate; every other scan output is fully rewritten.
-        TK_TRY(fill_u32(ctx, f->backdrops, s.backdrop_len, 0u));
-        TK_TRY(fill_u32(ctx, f->seg_counts, s.backdrop_len, 0u));
-        TK_TRY(fill_u32(ctx, f->status, 4, 0u));
-        // The coarse scan's lookback words start each frame at zero, so a replayed
-        // graph (whose epoch argument is fixed) never sees the previous frame's flags.
-        TK_TRY(fill_u32(ctx, f->coarse_status, status_words, 0u));
-        // The persistent launches' work counters (coarse count, coarse emit, fine) start at zero.
-        if (f->tuning.persistent) TK_TRY(fill_u32(ctx, f->queues, kQueueWords, 0u));
+        TK_TRY(clear_tables(ctx, {{f->backdrops, s.backdrop_len}, {f->seg_counts, s.backdrop_len}}));
+        TK_TRY(clear_tables(ctx, {clear[0], clear[1], clear[2], clear[3], clear[4]}));
     }
     const tk_args_draw_tables tables{f->draws, s.draw_count, f->paint, s.paint_words, s.paint_brush_base,
                                      diff ? nullptr : f->draw_brush, f->draw_entries, f->paths, s.path_count, f->batch_ids};
@@ -951,9 +963,7 @@ tk_status frame_render(tk_frame *f, uint32_t active_count = 0, const DiffTarget 
         a.raw_backdrops = f->capture_raw ? f->raw_backdrops : nullptr;
         a.backdrops = f->backdrops;
         a.segments = f->segments;
-        a.clear[0] = {f->status, 4};
-        a.clear[1] = {reinterpret_cast<uint32_t *>(f->coarse_status), status_words};
-        a.clear[2] = {f->queues, f->tuning.persistent ? kQueueWords : 0};
+        for (int k = 0; k < 5; ++k) a.clear[k] = {static_cast<uint32_t *>(clear[k].words), clear[k].count, clear[k].value};
         a.runs = uint32_t(path_scan_positions(s) / a.run) + 1u;
         a.tables = tables;
         TK_TRY(launch(ctx, ctx->f_path_scan, a.runs + div_up(s.draw_count, 256), 1, 256, a, TK_PATH_SCAN_LDS(a.run)));
@@ -1140,9 +1150,7 @@ tk_status frame_create(tk_context *ctx, const tk_scene *s, const BatchLayout *ba
         std::vector<uint32_t> pair_of, pair_layer;
         const uint64_t pairs = layer_pairs(s, pair_of, pair_layer);
         if (pairs * T <= kMaxLayerClassBytes) {
-            ALLOC(layer_pair_of, s->layer_count);
-            ALLOC(pair_layer, pairs);
-            ALLOC(batch_pairs, s->batch_count);
+            ALLOC(batch_pairs, s->batch_count + (uint64_t(s->layer_count) + pairs + 3) / 4);
             ALLOC(layer_bits, pairs * T);
             f->pair_capacity = uint32_t(pairs);
         }

@@ -28,6 +28,12 @@ struct tk_args_fill {
     uint32_t value;
 };
 
+struct tk_table_fill {
+    uint32_t *words;
+    uint64_t count;
+    uint32_t value;
+};
+
 struct tk_args_copy {
     const uint4 *src;
     uint4 *dst;
@@ -120,10 +126,13 @@ enum tk_draw_entry_kind : uint32_t {
     TK_ENTRY_FILL = 1,       // a brush over its path
     TK_ENTRY_GLYPH = 2,
     TK_ENTRY_CLIP = 3,
-    TK_ENTRY_SDF = 4,        // by its record
+    TK_ENTRY_SDF = 4,        // the words are {SDF offset, translation x and y, 0}, {solid colour, 0, batch, kind}
     TK_ENTRY_KIND = 7,
-    TK_ENTRY_SOLID_RECT = 8, // with FILL: a COLOR particle on tiles without segments
+    TK_ENTRY_SOLID_RECT = 8, // with FILL: a COLOR particle on tiles without segments; with SDF: a solid brush
     TK_ENTRY_RECORD_RULE = 16, // a fill rule too large for the entry
+    TK_ENTRY_COVERS = 32,    // with SDF: a COLOR or IMAGE particle on tiles inside the rectangle
+    TK_ENTRY_STROKE = 64,    // with SDF: nothing on tiles inside the stroke
+    TK_ENTRY_SDF_CLASS = 128,  // with SDF: its other particles are of the SDF tile class
     TK_ENTRY_RULE_SHIFT = 8,
 };
 struct tk_args_draw_tables {
@@ -157,10 +166,7 @@ struct tk_args_path_scan {
     int32_t *raw_backdrops;       // the deltas before their prefix sums; null: not wanted
     int32_t *backdrops;
     tk_line_segment *segments;
-    struct {
-        uint32_t *words;
-        uint64_t count;
-    } clear[3];                   // words to clear on the way
+    tk_table_fill clear[5];       // tables to clear on the way
     tk_args_draw_tables tables;   // built by the workgroups after the runs
 };
 
@@ -397,10 +403,7 @@ struct tk_args_fe_scan_short {
 };
 
 struct tk_args_clear {
-    struct {
-        uint32_t *words;
-        uint64_t count;
-    } tables[6];
+    tk_table_fill tables[6];
     uint32_t count;
 };
 
