@@ -5,12 +5,15 @@
 // and loaded by the host through hipModuleLoadData.  Each kernel takes one
 // argument block (tk_kernel_args.h) by value.
 //
-// Stage map (reference entry -> kernel):
+// Stage map (reference entry -> kernel).  A frame whose records lie path by path, as
+// recorded scenes' do, runs the five scan stages as tk_k_path_scan (pathscan.hip),
+// which builds coarse's and fine's per-draw tables beside; the separate scan kernels
+// serve the stage entry points and the other frames.
 //   scan_clear                       -> tk_k_scan_clear
 //   scan_count                       -> tk_k_scan_count
 //   scan_prefix_chunks + scan_chunk_offsets + scan_apply_chunk_offsets
-//                                    -> tk_k_scan_prefix (single pass, decoupled lookback)
-//   scan_emit                        -> tk_k_scan_emit (slot order canonicalised when fine stages a tile)
+//                                    -> tk_k_scan_prefix, tk_k_scan_chunk_apply
+//   scan_emit                        -> tk_k_scan_emit
 //   cumsum_*                         -> tk_k_cumsum
 //   coarse_count_bins   (x batches)  -> tk_k_coarse_count  (all batches, one pass over each tile list)
 //   coarse_prefix_*     (x batches)  -> tk_k_coarse_scan   (one decoupled-lookback pass over batch x tile)
@@ -2946,14 +2949,20 @@ TK_DIFF_KERNELS(_clips, false, true)
 TK_DIFF_KERNELS(_scenes_clips, true, true)
 #undef TK_DIFF_KERNELS
 
-// One thread per line: walks the pixels the line crosses inside its path's
-// tile box, row slab by row slab and then column by column, and integrates
-// dL/dcoverage along it.  For the part of the line with parameter s in
+// Walks the pixels that a line crosses inside its path's tile box, row slab by row
+// slab and then column by column, and integrates dL/dcoverage along it.  For the part of the line with parameter s in
 // [s_a, s_b] inside a pixel, the pixel's coverage moves by
 //   -n . (dp0 * int (1 - s) ds + dp1 * int s ds),   n = (p0.y - p1.y, p1.x - p0.x),
 // n pointing to the side where the winding number is one higher.
+//
+// Bound by the two dependent loads of a pixel, so eight lanes share a line, each
+// taking every fourth row and every second column, and a lane looks the record up
+// once per tile.  16,000 lines, 300 paths at 256x256: one thread per line 26 us, four
+// lanes 9.5, eight 5.8; 64 such scenes: 73, 48 and 48.
+constexpr uint32_t kLineRows = 4u, kLineColumns = 2u, kLineLanes = kLineRows * kLineColumns;
 extern "C" __global__ __launch_bounds__(256) void tk_k_line_backward(tk_args_line_backward a) {
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t i = blockIdx.x * (256u / kLineLanes) + threadIdx.x / kLineLanes;
+    const int row_of = (int)(threadIdx.x % kLineRows), column_of = (int)(threadIdx.x / kLineRows % kLineColumns);
     if (i >= a.line_count) return;
     const tk_line ln = a.lines[i];
     const float x0 = ln.p0[0], y0 = ln.p0[1], x1 = ln.p1[0], y1 = ln.p1[1];
@@ -2971,7 +2980,8 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_line_backward(tk_args_lin
             const int r1 = min(dy == 0.0f ? (int)floorf(fminf(ylo, (float)cy1 + 1.0f))
                                           : (int)ceilf(fminf(yhi, (float)cy1 + 2.0f)) - 1,
                                cy1);
-            for (int r = r0; r <= r1; ++r) {
+            uint32_t known = kNone, k = 0u;  // the tile looked up last, and its record
+            for (int r = r0 + row_of; r <= r1; r += (int)kLineRows) {
                 float sa = 0.0f, sb = 1.0f;
                 if (dy != 0.0f) {
                     const float ta = ((float)r - y0) / dy, tb = ((float)(r + 1) - y0) / dy;
@@ -2986,7 +2996,7 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_line_backward(tk_args_lin
                                               : (int)ceilf(fminf(xhi, (float)cx1 + 2.0f)) - 1,
                                    cx1);
                 const uint32_t row_base = p.data_offset + ((uint32_t)r / 16u - p.tile_y0) * bw;
-                for (int c = c0; c <= c1; ++c) {
+                for (int c = c0 + column_of; c <= c1; c += (int)kLineColumns) {
                     float ua = sa, ub = sb;
                     if (dx != 0.0f) {
                         const float ta = ((float)c - x0) / dx, tb = ((float)(c + 1) - x0) / dx;
@@ -2996,7 +3006,10 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_line_backward(tk_args_lin
                     if (!(ub > ua)) continue;
                     const uint32_t bd = row_base + (uint32_t)c / 16u - p.tile_x0;
                     if (bd >= a.rec_of_count) continue;
-                    const uint32_t k = a.rec_of[bd];
+                    if (bd != known) {
+                        known = bd;
+                        k = a.rec_of[bd];
+                    }
                     if (k >= a.adj_records) continue;  // no record there (kNone), or beyond the buffer
                     const float gv = a.adj[(size_t)k * 256u + ((uint32_t)r & 15u) * 16u + ((uint32_t)c & 15u)];
                     const float i1 = 0.5f * (ub * ub - ua * ua);
@@ -3006,6 +3019,11 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_line_backward(tk_args_lin
             }
         }
     }
+    for (int off = 1; off < (int)kLineLanes; off <<= 1) {
+        g0 += __shfl_xor(g0, off, (int)kLineLanes);
+        g1 += __shfl_xor(g1, off, (int)kLineLanes);
+    }
+    if (threadIdx.x % kLineLanes != 0u) return;
     const float nx = y0 - y1, ny = dx;
     float *out = a.line_grad + (size_t)i * 4u;
     out[0] = -nx * g0;

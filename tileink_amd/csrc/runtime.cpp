@@ -2217,7 +2217,7 @@ tk_status tk_frame_backward(tk_frame *f, const float *colors, const float *image
     if (s.line_count) {
         tk_args_line_backward b{f->lines, s.line_count, s.path_count, f->paths, f->diff_rec_of, s.backdrop_len,
                                 f->diff_adj, f->diff_adj_records, line_grad};
-        TK_TRY(tk::launch(ctx, ctx->f_line_backward, div_up(s.line_count, 256), 1, 256, b));
+        TK_TRY(tk::launch(ctx, ctx->f_line_backward, div_up(s.line_count, 32), 1, 256, b));
     }
     // The tile pass replaced the kept coverages with their gradients: another
     // backward needs another forward.
