@@ -577,10 +577,10 @@ __device__ __forceinline__ CoarseCtx coarse_ctx(const tk_args_coarse &a, const S
 }
 
 // What a frame's tile knows of the layers without a look at each: in lane k its class
-// of pair base + k, where the scene's pairs are at most 64, and which of those act on
-// the tile (reject it, wrap it or emit a record).
+// of pair k, where the scene's pairs are at most 64, and which of those act on the
+// tile (reject it, wrap it or emit a record).
 struct TileLayers {
-    uint32_t base, lane_bits;
+    uint32_t lane_bits;
     uint64_t acting;
     bool known;
 };
@@ -1408,7 +1408,7 @@ __device__ uint32_t stack_begins_single_pass(const CoarseCtx &c, uint32_t first,
     const tk_coarse_inputs &in = *c.in;
     const uint32_t i = first + lane;
     uint32_t lane_bits = 0u;
-    if (layers.known) lane_bits = (uint32_t)__shfl((int)layers.lane_bits, (int)(i < end ? c.class_pair_of[i] - layers.base : 0u), 64);
+    if (layers.known) lane_bits = (uint32_t)__shfl((int)layers.lane_bits, (int)(i < end ? c.class_pair_of[i] : 0u), 64);
     bool invalid = false, counted = false, emit = false;
     uint32_t tag = TK_PTCL_BEGIN_CLIP, winding = 0u, fill_rule = 0u, payload = 0u;
     tk_segment_range range{0u, 0u};
@@ -1517,14 +1517,11 @@ __device__ __forceinline__ Particle list_particle(const CoarseCtx &c, const List
     return draw_particle(c, e.batch, e.draw);
 }
 
-__device__ __forceinline__ TileLayers tile_layers(const tk_args_coarse &a, const CoarseCtx &c, const SceneView &v,
-                                                  uint32_t lane) {
-    TileLayers t{0u, 0u, 0ull, false};
-    if (!c.class_row || v.q0 >= v.q1) return t;
-    const uint4 first = a.classes.batch_pairs[v.q0];
-    t.base = uniform(first.z);
-    t.known = uniform(first.w) != 0u;
-    if (t.known && t.base + lane < c.class_pairs) t.lane_bits = c.class_row[t.base + lane];
+__device__ __forceinline__ TileLayers tile_layers(const CoarseCtx &c, uint32_t lane) {
+    TileLayers t{0u, 0ull, false};
+    if (!c.class_row) return t;
+    t.known = c.class_pairs <= 64u;
+    if (t.known && lane < c.class_pairs) t.lane_bits = c.class_row[lane];
     t.acting = __ballot((t.lane_bits & (kLayerInvalid | kLayerCounted | kLayerEmits)) != 0u);
     return t;
 }
@@ -1670,7 +1667,7 @@ __device__ __forceinline__ void coarse_count_tile(const tk_args_coarse &a, uint3
     const uint32_t Q = v.q1;
 
     TileLayers layers{};
-    if constexpr (kFrame) layers = tile_layers(a, c, v, lane);
+    if constexpr (kFrame) layers = tile_layers(c, lane);
     uint32_t next = v.q0;                   // the first batch that no entry has reached
     uint32_t pending = 0u;                  // batches held, one per lane
     uint32_t my_batch = 0u, my_particles = 0u;
@@ -1954,7 +1951,7 @@ __device__ __forceinline__ void coarse_emit_tile(const tk_args_coarse &a, uint32
         if (lane == 0u) kinds[table_index(v, cur)] = kind;
     };
     TileLayers layers{};
-    if constexpr (kFrame) layers = tile_layers(a, c, v, lane);
+    if constexpr (kFrame) layers = tile_layers(c, lane);
     // r and br: the batch's table range and record
     auto begin = [&](uint32_t bb, tk_segment_range r, tk_batch_record br) {
         cur = bb;
@@ -2955,12 +2952,15 @@ TK_DIFF_KERNELS(_scenes_clips, true, true)
 //   -n . (dp0 * int (1 - s) ds + dp1 * int s ds),   n = (p0.y - p1.y, p1.x - p0.x),
 // n pointing to the side where the winding number is one higher.
 //
-// Bound by the two dependent loads of a pixel, so eight lanes share a line, each
-// taking every fourth row and every second column, and a lane looks the record up
-// once per tile.  16,000 lines, 300 paths at 256x256: one thread per line 26 us, four
-// lanes 9.5, eight 5.8; 64 such scenes: 73, 48 and 48.
-constexpr uint32_t kLineRows = 4u, kLineColumns = 2u, kLineLanes = kLineRows * kLineColumns;
-extern "C" __global__ __launch_bounds__(256) void tk_k_line_backward(tk_args_line_backward a) {
+// Bound by the two dependent loads of a pixel, so kLineRows * kLineColumns lanes share
+// a line, every kLineRows-th row and kLineColumns-th column each, and a lane looks the
+// record up once per tile.  16,000 lines, 300 paths at 256x256: one lane a line 26 us,
+// four 9.5, eight 5.8; 64 such scenes: 73, 48 and 48; but 2.1 M lines, which fill the
+// chip by themselves and repeat their set-up in every lane: one 144, eight 181.  So
+// from TK_LINE_LANES_MAX lines on a line has one lane.
+template <uint32_t kLineRows, uint32_t kLineColumns>
+__device__ __forceinline__ void line_backward(const tk_args_line_backward &a) {
+    constexpr uint32_t kLineLanes = kLineRows * kLineColumns;
     const uint32_t i = blockIdx.x * (256u / kLineLanes) + threadIdx.x / kLineLanes;
     const int row_of = (int)(threadIdx.x % kLineRows), column_of = (int)(threadIdx.x / kLineRows % kLineColumns);
     if (i >= a.line_count) return;
@@ -3030,6 +3030,10 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_line_backward(tk_args_lin
     out[1] = -ny * g0;
     out[2] = -nx * g1;
     out[3] = -ny * g1;
+}
+extern "C" __global__ __launch_bounds__(256) void tk_k_line_backward(tk_args_line_backward a) { line_backward<4u, 2u>(a); }
+extern "C" __global__ __launch_bounds__(256) void tk_k_line_backward_many(tk_args_line_backward a) {
+    line_backward<1u, 1u>(a);
 }
 
 // The GPU front end of polygon scenes (tk_frame_set_polygons).

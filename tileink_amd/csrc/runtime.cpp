@@ -80,7 +80,7 @@ struct tk_context {
                   f_draw_tables = nullptr,
                   f_fine = nullptr, f_coarse_count_scenes = nullptr, f_coarse_emit_scenes = nullptr,
                   f_fine_scenes = nullptr, f_fine_diff = nullptr, f_fine_diff_scenes = nullptr,
-                  f_fine_backward = nullptr, f_fine_backward_scenes = nullptr, f_line_backward = nullptr,
+                  f_fine_backward = nullptr, f_fine_backward_scenes = nullptr, f_line_backward = nullptr, f_line_backward_many = nullptr,
                   f_draw_tiles = nullptr, f_fine_diff_clips = nullptr, f_fine_diff_scenes_clips = nullptr,
                   f_fine_backward_clips = nullptr, f_fine_backward_scenes_clips = nullptr,
                   // the same kernels keeping the forward's coverages for the backward
@@ -583,28 +583,15 @@ uint64_t atlas_words(const tk_scene &s) {
     return s.atlas ? uint64_t(s.atlas_width) * s.atlas_height * s.atlas_pages : 0ull;
 }
 
-// tk_layer_classes::batch_pairs of the scene's batches, whose layers' pairs are in
-// host_pair_of.
-void batch_pairs(const tk_frame &f, const tk_scene &s, std::vector<uint4> &out) {
-    const std::vector<uint32_t> &scene_of = f.fe_scene_of_batch_host;
-    const auto scene = [&](uint32_t b) { return b < scene_of.size() ? scene_of[b] : 0u; };
-    const auto layers = [&](uint32_t b, auto body) {
-        for (uint32_t i = s.batches[b].layer_start; i < std::min(s.batches[b].layer_end, s.layer_count); ++i)
-            body(f.host_pair_of[i]);
-    };
-    std::vector<uint32_t> first(std::max<size_t>(f.scene_count, 1), 0xFFFFFFFFu), last(first.size(), 0u);
-    for (uint32_t b = 0; b < s.batch_count; ++b)
-        layers(b, [&](uint32_t pair) {
-            first[scene(b)] = std::min(first[scene(b)], pair);
-            last[scene(b)] = std::max(last[scene(b)], pair);
-        });
+// tk_layer_classes::batch_pairs of the scene's batches, the layers' pairs in `pair_of`.
+void batch_pairs(const tk_scene &s, const std::vector<uint32_t> &pair_of, uint32_t pairs, std::vector<uint4> &out) {
     out.assign(s.batch_count, uint4{0u, 0u, 0u, 0u});
+    if (pairs > 64) return;
     for (uint32_t b = 0; b < s.batch_count; ++b) {
-        const uint32_t base = first[scene(b)] == 0xFFFFFFFFu ? 0u : first[scene(b)];
-        if (last[scene(b)] - base >= 64u && last[scene(b)] >= base) continue;
-        uint64_t pairs = 0;
-        layers(b, [&](uint32_t pair) { pairs |= 1ull << (pair - base); });
-        out[b] = uint4{uint32_t(pairs), uint32_t(pairs >> 32), base, 1u};
+        uint64_t set = 0;
+        for (uint32_t i = s.batches[b].layer_start; i < std::min(s.batches[b].layer_end, s.layer_count); ++i)
+            set |= 1ull << pair_of[i];
+        out[b] = uint4{uint32_t(set), uint32_t(set >> 32), 0u, 1u};
     }
 }
 
@@ -690,7 +677,7 @@ tk_status frame_upload(tk_frame *f, const tk_scene *s) {
         const uint32_t pairs = layer_pairs(s, f->host_pair_of, f->host_pair_layer);
         if (pairs <= f->pair_capacity) {  // else: no table for this scene
             // one buffer, one copy: the batches' pairs, the layers', and the pairs' layers
-            batch_pairs(*f, *s, f->host_batch_pairs);
+            batch_pairs(*s, f->host_pair_of, pairs, f->host_batch_pairs);
             const size_t batches = f->host_batch_pairs.size();
             f->host_batch_pairs.resize(batches + (uint64_t(s->layer_count) + pairs + 3) / 4);
             uint32_t *words = reinterpret_cast<uint32_t *>(f->host_batch_pairs.data() + batches);
@@ -1276,6 +1263,7 @@ tk_status tk_context_create(int device, tk_context **out) {
         {&ctx->f_fine_backward, "tk_k_fine_backward"},
         {&ctx->f_fine_backward_scenes, "tk_k_fine_backward_scenes"},
         {&ctx->f_line_backward, "tk_k_line_backward"},
+        {&ctx->f_line_backward_many, "tk_k_line_backward_many"},
         {&ctx->f_draw_tiles, "tk_k_draw_tiles"},
         {&ctx->f_fine_diff_clips, "tk_k_fine_diff_clips"},
         {&ctx->f_fine_diff_scenes_clips, "tk_k_fine_diff_scenes_clips"},
@@ -2217,7 +2205,9 @@ tk_status tk_frame_backward(tk_frame *f, const float *colors, const float *image
     if (s.line_count) {
         tk_args_line_backward b{f->lines, s.line_count, s.path_count, f->paths, f->diff_rec_of, s.backdrop_len,
                                 f->diff_adj, f->diff_adj_records, line_grad};
-        TK_TRY(tk::launch(ctx, ctx->f_line_backward, div_up(s.line_count, 32), 1, 256, b));
+        const bool many = s.line_count >= TK_LINE_LANES_MAX;
+        TK_TRY(tk::launch(ctx, many ? ctx->f_line_backward_many : ctx->f_line_backward,
+                          div_up(s.line_count, many ? 256 : 32), 1, 256, b));
     }
     // The tile pass replaced the kept coverages with their gradients: another
     // backward needs another forward.
