@@ -555,7 +555,7 @@ class Frame:
 
     def __del__(self):
         h = getattr(self, "_h", None)
-        if h is not None and h.value and not getattr(self, "_borrowed", False):
+        if h is not None and h.value and getattr(self, "_borrowed", None) is None:
             lib().tk_frame_destroy(h)
             self._h = None
 
@@ -702,6 +702,18 @@ class Frame:
         return out
 
 
+class _BatchHandle:
+    """A tk_batch, destroyed with the last of the Batch and its frame: the frame's
+    native handle is the batch's own."""
+
+    def __init__(self, context, handle):
+        self.context, self._h = context, handle
+
+    def __del__(self):
+        if self._h.value:
+            lib().tk_batch_destroy(self._h)
+
+
 class Batch:
     """Independent scenes rendered as one frame (tk_batch_*): `scenes` are encoded
     tk_scene views (Canvas.encode / SceneArrays.to_scene), kept alive by the batch."""
@@ -713,18 +725,13 @@ class Batch:
         h = C.c_void_p()
         check(lib().tk_batch_create(context.handle, arr, len(self._scenes), C.byref(h)))
         self._h = h
+        self._owner = _BatchHandle(context, h)
         self.sizes = [(sc.width, sc.height) for sc in self._scenes]
         frame = Frame.__new__(Frame)
-        frame._borrowed = True
+        frame._borrowed = self._owner
         frame._h = C.c_void_p(lib().tk_batch_frame(h))
         frame.context, frame._scene = context, None
         self.frame = frame  # stats, stage times, timing and graph switches
-
-    def __del__(self):
-        h = getattr(self, "_h", None)
-        if h is not None and h.value:
-            lib().tk_batch_destroy(h)
-            self._h = None
 
     def __len__(self):
         return len(self._scenes)
