@@ -805,7 +805,7 @@ __device__ __forceinline__ uint32_t record_segments(uint32_t start, uint32_t end
 
 // One record of a tile's walk, as scalars.
 struct WalkRecord {
-    uint32_t tag, fill_rule, color, kind;  // kind: the tile kind word's kind of its stream
+    uint32_t tag, fill_rule, color, kind;  // tag: 255 for any larger; kind: the tile kind word's kind of its stream
     uint32_t mark;                         // what mark(kind, tag, color) gave it (0-15)
     int32_t backdrop;
     uint32_t index;                        // its place in the PTCL
@@ -873,7 +873,7 @@ __device__ __forceinline__ void walk_tile(const SceneView &v, const uint32_t *ti
             stale = __builtin_amdgcn_readlane((int)(dead || r.tag == TK_PTCL_END), 63) != 0;
             const uint32_t n =
                 live && covers(my_kind, r.tag, r.color) ? record_segments(r.segment_start, r.segment_end, segment_capacity) : 0u;
-            const uint32_t meta = (r.tag & 0xFFu) | (my_kind << 8) | (r.fill_rule == TK_FILL_EVEN_ODD ? 1u << 16 : 0u) |
+            const uint32_t meta = min(r.tag, 0xFFu) | (my_kind << 8) | (r.fill_rule == TK_FILL_EVEN_ODD ? 1u << 16 : 0u) |
                                   (last || r.tag == TK_PTCL_END ? 1u << 17 : 0u) |
                                   (live ? mark(my_kind, r.tag, r.color) << 18 : 0u);
             uint64_t todo = __ballot(live), fills = __ballot(n != 0u);
