@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import tileink_amd as tk
+from tileink_amd import _abi
 
 import oracle
 
@@ -145,3 +146,47 @@ def test_incremental_render_and_graph_replay_of_shared_rows(ctx):
     for _ in range(3):
         frame.render()
         assert np.array_equal(frame.image(), want)
+
+
+def _many_batches(width, height, clips):
+    """Nothing but rectangles under a clip each, and two triangles: few runs, large tables."""
+    rng = np.random.default_rng(clips)
+    canvas = tk.Canvas(width, height)
+    for _ in range(2):
+        _zigzag(canvas, 3, width, height, rng)
+    for _ in range(clips):
+        x, y = rng.uniform(0, 0.8, 2) * (width, height)
+        canvas.push_clip_sdf_rect_layer(x, y, x + 90, y + 60, 6.0)
+        canvas.push_rect(x - 4, y, x + 70, y + 50, 8.0, tk.Color(*rng.uniform(0, 1, 3), 0.6))
+        canvas.pop_layer()
+        canvas.push_rect(x, y, x + 20, y + 20, 2.0, tk.Color(*rng.uniform(0, 1, 3), 1.0))
+    return canvas
+
+
+# tables cleared by the workgroups of the runs alone, by as many as their words ask for
+# (4096 a workgroup), and by as many as there may be (2048)
+@pytest.mark.parametrize("width,height,clips", [(48, 32, 3), (500, 300, 60), (4096, 4096, 70)])
+def test_tables_of_many_batches_start_cleared(ctx, width, height, clips):
+    arrays = _many_batches(width, height, clips).arrays(0)
+    swapped = tk.SceneArrays.__new__(tk.SceneArrays)
+    swapped.__dict__.update(arrays.__dict__)
+    swapped.lines = arrays.lines.copy()
+    swapped.lines[[2, 3]] = arrays.lines[[3, 2]]  # of two paths: the separate stages, whose tables are cleared in front
+    frame = tk.Frame(ctx, arrays.to_scene())
+    n = frame.batch_count * frame.tiles
+
+    def tables():
+        return [frame.image()] + [frame.buffer(b, np.uint32, n) for b in (_abi.BUF_TILE_PTCL_COUNTS, _abi.BUF_TILE_KINDS)]
+
+    frame.render()
+    first = tables()
+    if n < 20000:
+        assert np.array_equal(first[0], oracle.render_frame(arrays)[0])
+    frame.update(swapped.to_scene())
+    frame.render()
+    for a, b in zip(first, tables()):
+        assert np.array_equal(a, b)
+    frame.update(arrays.to_scene())
+    frame.render()
+    for a, b in zip(first, tables()):
+        assert np.array_equal(a, b)

@@ -629,6 +629,14 @@ uint32_t path_scan_run(const tk_frame *f) {
     return uint32_t(std::min<uint64_t>(run, TK_PATH_SCAN_RUN));
 }
 
+// The launch's workgroups clear the batch tables between them, so it has one for every
+// kPathScanClear words at least, up to kPathScanFillers: a scene of a few draws in many
+// batches has hardly a workgroup of its own.  (No path, 400 batches of 65,536 tiles, 400
+// of 14,400 and 100 of 1,600: 36, 13 and 7 us; by the few workgroups of its draws 1288,
+// 293 and 23.)
+constexpr uint64_t kPathScanClear = 4096;
+constexpr uint32_t kPathScanFillers = 2048;
+
 // Whether tk_k_path_scan takes the scene whose records are in the frame's buffers:
 // *ctx->refused once the stream is idle.
 tk_status path_scan_check(tk_frame *f, const tk_scene &s) {
@@ -953,7 +961,11 @@ tk_status frame_render(tk_frame *f, uint32_t active_count = 0, const DiffTarget 
         for (int k = 0; k < 5; ++k) a.clear[k] = {static_cast<uint32_t *>(clear[k].words), clear[k].count, clear[k].value};
         a.runs = uint32_t(path_scan_positions(s) / a.run) + 1u;
         a.tables = tables;
-        TK_TRY(launch(ctx, ctx->f_path_scan, a.runs + div_up(s.draw_count, 256), 1, 256, a, TK_PATH_SCAN_LDS(a.run)));
+        uint64_t words = 0;
+        for (const tk_table_fill &t : a.clear) words += t.count;
+        const uint32_t fillers = uint32_t(std::min<uint64_t>(div_up(words, kPathScanClear), kPathScanFillers));
+        const uint32_t blocks = std::max(a.runs + div_up(s.draw_count, 256), fillers);
+        TK_TRY(launch(ctx, ctx->f_path_scan, blocks, 1, 256, a, TK_PATH_SCAN_LDS(a.run)));
         for (int mark : {2, 3, 4, 5, 6}) TK_TRY(record(f, mark));
         TK_TRY(coarse());
     } else {
