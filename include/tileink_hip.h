@@ -592,7 +592,8 @@ typedef struct tk_frame_stats {
     uint32_t segments_emitted;                      /* S after the last render */
     uint32_t overflow;                              /* nonzero when a bound was exceeded */
     uint64_t device_bytes;                          /* device memory held by the frame */
-    uint32_t scan_chunk_count, cumsum_chunk_count, cumsum_row_count, pad;
+    uint32_t scan_chunk_count, cumsum_chunk_count, cumsum_row_count;
+    uint32_t one_kernel_scan;                       /* 1: later renders scan in one kernel, 0: in separate stages */
     uint64_t ptcl_bound;                            /* the scene's PTCL bound (<= ptcl_capacity) */
 } tk_frame_stats;
 /* Synchronises; ptcl_records / segments_emitted / overflow come from the device. */

@@ -126,7 +126,7 @@ class FrameStats(C.Structure):
         ("ptcl_capacity", C.c_uint64), ("ptcl_records", C.c_uint64), ("segments_emitted", C.c_uint32),
         ("overflow", C.c_uint32), ("device_bytes", C.c_uint64),
         ("scan_chunk_count", C.c_uint32), ("cumsum_chunk_count", C.c_uint32), ("cumsum_row_count", C.c_uint32),
-        ("pad", C.c_uint32), ("ptcl_bound", C.c_uint64)]
+        ("one_kernel_scan", C.c_uint32), ("ptcl_bound", C.c_uint64)]
 
 
 class StageTimes(C.Structure):

@@ -21,6 +21,7 @@
 // integer rules.
 
 #include "flatten.h"
+#include "path_scan_rule.h"
 #include "scan_line.h"
 
 namespace {
@@ -140,7 +141,6 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_fe_paths(tk_args_frontend
     }
     capacity = fe_wave_sum_u64(capacity);
     if (lane != 0u) return;
-    if (lines > TK_PATH_SCAN_LINES) atomicOr(a.status, 4u);  // scanned by the separate stages
     const uint32_t stride = tb[2] > tb[0] ? tb[2] - tb[0] : 0u, height = tb[3] > tb[1] ? tb[3] - tb[1] : 0u;
     const uint32_t data_len = stride * height;
     const uint32_t rows = stride && height ? height : 0u;
@@ -148,6 +148,12 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_fe_paths(tk_args_frontend
     a.path_vals[TK_FE_LINES * P + p] = lines;
     a.path_vals[TK_FE_BACKDROPS * P + p] = data_len;
     a.path_vals[TK_FE_SEGMENTS * P + p] = capacity > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)capacity;
+    const uint32_t visits = a.path_vals[TK_FE_SEGMENTS * P + p];
+    if (const uint32_t excess = tk::path_scan_excess(lines, visits, data_len))
+        atomicMax(&a.totals[TK_FE_SCAN_EXCESS], (unsigned long long)excess);
+    if (const uint64_t shared = tk::path_scan_shared(lines, visits, data_len))
+        atomicAdd(&a.totals[TK_FE_SCAN_SHARED], (unsigned long long)shared);
+    if (lines > TK_PATH_SCAN_LINES) atomicOr(a.status, 4u);  // scanned by the separate stages
     a.path_vals[TK_FE_SCAN_CHUNKS * P + p] = (data_len + TK_SCAN_CHUNK_SIZE - 1u) / TK_SCAN_CHUNK_SIZE;
     a.path_vals[TK_FE_CUMSUM_ROWS * P + p] = rows;
     a.path_vals[TK_FE_CUMSUM_CHUNKS * P + p] = rows * ((stride + TK_CUMSUM_CHUNK_SIZE - 1u) / TK_CUMSUM_CHUNK_SIZE);
@@ -161,7 +167,7 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_fe_paths(tk_args_frontend
     r.tile_y0 = tb[1];
     r.tile_x1 = tb[2];
     r.tile_y1 = tb[3];
-    r.segment_capacity = a.path_vals[TK_FE_SEGMENTS * P + p];
+    r.segment_capacity = visits;
     r.segment_count = 0u;
     r.transform = tk_affine{1.0f, 0.0f, 0.0f, 1.0f, 0.0f, 0.0f};
     a.paths[p] = r;  // line_start, data_offset and segment_start follow the scan

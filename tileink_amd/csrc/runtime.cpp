@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "tk_internal.h"
+#include "path_scan_rule.h"
 #include "tk_kernel_args.h"
 
 extern "C" const unsigned char tk_code_object_begin[];
@@ -637,6 +638,17 @@ uint32_t path_scan_run(const tk_frame *f) {
 constexpr uint64_t kPathScanClear = 4096;
 constexpr uint32_t kPathScanFillers = 2048;
 
+// path_scan_rule.h's, of the scene's path records.
+bool scene_scan_pays(const tk_scene &s) {
+    uint64_t excess = 0, shared = 0;
+    for (uint32_t i = 0; i < s.path_count; ++i) {
+        const tk_path_record &p = s.paths[i];
+        excess = std::max<uint64_t>(excess, path_scan_excess(p.line_count, p.segment_capacity, p.data_len));
+        shared += path_scan_shared(p.line_count, p.segment_capacity, p.data_len);
+    }
+    return path_scan_pays(s.line_count, excess, shared);
+}
+
 // Whether tk_k_path_scan takes the scene whose records are in the frame's buffers:
 // *ctx->refused once the stream is idle.
 tk_status path_scan_check(tk_frame *f, const tk_scene &s) {
@@ -679,7 +691,8 @@ tk_status frame_upload(tk_frame *f, const tk_scene *s) {
     TK_TRY(upload(f, f->cs_lens, s->cumsum_chunk_lens, s->cumsum_chunk_count));
     TK_TRY(upload(f, f->cs_row_starts, s->cumsum_row_starts, s->cumsum_row_count));
     TK_TRY(upload(f, f->cs_row_ends, s->cumsum_row_ends, s->cumsum_row_count));
-    TK_TRY(path_scan_check(f, *s));
+    const bool pays = scene_scan_pays(*s);
+    if (pays) TK_TRY(path_scan_check(f, *s));
     f->pair_count = 0;
     if (f->layer_bits && s->layer_count && s->layers) {
         const uint32_t pairs = layer_pairs(s, f->host_pair_of, f->host_pair_layer);
@@ -698,7 +711,7 @@ tk_status frame_upload(tk_frame *f, const tk_scene *s) {
         }
     }
     TK_HIP(hipStreamSynchronize(f->ctx->stream));
-    f->path_scan = *f->ctx->refused == 0u;
+    f->path_scan = pays && *f->ctx->refused == 0u;
     return TK_OK;
 }
 
@@ -1680,11 +1693,12 @@ tk_status frame_set_geometry(tk_frame *f, const FeInput &in) {
     s.tile_draw_index_count = uint32_t(t[TK_FE_TILE_REFS]);
     s.ptcl_capacity = t[TK_FE_PTCL];
     f->diff_ready = false;
-    // The front end lays paths out as the one-kernel scan takes them, unless one is too
-    // long (status bit 2) or too wide for it.
+    // The front end lays paths out as the one-kernel scan takes them, unless one has too
+    // many lines (status bit 2) or is too wide for it.
     uint32_t highest = 0;
     for (const tk_fe_scene &scene : f->fe_scenes_host) highest = std::max(highest, scene.tiles_height);
-    f->path_scan = !(flags & 4u) && frame_tiles_width(f) <= TK_PATH_SCAN_RUN && highest <= 0xFFFFu;
+    f->path_scan = !(flags & 4u) && frame_tiles_width(f) <= TK_PATH_SCAN_RUN && highest <= 0xFFFFu &&
+                   path_scan_pays(lines, t[TK_FE_SCAN_EXCESS], t[TK_FE_SCAN_SHARED]);
     return TK_OK;
 }
 
@@ -2449,6 +2463,7 @@ tk_status tk_frame_stats_read(tk_frame *f, tk_frame_stats *out) {
     out->scan_chunk_count = s.scan_chunk_count;
     out->cumsum_chunk_count = s.cumsum_chunk_count;
     out->cumsum_row_count = s.cumsum_row_count;
+    out->one_kernel_scan = f->path_scan ? 1u : 0u;
     out->ptcl_records = status[1];
     out->overflow = status[0] | (status[3] << 1) | (status[1] > f->ptcl_capacity ? 4u : 0u) | (status[2] << 4);
     uint32_t emitted = 0;

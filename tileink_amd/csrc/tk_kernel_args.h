@@ -150,7 +150,7 @@ struct tk_args_draw_tables {
 // The scan of a frame laid out path by path, in one kernel (pathscan.hip).
 #define TK_PATH_SCAN_RUN 928u      // lines, tiles and paths (four each) per run, at most
 #define TK_PATH_SCAN_LDS(run) (16u * (((run) + 3u) / 4u) + 24u * (run) + 4u)  // bytes of LDS for a run's tables
-#define TK_PATH_SCAN_LINES 8192u   // lines of the longest path it takes
+#define TK_PATH_SCAN_LINES 64512u  // lines of the longest path it takes: its queues number them in 16 bits
 struct tk_args_path_scan {
     tk_scan_config cfg;
     const tk_line *lines;
@@ -336,7 +336,9 @@ enum tk_fe_total : uint32_t {
     TK_FE_TILE_REFS = 6,
     TK_FE_ROW_ENTRIES = 7,
     TK_FE_PTCL = 8,
-    TK_FE_TOTALS = 9,
+    TK_FE_SCAN_EXCESS = 9,   // the largest path_scan_excess
+    TK_FE_SCAN_SHARED = 10,  // the sum of path_scan_shared
+    TK_FE_TOTALS = 11,
 };
 
 struct tk_args_frontend {
