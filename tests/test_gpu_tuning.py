@@ -141,3 +141,90 @@ def test_invalid_run_lengths_are_rejected(ctx):
             frame.set_tuning(**bad)
         assert err.value.status == _abi.TK_ERR_INVALID, bad
     assert frame.tuning() == before
+
+
+# The scan parameters are of the separate stages, which a frame runs whose lines do not
+# lie path by path; recorded scenes scan in one kernel and do not read them.
+
+
+def _by_stages(arrays):
+    """The scene with its lines in another order."""
+    out = tk.SceneArrays.__new__(tk.SceneArrays)
+    out.__dict__.update(arrays.__dict__)
+    out.lines = arrays.lines[np.random.default_rng(4).permutation(len(arrays.lines))].copy()
+    return out
+
+
+STAGE_SHAPES = [(0, 64, 4, 4096), (0, 128, 4, 4096), (0, 256, 4, 4096), (0, 512, 4, 4096), (0, 1024, 4, 4096)] + SHAPES
+
+
+@pytest.mark.parametrize("scene", ["clipped", "mixed"])
+def test_separate_scan_stages_render_the_same_frame_at_every_block_size(ctx, scene):
+    canvas = scenes.clipped_paths_small(8) if scene == "clipped" else scenes.mixed_scene_640x360()
+    arrays = canvas.arrays(0)
+    frame = tk.Frame(ctx, arrays.to_scene())
+    frame.render()
+    assert frame.stats()["one_kernel_scan"] == 1
+    ref = frame_tables(frame)
+    T = arrays.tiles_width * arrays.tiles_height
+    shuffled = _by_stages(arrays)
+    stages = tk.Frame(ctx, shuffled.to_scene())
+    for shape in STAGE_SHAPES:
+        for run in (0, 1, 16, 1024):
+            shaped(stages, shape, (run, 64, 256))
+            stages.render()
+            got = frame_tables(stages)
+            for name, a, b in zip(("image", "kinds", "ranges", "ptcl"), got, ref):
+                assert np.array_equal(a, b), (shape, run, name)
+            stats = stages.stats()
+            assert stats["overflow"] == 0 and stats["one_kernel_scan"] == 0
+        stages.render_tiles(np.random.default_rng(3).permutation(T)[: T // 3])
+        assert np.array_equal(stages.image(), ref[0]), shape
+    stages.set_graph(True)
+    for k, shape in enumerate(STAGE_SHAPES):
+        shaped(stages, shape)
+        for _ in range(2):
+            stages.render()
+            assert np.array_equal(stages.image(), ref[0]), shape
+        if k % 3 == 0:
+            stages.render_tiles(np.arange(0, T, 5))
+    stages.set_graph(False)
+    chosen = stages.autotune(repeats=1)
+    assert chosen == stages.tuning()
+    stages.render()
+    assert np.array_equal(stages.image(), ref[0])
+
+
+def test_separate_scan_stages_in_batches_and_set_polygons(ctx):
+    canvases = [scenes.scene_set_member(w, h, n, i) for i, (w, h, n) in
+                enumerate([(96, 64, 40), (300, 140, 120), (700, 333, 900)])]
+    arrays = [c.arrays(0) for c in canvases]
+    ref = tk.Batch(ctx, [a.to_scene() for a in arrays])
+    ref.render()
+    assert ref.frame.stats()["one_kernel_scan"] == 1
+    shuffled = [_by_stages(a) for a in arrays]
+    batch = tk.Batch(ctx, [a.to_scene() for a in shuffled])
+    for shape in STAGE_SHAPES:
+        shaped(batch.frame, shape)
+        for graph in (False, True):
+            batch.frame.set_graph(graph)
+            for _ in range(1 + graph):
+                batch.render()
+                for i in range(len(canvases)):
+                    assert np.array_equal(batch.image(i), ref.image(i)), (shape, graph, i)
+    assert batch.frame.stats()["one_kernel_scan"] == 0
+
+    rng = np.random.default_rng(6)  # a path whose visits outweigh its lines: the front end's frames by stages
+    polys = [rng.uniform(1, 199, (n, 2)).astype(np.float32) for n in (3000, 20)]
+    canvas = tk.Canvas(200, 200)
+    for p in polys:
+        canvas.push_polygon(p.astype(np.float64), tk.Color(0.3, 0.5, 0.9, 0.5), rule=tk.FillRule.EvenOdd)
+    frame = tk.Frame(ctx, canvas.encode(0))
+    frame.set_polygons(np.concatenate(polys), np.array([0, 3000, 3020], np.uint32))
+    frame.render()
+    image = frame.image()
+    assert frame.stats()["one_kernel_scan"] == 0
+    for shape in STAGE_SHAPES:
+        shaped(frame, shape)
+        frame.render()
+        assert np.array_equal(frame.image(), image), shape
