@@ -560,8 +560,8 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_clear(tk_args_clear a) {
 //
 // Bound by the chain of FP64 divisions and roots along a cubic.  Eight lanes take a
 // path, a cubic each in turn, since a path has few; pass 2 counts a cubic again before
-// it writes it, to place it behind its neighbours.  One thread per path: 94 waves for
-// 6000 paths of six cubics, 119 us a pass; eight: 26 and 47 us.
+// it writes it, to place it behind its neighbours (one alone has none).  One thread per
+// path: 94 waves for 6000 paths of six cubics, 119 us a pass; eight: 26 and 47 us.
 constexpr uint32_t kFlattenLanes = 8u;
 __device__ __forceinline__ bool fl_contour(const tk_args_flatten &a, uint32_t p, uint32_t &first, uint32_t &cubics) {
     first = a.starts[p];
@@ -658,7 +658,7 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_flatten_emit(tk_args_flat
         tk::FPt q[4];
         const bool mine = fl_cubic(c, cubics, base + member, q);
         uint32_t count = 0u;
-        if (mine) tk::flatten_cubic(q[0], q[1], q[2], q[3], a.tolerance, [&](tk::FPt) { ++count; });
+        if (mine && cubics > 1u) tk::flatten_cubic(q[0], q[1], q[2], q[3], a.tolerance, [&](tk::FPt) { ++count; });
         uint32_t upto = count;
         for (uint32_t off = 1u; off < kFlattenLanes; off <<= 1) {
             const uint32_t below = (uint32_t)__shfl_up((int)upto, off, kFlattenLanes);
