@@ -54,3 +54,27 @@ def test_contours_of_any_number_of_cubics_flatten_like_the_recorder(ctx):
         frame.render()
         ref.render()
         assert np.array_equal(frame.image(), ref.image())
+
+
+@pytest.mark.parametrize("paths", [11264, 11265])  # the flattener's table alone: one workgroup, three launches
+def test_flattened_tables_of_either_scan(ctx, paths):
+    rng = np.random.default_rng(paths)
+    ctrl = rng.uniform(2, 118, (paths, 1, 2)) + rng.uniform(-4, 4, (paths, 7, 2))
+    ctrl[:, 6] = ctrl[:, 0]
+    ctrl[::5, 3] = ctrl[::5, 0]  # curves of another number of lines
+
+    def record():
+        canvas = tk.Canvas(120, 120)
+        for c in ctrl:
+            path = tk.BezPath().move_to(*c[0]).curve_to(*c[1:4].reshape(-1)).curve_to(*c[4:7].reshape(-1))
+            canvas.push_path(path.close_path(), tk.Color(0.3, 0.6, 0.2, 0.1))
+        return canvas.encode(0)
+
+    scene = record()
+    frame = tk.Frame(ctx, scene)
+    want = scene_arrays(frame)
+    ctrl += 1.0
+    frame.set_cubic_paths(ctrl.reshape(-1, 2), np.arange(paths + 1, dtype=np.uint32) * 7)
+    ctrl -= 1.0
+    frame.set_cubic_paths(ctrl.reshape(-1, 2), np.arange(paths + 1, dtype=np.uint32) * 7)
+    assert_same_scene(scene_arrays(frame), want)

@@ -1512,8 +1512,10 @@ tk_status fe_prepare(tk_frame *f) {
 
 // In-place exclusive scans of the front end's tables (at most eight columns).  The
 // columns of up to TK_FE_SHORT_SCAN values share one launch, a workgroup each; the
-// others take three launches a table.  (Three launches are 13.5 us; a workgroup
-// starts in 4 us and scans 2048 values in 1.5, 6000 in 8.5: even at that length.)
+// others take three launches a table.  A table alone is even earlier, as nothing shares
+// the launch.  (One table of 4,000, 8,000, 12,000 and 16,000 values by its workgroup 6,
+// 10.4, 15.1 and 19.5 us, by three launches 14-17; three tables of 6,000 and 16,000
+// together 30 and 20 us, by nine launches 110 and 95.)
 struct FeTable {
     uint32_t *values;
     uint32_t count, columns;
@@ -1523,8 +1525,9 @@ tk_status fe_scan(tk_context *ctx, tk_frame *f, std::initializer_list<FeTable> t
     tk_args_fe_scan_short s{};
     s.overflow = f->fe_status + 1;
     uint32_t n = 0;
+    const uint32_t longest = tables.size() > 1 ? TK_FE_SHORT_SCAN : TK_FE_SHORT_SCAN_ALONE;
     for (const FeTable &t : tables) {
-        if (t.count <= TK_FE_SHORT_SCAN) {
+        if (t.count <= longest) {
             for (uint32_t c = 0; c < t.columns; ++c)
                 s.columns[n++] = {t.values + uint64_t(c) * t.count, t.count, t.totals + c};
             continue;

@@ -396,6 +396,7 @@ struct tk_args_fe_scan {
 
 // The same of up to eight columns of their own lengths, each by one workgroup.
 #define TK_FE_SHORT_SCAN 16384u
+#define TK_FE_SHORT_SCAN_ALONE 11264u
 struct tk_args_fe_scan_short {
     struct {
         uint32_t *values;
