@@ -1552,7 +1552,7 @@ __device__ __forceinline__ ChunkRuns chunk_runs(const tk_args_coarse &a, const T
     if (a.cfg.layer_count && lane < n) {
         acts = true;
         if (t.known) {
-            const uint4 pairs = a.classes.batch_pairs[b];
+            const uint2 pairs = a.classes.batch_pairs[b];
             acts = ((((uint64_t)pairs.y << 32) | pairs.x) & t.acting) != 0ull;
         }
     }

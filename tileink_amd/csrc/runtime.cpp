@@ -301,7 +301,7 @@ struct LayerClassPlan {
     const uint32_t *pair_layer = nullptr, *pair_of = nullptr;
     uint32_t pair_count = 0;
     uint8_t *bits = nullptr;
-    const uint4 *batch_pairs = nullptr;
+    const uint2 *batch_pairs = nullptr;
 };
 
 tk_status run_coarse(tk_context *ctx, const tk_coarse_config &cfg, const tk_coarse_inputs &in,
@@ -426,9 +426,9 @@ struct tk_frame {
     uint32_t *layer_pair_of = nullptr, *pair_layer = nullptr;
     uint8_t *layer_bits = nullptr;
     uint32_t pair_capacity = 0, pair_count = 0;
-    uint4 *batch_pairs = nullptr;  // with layer_pair_of and pair_layer behind it
+    uint2 *batch_pairs = nullptr;  // with layer_pair_of and pair_layer behind it
     std::vector<uint32_t> host_pair_of, host_pair_layer;
-    std::vector<uint4> host_batch_pairs;
+    std::vector<uint2> host_batch_pairs;
     // incremental renders: the listed tiles, the damage summed-area table, per-path flags
     uint32_t *active_tiles = nullptr, *damage_sat = nullptr, *path_active = nullptr;
     std::vector<uint32_t> host_active, host_sat;
@@ -585,14 +585,14 @@ uint64_t atlas_words(const tk_scene &s) {
 }
 
 // tk_layer_classes::batch_pairs of the scene's batches, the layers' pairs in `pair_of`.
-void batch_pairs(const tk_scene &s, const std::vector<uint32_t> &pair_of, uint32_t pairs, std::vector<uint4> &out) {
-    out.assign(s.batch_count, uint4{0u, 0u, 0u, 0u});
+void batch_pairs(const tk_scene &s, const std::vector<uint32_t> &pair_of, uint32_t pairs, std::vector<uint2> &out) {
+    out.assign(s.batch_count, uint2{0u, 0u});
     if (pairs > 64) return;
     for (uint32_t b = 0; b < s.batch_count; ++b) {
         uint64_t set = 0;
         for (uint32_t i = s.batches[b].layer_start; i < std::min(s.batches[b].layer_end, s.layer_count); ++i)
             set |= 1ull << pair_of[i];
-        out[b] = uint4{uint32_t(set), uint32_t(set >> 32), 0u, 1u};
+        out[b] = uint2{uint32_t(set), uint32_t(set >> 32)};
     }
 }
 
@@ -700,7 +700,7 @@ tk_status frame_upload(tk_frame *f, const tk_scene *s) {
             // one buffer, one copy: the batches' pairs, the layers', and the pairs' layers
             batch_pairs(*s, f->host_pair_of, pairs, f->host_batch_pairs);
             const size_t batches = f->host_batch_pairs.size();
-            f->host_batch_pairs.resize(batches + (uint64_t(s->layer_count) + pairs + 3) / 4);
+            f->host_batch_pairs.resize(batches + (uint64_t(s->layer_count) + pairs + 1) / 2);
             uint32_t *words = reinterpret_cast<uint32_t *>(f->host_batch_pairs.data() + batches);
             std::copy(f->host_pair_of.begin(), f->host_pair_of.end(), words);
             std::copy(f->host_pair_layer.begin(), f->host_pair_layer.end(), words + s->layer_count);
@@ -1162,7 +1162,7 @@ tk_status frame_create(tk_context *ctx, const tk_scene *s, const BatchLayout *ba
         std::vector<uint32_t> pair_of, pair_layer;
         const uint64_t pairs = layer_pairs(s, pair_of, pair_layer);
         if (pairs * T <= kMaxLayerClassBytes) {
-            ALLOC(batch_pairs, s->batch_count + (uint64_t(s->layer_count) + pairs + 3) / 4);
+            ALLOC(batch_pairs, s->batch_count + (uint64_t(s->layer_count) + pairs + 1) / 2);
             ALLOC(layer_bits, pairs * T);
             f->pair_capacity = uint32_t(pairs);
         }

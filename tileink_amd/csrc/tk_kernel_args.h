@@ -201,9 +201,9 @@ struct tk_layer_classes {
     const uint8_t *bits;        // columns * pair_count (one row of pair_count bytes per table column)
     const uint32_t *pair_of;    // per layer record: its pair
     uint32_t pair_count;
-    // Per batch {the set of its layers' pairs, low and high word, 0, 1}; zeros when the
-    // scene has more than 64 pairs.
-    const uint4 *batch_pairs;
+    // Per batch the set of its layers' pairs {low, high word}; zeros when the scene has
+    // more than 64 pairs.
+    const uint2 *batch_pairs;
 };
 
 struct tk_args_coarse {
@@ -289,7 +289,7 @@ struct tk_args_fine_diff {
     uint32_t xcd_run;           // as tk_args_fine
 };
 
-#define TK_LINE_LANES_MAX (1u << 20)  // lines up to which eight lanes share one
+#define TK_LINE_LANES_MAX (1u << 20)  // below this many lines eight lanes share one
 struct tk_args_line_backward {
     const tk_line *lines;
     uint32_t line_count, path_count;
