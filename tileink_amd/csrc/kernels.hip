@@ -806,7 +806,7 @@ __device__ __forceinline__ uint32_t record_segments(uint32_t start, uint32_t end
 // One record of a tile's walk, as scalars.
 struct WalkRecord {
     uint32_t tag, fill_rule, color, kind;  // tag: 255 for any larger; kind: the tile kind word's kind of its stream
-    uint32_t mark;                         // what mark(kind, tag, color) gave it (0-15)
+    uint32_t mark;                         // what mark(kind, tag, color) gave it (14 bits)
     int32_t backdrop;
     uint32_t index;                        // its place in the PTCL
     bool covered;                          // its coverage has segments, summed in `d`
@@ -821,8 +821,10 @@ struct WalkRecord {
 // every wave holds a window of 64 consecutive records, one per lane, and reads
 // what steers the walk with v_readlane.  The workgroup's waves hold the same
 // window, so control flow and barriers are the workgroup's.  mark(kind, tag, color)
-// looks at a record by lane, so that a gather answers for 64 of them.
-template <class Covers, class Mark, class Visit>
+// looks at a record by lane, so that a gather answers for 64 of them.  kPlain: a canvas of
+// one batch has one stream, which needs no search (65,536 tiles of one colour 144 -> 134
+// us; the builds for many scenes lose 1 % to the test).
+template <bool kPlain, class Covers, class Mark, class Visit>
 __device__ __forceinline__ void walk_tile(const SceneView &v, const uint32_t *tile_kinds,
                                           const tk_segment_range *tile_ranges, const tk_ptcl_record *ptcl,
                                           uint32_t ptcl_capacity, const tk_line_segment *segs,
@@ -851,10 +853,12 @@ __device__ __forceinline__ void walk_tile(const SceneView &v, const uint32_t *ti
             // Lane r takes record w0 + r: its stream is the first that ends past it.
             const uint32_t at = w0 + lane;
             uint32_t j = 0u;
+            if (!kPlain || q1 - b0 > 1u) {
 #pragma unroll
-            for (uint32_t step = 32u; step >= 1u; step >>= 1)
-                if (lane_value(upto, j + step - 1u) <= at) j += step;
-            j = min(j, 63u);
+                for (uint32_t step = 32u; step >= 1u; step >>= 1)
+                    if (lane_value(upto, j + step - 1u) <= at) j += step;
+                j = min(j, 63u);
+            }
             const uint32_t end_at = lane_value(upto, j);
             uint32_t my_kind = TK_TILE_KIND_EMPTY, index = 0u, off = 0u;
             tk_ptcl_record r{};
@@ -2186,7 +2190,7 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_draw_tables(tk_args_draw_
 }
 
 // Marks of fine's walk.
-constexpr uint32_t kFlatTranslucent = 1u, kFlatOpaque = 2u;
+constexpr uint32_t kFlat = 1u << 13, kFlatOpaque = kFlat + 1u, kWholeColor = 1u;
 
 // fine_tile_main for every batch: one 256-lane workgroup per tile, one lane per
 // pixel.  Between batches the pixel goes through the RGBA8 store/load round trip
@@ -2271,15 +2275,26 @@ __device__ __forceinline__ void fine_tile(const tk_args_fine &a) {
                 pixel = over;
             }
         };
+        // A colour over the whole tile, in a stream without clips and coverage (COLOR tiles
+        // hold nothing else, SDF and MIXED tiles some: fine/specialized.hlsli:19-111).  Marked by
+        // lane, since paint_record, which would do the same, took three times as long: 100
+        // translucent rectangles over 2048x2048 1120 -> 386 us, 5,000 rounded ones on 1920x1920
+        // 850 -> 572.
+        const auto paint_color = [&](uint32_t color) {
+            const Px src = rgba8_to_unorm(color);
+            if (premul_opaque(color)) {
+                pixel = src;
+            } else if ((color >> 24) != 0u) {
+                const float inv = 1.0f - src.a;
+                pixel = Px{src.r + pixel.r * inv, src.g + pixel.g * inv, src.b + pixel.b * inv, src.a + pixel.a * inv};
+            }
+        };
         const auto paint_record = [&](const WalkRecord &rec) {
-            // COLOR tiles hold colour records only; SDF and MIXED tiles colours, images
-            // and solid SDF rectangles (fine/specialized.hlsli:19-111): no clips, no coverage.
+            // SDF and MIXED tiles hold, beside the colours that paint_color takes, images and
+            // solid SDF rectangles (fine/specialized.hlsli:19-111): no clips, no coverage.
             const bool special = rec.kind != TK_TILE_KIND_INTERPRETER;
             uint32_t tag = rec.tag;
-            if (special) {
-                if (rec.kind == TK_TILE_KIND_COLOR) tag = TK_PTCL_COLOR;
-                else if (tag != TK_PTCL_COLOR && tag != kPtclImage) tag = TK_PTCL_SDF;
-            }
+            if (special && tag != kPtclImage) tag = TK_PTCL_SDF;
             // What the record draws: a colour every pixel shares (flat, its bytes as
             // floats in flat_*) or its draw's brush, under `masked` (0-255).
             uint32_t masked = clip_mask, color = rec.color;
@@ -2344,7 +2359,7 @@ __device__ __forceinline__ void fine_tile(const tk_args_fine &a) {
                 flat_b = asfloat(entry[6]);
                 flat_a = asfloat(entry[7]);
             }
-            // In a special tile a colour or image is not scaled by a coverage.
+            // In a special tile an image is not scaled by a coverage.
             const bool whole = special && tag != TK_PTCL_SDF;
             if (flat && tag != kPtclPathGlyph) {
                 if ((color >> 24) != 0u && masked != 0u) {
@@ -2370,20 +2385,25 @@ __device__ __forceinline__ void fine_tile(const tk_args_fine &a) {
                                                                : scale_premul_u8_to_unorm(color, masked));
             }
         };
-        walk_tile(v, a.in.tile_kinds, a.in.tile_ptcl_ranges, a.in.ptcl, cfg.ptcl_capacity, a.in.segments,
+        walk_tile<!kScenes>(v, a.in.tile_kinds, a.in.tile_ptcl_ranges, a.in.ptcl, cfg.ptcl_capacity, a.in.segments,
                   cfg.segment_capacity, cov_acc, acc_sel,
                   [](uint32_t kind, uint32_t tag, uint32_t) {
                       return kind == TK_TILE_KIND_INTERPRETER && is_coverage_tag(tag);
                   },
                   [&](uint32_t kind, uint32_t tag, uint32_t color) -> uint32_t {
-                      if (kind != TK_TILE_KIND_INTERPRETER || tag != TK_PTCL_FILL || color >= cfg.draw_count) return 0u;
+                      if (kind != TK_TILE_KIND_INTERPRETER)
+                          return tag != TK_PTCL_END && (kind == TK_TILE_KIND_COLOR || tag == TK_PTCL_COLOR) ? kWholeColor : 0u;
+                      if (tag != TK_PTCL_FILL || color >= cfg.draw_count) return 0u;
                       const uint2 entry = *reinterpret_cast<const uint2 *>(a.draw_brush + (size_t)color * TK_DRAW_BRUSH_WORDS);
                       if (entry.x == 0u || (entry.y >> 24) == 0u) return 0u;
-                      return premul_opaque(entry.y) ? kFlatOpaque : kFlatTranslucent;
+                      return premul_opaque(entry.y) ? kFlatOpaque : kFlat;
                   },
                   [&](const WalkRecord &rec) {
-                      if (__builtin_expect(rec.mark != 0u, 1)) paint_flat_fill(rec);
-                      else if (rec.tag != TK_PTCL_END) paint_record(rec);
+                      if (__builtin_expect((rec.mark & kFlat) != 0u, 1)) paint_flat_fill(rec);
+                      else if (rec.tag != TK_PTCL_END) {
+                          if (rec.mark != 0u) paint_color(rec.color);
+                          else paint_record(rec);
+                      }
                       if (rec.ends) {
                           pixel = Px{quantized_channel(pixel.r), quantized_channel(pixel.g), quantized_channel(pixel.b),
                                      quantized_channel(pixel.a)};
@@ -2734,7 +2754,7 @@ __device__ __forceinline__ void for_each_fill(const tk_args_fine_diff &a, const 
         return ((tag == TK_PTCL_FILL) & (color < cfg.draw_count)) | (kClips & (tag == TK_PTCL_BEGIN_CLIP));
     };
     ClipMask clip{1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 0u};
-    walk_tile(t.v, a.in.tile_kinds, a.in.tile_ptcl_ranges, a.in.ptcl, cfg.ptcl_capacity, a.in.segments,
+    walk_tile<false>(t.v, a.in.tile_kinds, a.in.tile_ptcl_ranges, a.in.ptcl, cfg.ptcl_capacity, a.in.segments,
               cfg.segment_capacity, cov_acc, sel, covers, [](uint32_t, uint32_t, uint32_t) { return 0u; },
               [&](const WalkRecord &rec) {
                   if (rec.tag != TK_PTCL_END) {
