@@ -806,7 +806,7 @@ __device__ __forceinline__ uint32_t record_segments(uint32_t start, uint32_t end
 // One record of a tile's walk, as scalars.
 struct WalkRecord {
     uint32_t tag, fill_rule, color, kind;  // tag: 255 for any larger; kind: the tile kind word's kind of its stream
-    uint32_t mark;                         // what mark(kind, tag, color) gave it (14 bits)
+    uint32_t mark;                         // what mark(kind, tag, color) gave it (0-15)
     int32_t backdrop;
     uint32_t index;                        // its place in the PTCL
     bool covered;                          // its coverage has segments, summed in `d`
@@ -2190,7 +2190,7 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_draw_tables(tk_args_draw_
 }
 
 // Marks of fine's walk.
-constexpr uint32_t kFlat = 1u << 13, kFlatOpaque = kFlat + 1u, kWholeColor = 1u;
+constexpr uint32_t kFlat = 2u, kFlatOpaque = 3u, kWholeColor = 1u;
 
 // fine_tile_main for every batch: one 256-lane workgroup per tile, one lane per
 // pixel.  Between batches the pixel goes through the RGBA8 store/load round trip
