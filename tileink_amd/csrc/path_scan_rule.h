@@ -1,6 +1,6 @@
 // What the one-kernel scan (pathscan.hip) costs a path beyond its share, which decides
-// whether a frame takes it: added up on the host for an upload, on the device by the
-// front end.  `visits` is the path's segment capacity, the tiles its lines visit.
+// whether a frame takes it: at an upload by the host and tk_k_path_scan_check, else by
+// the front end.  `visits` is the path's segment capacity, the tiles its lines visit.
 #pragma once
 
 #include "scan_line.h"
@@ -26,9 +26,9 @@ TK_HD inline uint32_t path_scan_excess(uint32_t lines, uint32_t visits, uint32_t
 
 // A path of more tiles than two runs is shared by several workgroups, each of which takes
 // all its lines: those workgroups, by their lines and visits over a fixed part.
+constexpr uint32_t kPathScanSharedTiles = 1280u;
 TK_HD inline uint64_t path_scan_shared(uint32_t lines, uint32_t visits, uint32_t tiles) {
-    constexpr uint32_t run = 640u;
-    return tiles > 2u * run ? uint64_t(tiles / run) * (8192ull + lines + visits) : 0ull;
+    return tiles > kPathScanSharedTiles ? uint64_t(tiles / (kPathScanSharedTiles / 2u)) * (8192ull + lines + visits) : 0ull;
 }
 
 // Whether the one-kernel scan is the faster for a frame of `lines` lines, by its paths'

@@ -339,7 +339,7 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_path_scan(tk_args_path_sc
 // Whether a scene is laid out as tk_k_path_scan takes it: lines and slabs path by
 // path without gaps, slabs as large as their tile boxes, scan chunks and cumsum rows
 // that cut every slab as the recorder does, no path of more than TK_PATH_SCAN_LINES
-// lines and no box beyond the canvas or, where that is wider, beyond TK_PATH_SCAN_RUN.
+// lines or too long for the frame (path_scan_rule.h), and no box beyond the canvas or, where that is wider, beyond TK_PATH_SCAN_RUN.
 // Anything else is left to the separate stages, whose result for it is the
 // reference's.  One thread per line, path, chunk and row; 5 us of an upload of 3,900
 // lines (75 -> 80 us), 9 of one of 107,000 (216 -> 237), 198 of one of 45.5 M.
@@ -357,7 +357,8 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_path_scan_check(tk_args_p
              (!last || (p.line_start + p.line_count == cfg.line_count && p.data_offset + p.data_len == cfg.backdrop_len)) &&
              p.tile_x0 <= p.tile_x1 && p.tile_y0 <= p.tile_y1 && p.tile_x1 <= a.widest && p.tile_y1 <= 0xFFFFu &&
              (uint64_t)(p.tile_x1 - p.tile_x0) * (p.tile_y1 - p.tile_y0) == p.data_len &&
-             p.line_count <= TK_PATH_SCAN_LINES;
+             p.line_count <= TK_PATH_SCAN_LINES &&
+             tk::path_scan_excess(p.line_count, p.segment_capacity, p.data_len) <= cfg.line_count / 256u;
         const tk_scan_chunk_range r = a.chunk_ranges[i];
         ok = ok && r.start == (i ? a.chunk_ranges[i - 1u].end : 0u) && r.end >= r.start &&
              r.end - r.start == (p.data_len + TK_SCAN_CHUNK_SIZE - 1u) / TK_SCAN_CHUNK_SIZE &&
