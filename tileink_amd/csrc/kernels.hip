@@ -1534,7 +1534,9 @@ __device__ __forceinline__ TileLayers tile_layers(const CoarseCtx &c, uint32_t l
 // (the batch left open before, or kNone): its runs of one batch each.  A run is
 // `closed` when the chunk holds all of it and none of its layers acts on the tile, as
 // most are inside nested clips; then the run's stream is its particles and END, and all
-// such runs are worked out at once, a lane each, instead of one after another.
+// such runs are worked out at once, a lane each, instead of one after another.  Where
+// the tile does not know its layers (more than 64 pairs in the scene, a batch of scenes,
+// no class table), every run of a scene with layers counts as acted on.
 // (Emission of 50,000 paths under 32 clips, 65 batches a tile: 231 -> 142 us; of 200,000
 // polygons, one or two batches a tile: 240 -> 114.)
 struct ChunkRuns {
@@ -2434,8 +2436,9 @@ __device__ __forceinline__ void fine_tile(const tk_args_fine &a) {
     }
 }
 
-// Seven waves per SIMD: at most 72 VGPRs (a few dwords spill, in the per-batch-run
-// setup outside the record loop).
+// Seven waves per SIMD: at most 72 VGPRs, two or three of them spilled once per window
+// of records (some 300 bytes a wave).  Seven workgroups fit a CU's LDS too, 16 KiB each
+// and 256 bytes per clip level beyond four, up to 31 levels; under 32 clips six do.
 extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void tk_k_fine(tk_args_fine a) {
     fine_tile<false, false>(a);
 }
