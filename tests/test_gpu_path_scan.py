@@ -357,3 +357,35 @@ def test_moves_on_the_widest_canvas(ctx, tiles):
         frame.render()
         assert frame.stats()["one_kernel_scan"] == (tiles == RUN)
         assert np.array_equal(frame.image(), oracle.render_frame(canvas_of(ps).arrays(0))[0])
+
+
+@pytest.mark.parametrize("scale,shift", [(1.0, (32.0, -48.0)), (2.0, (0.0, 0.0)), (0.5, (16.0, 7.5))])
+def test_path_transforms_match_oracle(ctx, scale, shift):
+    """Lines in a path's own space: every third path's, the others' transform the identity."""
+    rng = np.random.default_rng(9)
+    canvas = tk.Canvas(700, 500)
+    for k in range(90):
+        pts = np.round(rng.uniform(-40, 90, (6, 2)) * 8) / 8 + 16 * rng.integers(0, 36, 2)
+        canvas.push_polygon(pts, tk.Color(*rng.uniform(0, 1, 3), 0.5), rule=tk.FillRule(k % 2))
+    canvas.push_polygon(np.round(rng.uniform(0, 690, (30, 2))), tk.Color(0.1, 0.2, 0.8, 0.3), rule=tk.FillRule.EvenOdd)
+    plain = canvas.arrays(0)
+    moved = tk.SceneArrays.__new__(tk.SceneArrays)
+    moved.__dict__.update(plain.__dict__)
+    moved.lines, moved.paths = plain.lines.copy(), plain.paths.copy()
+    own = np.arange(len(moved.paths)) % 3 == 0
+    transform = np.array([scale, 0.0, 0.0, scale, *shift], np.float32)
+    moved.paths[own, 13:19] = transform.view(np.uint32)
+    mine = own[moved.lines["path_id"]]
+    for end in ("p0", "p1"):  # exact: eighths of a pixel by powers of two
+        moved.lines[end][mine] = (plain.lines[end][mine] - np.float32(shift)) / np.float32(scale)
+    frame = tk.Frame(ctx, moved.to_scene())
+    frame.render()
+    assert frame.stats()["one_kernel_scan"] == 1
+    want = oracle.render_frame(moved)[0]
+    assert np.array_equal(want, oracle.render_frame(plain)[0])
+    assert np.array_equal(frame.image(), want)
+    other = _swapped(moved)
+    frame.update(other.to_scene())
+    frame.render()
+    assert frame.stats()["one_kernel_scan"] == 0
+    assert np.array_equal(frame.image(), want)
