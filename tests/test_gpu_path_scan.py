@@ -21,10 +21,12 @@ MOST = 64512   # lines of the longest path it takes (TK_PATH_SCAN_LINES)
 def _pays(arrays):
     """path_scan_rule.h: whether the one-kernel scan is the faster for a scene."""
     lines, tiles, visits = (arrays.paths[:, k].astype(np.int64) for k in (1, 5, 11))
-    even = 4096 + lines + np.minimum(3 * tiles, 1024 * visits // np.maximum(lines, 1))
+    reach = np.minimum(3 * tiles, 1024 * visits // np.maximum(lines, 1))
+    even = 4096 + lines + reach
+    most = len(arrays.lines) // 256 + int(np.where(tiles > 1280, reach, 0).max()) // 3
     worst = max(0, (visits - even).max(), (lines - 6144 - np.minimum(2 * tiles, 2048)).max())
     shared = np.where(tiles > 1280, tiles // 640 * (8192 + lines + visits), 0).sum()
-    return bool(worst <= len(arrays.lines) // 256 and shared <= (1 << 27) + 12 * len(arrays.lines))
+    return bool(worst <= most and shared <= (1 << 27) + 12 * len(arrays.lines))
 
 
 def _swapped(arrays):
@@ -220,13 +222,17 @@ def test_tables_of_many_batches_start_cleared(ctx, width, height, clips):
 # across one run's tiles, across shared ones, and lines of a visit each
 @pytest.mark.parametrize("kind,lines,width,one", [
     ("across", 700, 120, True), ("across", 1100, 120, False), ("across", 250, 500, True), ("across", 900, 500, False),
-    ("along", 5500, 120, True), ("along", 6600, 120, False), ("along", 8000, 600, True), ("along", 8400, 600, False),
+    ("along", 5500, 120, True), ("along", 6600, 120, False), ("along", 8000, 600, True), ("along", 9900, 600, False),
+    ("far", 5000, 1500, True), ("far", 11000, 1500, False),
 ])
 def test_long_paths_take_the_route_of_the_rule(ctx, kind, lines, width, one):
     rng = np.random.default_rng(lines)
     canvas = tk.Canvas(width, width)
     _zigzag(canvas, 40, width, width, rng)
-    if kind == "across":
+    if kind == "far":  # short lines in a corner, beside a path whose lines reach across
+        _zigzag(canvas, 30, width, width, rng)
+        pts = 60.0 * rng.uniform(size=(lines, 2)) + 2.0
+    elif kind == "across":
         pts = rng.uniform(1.0, width - 1.0, (lines, 2))
     else:  # a curve of steps far shorter than a tile
         t = np.arange(lines) * 0.005

@@ -151,8 +151,10 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_fe_paths(tk_args_frontend
     const uint32_t visits = a.path_vals[TK_FE_SEGMENTS * P + p];
     if (const uint32_t excess = tk::path_scan_excess(lines, visits, data_len))
         atomicMax(&a.totals[TK_FE_SCAN_EXCESS], (unsigned long long)excess);
-    if (const uint64_t shared = tk::path_scan_shared(lines, visits, data_len))
+    if (const uint64_t shared = tk::path_scan_shared(lines, visits, data_len)) {
         atomicAdd(&a.totals[TK_FE_SCAN_SHARED], (unsigned long long)shared);
+        atomicMax(&a.totals[TK_FE_SCAN_REACH], (unsigned long long)tk::path_scan_reach(lines, visits, data_len));
+    }
     if (lines > TK_PATH_SCAN_LINES) atomicOr(a.status, 4u);  // scanned by the separate stages
     a.path_vals[TK_FE_SCAN_CHUNKS * P + p] = (data_len + TK_SCAN_CHUNK_SIZE - 1u) / TK_SCAN_CHUNK_SIZE;
     a.path_vals[TK_FE_CUMSUM_ROWS * P + p] = rows;

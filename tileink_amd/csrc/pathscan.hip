@@ -358,7 +358,7 @@ extern "C" __global__ __launch_bounds__(256) void tk_k_path_scan_check(tk_args_p
              p.tile_x0 <= p.tile_x1 && p.tile_y0 <= p.tile_y1 && p.tile_x1 <= a.widest && p.tile_y1 <= 0xFFFFu &&
              (uint64_t)(p.tile_x1 - p.tile_x0) * (p.tile_y1 - p.tile_y0) == p.data_len &&
              p.line_count <= TK_PATH_SCAN_LINES &&
-             tk::path_scan_excess(p.line_count, p.segment_capacity, p.data_len) <= cfg.line_count / 256u;
+             tk::path_scan_excess(p.line_count, p.segment_capacity, p.data_len) <= a.most_excess;
         const tk_scan_chunk_range r = a.chunk_ranges[i];
         ok = ok && r.start == (i ? a.chunk_ranges[i - 1u].end : 0u) && r.end >= r.start &&
              r.end - r.start == (p.data_len + TK_SCAN_CHUNK_SIZE - 1u) / TK_SCAN_CHUNK_SIZE &&

@@ -638,23 +638,27 @@ uint32_t path_scan_run(const tk_frame *f) {
 constexpr uint64_t kPathScanClear = 4096;
 constexpr uint32_t kPathScanFillers = 2048;
 
-// path_scan_rule.h's, but for the paths' excess, which the check looks at.  Few paths are
-// shared, and their chunks tell them, a tenth of the records' bytes (200,000 paths: by
-// their records an upload took 5.2 ms, without 4.8).
-bool scene_scan_pays(const tk_scene &s) {
-    uint64_t shared = 0;
+// path_scan_rule.h's for a scene, but for the paths' excess, which the check holds against
+// `most_excess`.  Few paths are shared, and their chunks tell them, a tenth of the records'
+// bytes (200,000 paths: by their records an upload took 5.2 ms, without 4.8).
+bool scene_scan_pays(const tk_scene &s, uint64_t &most_excess) {
+    uint64_t reach = 0, shared = 0;
     for (uint32_t i = 0; i < s.path_count; ++i) {
         const tk_scan_chunk_range r = s.scan_chunk_ranges[i];
         if (r.end - r.start < kPathScanSharedTiles / TK_SCAN_CHUNK_SIZE) continue;
         const tk_path_record &p = s.paths[i];
-        shared += path_scan_shared(p.line_count, p.segment_capacity, p.data_len);
+        const uint64_t part = path_scan_shared(p.line_count, p.segment_capacity, p.data_len);
+        if (!part) continue;
+        shared += part;
+        reach = std::max<uint64_t>(reach, path_scan_reach(p.line_count, p.segment_capacity, p.data_len));
     }
-    return path_scan_pays(s.line_count, 0u, shared);
+    most_excess = path_scan_most_excess(s.line_count, reach);
+    return path_scan_pays(s.line_count, 0u, reach, shared);
 }
 
 // Whether tk_k_path_scan takes the scene whose records are in the frame's buffers:
 // *ctx->refused once the stream is idle.
-tk_status path_scan_check(tk_frame *f, const tk_scene &s) {
+tk_status path_scan_check(tk_frame *f, const tk_scene &s, uint64_t most_excess) {
     tk_args_path_scan_check a{};
     a.cfg = frame_scan_config(s);
     a.lines = f->lines;
@@ -668,6 +672,7 @@ tk_status path_scan_check(tk_frame *f, const tk_scene &s) {
     a.row_count = s.cumsum_row_count;
     a.cs_chunk_count = s.cumsum_chunk_count;
     a.widest = std::min<uint32_t>(frame_tiles_width(f), TK_PATH_SCAN_RUN);
+    a.most_excess = most_excess;
     *f->ctx->refused = 0u;
     TK_HIP(hipHostGetDevicePointer(reinterpret_cast<void **>(&a.refused), f->ctx->refused, 0));
     const uint32_t threads = std::max({1u, s.path_count, s.line_count, s.scan_chunk_count, s.cumsum_row_count});
@@ -694,8 +699,9 @@ tk_status frame_upload(tk_frame *f, const tk_scene *s) {
     TK_TRY(upload(f, f->cs_lens, s->cumsum_chunk_lens, s->cumsum_chunk_count));
     TK_TRY(upload(f, f->cs_row_starts, s->cumsum_row_starts, s->cumsum_row_count));
     TK_TRY(upload(f, f->cs_row_ends, s->cumsum_row_ends, s->cumsum_row_count));
-    const bool pays = scene_scan_pays(*s);
-    if (pays) TK_TRY(path_scan_check(f, *s));
+    uint64_t most_excess;
+    const bool pays = scene_scan_pays(*s, most_excess);
+    if (pays) TK_TRY(path_scan_check(f, *s, most_excess));
     f->pair_count = 0;
     if (f->layer_bits && s->layer_count && s->layers) {
         const uint32_t pairs = layer_pairs(s, f->host_pair_of, f->host_pair_layer);
@@ -1704,7 +1710,7 @@ tk_status frame_set_geometry(tk_frame *f, const FeInput &in) {
     uint32_t highest = 0;
     for (const tk_fe_scene &scene : f->fe_scenes_host) highest = std::max(highest, scene.tiles_height);
     f->path_scan = !(flags & 4u) && frame_tiles_width(f) <= TK_PATH_SCAN_RUN && highest <= 0xFFFFu &&
-                   path_scan_pays(lines, t[TK_FE_SCAN_EXCESS], t[TK_FE_SCAN_SHARED]);
+                   path_scan_pays(lines, t[TK_FE_SCAN_EXCESS], t[TK_FE_SCAN_REACH], t[TK_FE_SCAN_SHARED]);
     return TK_OK;
 }
 

@@ -179,6 +179,7 @@ struct tk_args_path_scan_check {
     const uint32_t *cs_offsets, *cs_lens, *row_starts, *row_ends;
     uint32_t row_count, cs_chunk_count;
     uint32_t widest;              // tiles of the widest canvas, TK_PATH_SCAN_RUN at most
+    uint64_t most_excess;         // the largest path_scan_excess it takes
     uint32_t *refused;            // set to 1 when tk_k_path_scan does not take the scene
 };
 
@@ -337,8 +338,9 @@ enum tk_fe_total : uint32_t {
     TK_FE_ROW_ENTRIES = 7,
     TK_FE_PTCL = 8,
     TK_FE_SCAN_EXCESS = 9,   // the largest path_scan_excess
-    TK_FE_SCAN_SHARED = 10,  // the sum of path_scan_shared
-    TK_FE_TOTALS = 11,
+    TK_FE_SCAN_REACH = 10,   // the largest path_scan_reach of a shared path
+    TK_FE_SCAN_SHARED = 11,  // the sum of path_scan_shared
+    TK_FE_TOTALS = 12,
 };
 
 struct tk_args_frontend {
